@@ -293,7 +293,7 @@ int lmx_cg_ddagd_padded_f32(lmx_wilson* op, void* x, const void* b, int nw, void
  * loops, harnesses that forbid hipMalloc).  Same arguments, kernels and
  * results (bit for bit) as lmx_cg_ddagd; it calls no hipMalloc / hipFree.
  * The reduction partials and the CG state live in a static device array of
- * 1 MiB + 256 B that each GPU holds until the process ends, so the lattice
+ * 2 MiB + 256 B that each GPU holds until the process ends, so the lattice
  * volume is at most 2^24 sites (64^4; LMX_ERR_ARG beyond).  Every call on
  * one GPU shares that array: calls that overlap on one GPU (several host
  * threads or streams at once) race and must be serialised by the caller.

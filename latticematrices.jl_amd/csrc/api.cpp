@@ -124,7 +124,7 @@ int ensure_lo_links(lmx_wilson* op) {
 constexpr size_t kNoAllocStateBytes = 256;                 // one CGState, padded
 constexpr int64_t kNoAllocMaxVolume = int64_t(1) << 24;    // 64^4 sites
 constexpr size_t kNoAllocScratchBytes =
-    kNoAllocStateBytes + sizeof(double) * 2 * (size_t)(kNoAllocMaxVolume / kRedBlock);  // 1 MiB + 256 B
+    kNoAllocStateBytes + sizeof(double) * (size_t)(kNoAllocMaxVolume / 64);  // one sum per 64 sites: 2 MiB + 256 B
 static_assert(sizeof(CGState) <= kNoAllocStateBytes, "CGState must fit its scratch slot");
 
 }  // namespace lmx

@@ -104,18 +104,20 @@ __device__ __forceinline__ void store_partials(double re, double im, bool want_i
 
 // Second stage of every reduction: one block sums the partials in a fixed
 // order and updates the device CG state (or writes the scalar out).
+// n64 > 0: partials holds the sums of 64 consecutive sites instead (n64 of
+// them), combined here four by four as block_tree does.
 __global__ void __launch_bounds__(256) k_finalize(const double* __restrict__ partials, int nb, int kind, int want_im,
-                                                  CGState* st, double* out2) {
+                                                  CGState* st, double* out2, int n64) {
     if (st != nullptr && st->done) return;
     __shared__ double lds4[4];
-    double fre = finish_partials(partials, nb, lds4);
+    double fre = n64 > 0 ? finish_wave_partials(partials, nb, n64, lds4) : finish_partials(partials, nb, lds4);
     double fim = want_im ? finish_partials(partials + nb, nb, lds4) : 0.0;
     if (threadIdx.x == 0) finalize_scalar(kind, st, fre, fim, out2);
 }
 
-int launch_finalize(lmx_context* ctx, int nb, int kind, bool want_im, CGState* st, double* out2) {
+int launch_finalize(lmx_context* ctx, int nb, int kind, bool want_im, CGState* st, double* out2, bool waves) {
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(256), 0, ctx->stream, ctx->partials, nb, kind, want_im ? 1 : 0, st,
-                       out2);
+                       out2, waves ? (int)((ctx->V + 63) / 64) : 0);
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }

@@ -264,6 +264,11 @@ struct SpF64In {
         double c;
         ld12s(r, s, z, c);
     }
+    // one component
+    __device__ __forceinline__ cx<double> ld1(int r, int k, int s) const {
+        const double2 v = ldg_stream(p + ((size_t)r * 12 + k) * V, s);
+        return mk<double>(v.x, v.y);
+    }
     // streamed form (a field read once, at the site itself)
     __device__ __forceinline__ void ld12_stream(int r, int s, cx<double>* z) const {
         const double2* q = p + (size_t)r * 12 * V;
@@ -282,6 +287,9 @@ struct SpF64Out {
         double2* q = p + (size_t)r * 12 * V;
 #pragma unroll
         for (int k = 0; k < 12; ++k) st_out((double2*)((char*)(q + (size_t)k * V) + (unsigned)s * 16u), z[k].re, z[k].im);
+    }
+    __device__ __forceinline__ void st1(int r, int k, int s, cx<double> z) const {
+        st_out((double2*)((char*)(p + ((size_t)r * 12 + k) * V) + (unsigned)s * 16u), z.re, z.im);
     }
 };
 // A 256-site slice of one right-hand side staged in LDS by the LDS-staged
@@ -330,6 +338,11 @@ struct SpF32In {
         float c;
         ld12s(r, s, z, c);
     }
+    // one component
+    __device__ __forceinline__ cx<float> ld1(int r, int k, int s) const {
+        const float2 v = ldg_stream(p + ((size_t)r * 12 + k) * V, s);
+        return mk<float>(v.x, v.y);
+    }
     // streamed forms (fields read once, at the site itself)
     __device__ __forceinline__ void ld12s_stream(int r, int s, cx<float>* z, float& c) const {
         const float2* q = p + (size_t)r * 12 * V;
@@ -354,6 +367,9 @@ struct SpF32Out {
         float2* q = p + (size_t)r * 12 * V;
 #pragma unroll
         for (int k = 0; k < 12; ++k) st_out((float2*)((char*)(q + (size_t)k * V) + (unsigned)s * 8u), z[k].re, z[k].im);
+    }
+    __device__ __forceinline__ void st1(int r, int k, int s, cx<float> z) const {
+        st_out((float2*)((char*)(p + ((size_t)r * 12 + k) * V) + (unsigned)s * 8u), z.re, z.im);
     }
 };
 
@@ -894,6 +910,19 @@ __device__ __forceinline__ double block_tree(double v, double* lds4) {
 __device__ __forceinline__ double finish_partials(const double* partials, int nb, double* lds4) {
     double acc = 0.0;
     for (int b = threadIdx.x; b < nb; b += kRedBlock) acc = acc + partials[b];
+    return block_tree(acc, lds4);
+}
+
+// The same from the sums of 64 consecutive sites (n64 of them; a block's
+// missing ones are zero, as block_tree finds its idle wavefronts).
+__device__ __forceinline__ double finish_wave_partials(const double* w, int nb, int n64, double* lds4) {
+    double acc = 0.0;
+    for (int b = threadIdx.x; b < nb; b += kRedBlock) {
+        const int k = 4 * b;
+        const double w0 = w[k], w1 = k + 1 < n64 ? w[k + 1] : 0.0, w2 = k + 2 < n64 ? w[k + 2] : 0.0,
+                     w3 = k + 3 < n64 ? w[k + 3] : 0.0;
+        acc = acc + ((w0 + w2) + (w1 + w3));
+    }
     return block_tree(acc, lds4);
 }
 

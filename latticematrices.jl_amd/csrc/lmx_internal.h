@@ -111,6 +111,12 @@ struct Epilogue {
 
 int launch_wilson_f64(lmx_context* ctx, const double2* U, const double2* clover, double kappa, double csw,
                       double2* out, const double2* in, int nrhs, int flags, const Epilogue& epi);
+// The same by the eight-wavefront kernel (wilson_hops.hip), and whether it is
+// the faster one on this lattice.  Epilogue kind 1 leaves one p.Ap sum per 64
+// consecutive sites in e.partials (for launch_finalize's `waves`).
+bool hops_f64(const lmx_context* ctx, bool clover);
+int launch_hops_f64(lmx_context* ctx, double2* out, const double2* in, const double2* U, const double2* clover,
+                    const double2* p, double kappa, double csw, int nrhs, int flags, const Epilogue& e);
 // FP64 D^dagger of the mixed solver's reliable update with the true residual
 // fused: r = b - D^dagger in, written in the inner format (spinor_prec LMX_H16
 // with its scales r_norm, or LMX_F32) for the RHS not retired (done) -- or, if
@@ -218,7 +224,8 @@ inline int link_nelem(const lmx_context* ctx) { return ctx->nc * ctx->nc; }
 
 // ---- BLAS / CG kernels (blas.hip) ----
 enum { FIN_OUT = 0, FIN_BB = 1, FIN_RR0 = 2, FIN_RRNEW = 3, FIN_PAP = 4 };
-int launch_finalize(lmx_context* ctx, int nb, int kind, bool want_im, CGState* st, double* out2);
+// waves: the partials are the sums of 64 consecutive sites (four per 256-site block)
+int launch_finalize(lmx_context* ctx, int nb, int kind, bool want_im, CGState* st, double* out2, bool waves = false);
 int launch_dot(lmx_context* ctx, const double2* A, const double2* B, int fin_kind, CGState* st, double* out2);
 int launch_axpby(lmx_context* ctx, double a, const double2* X, double b, double2* Y, int64_t n);
 int launch_zero(lmx_context* ctx, double2* p, int64_t n);

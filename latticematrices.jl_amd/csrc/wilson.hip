@@ -29,6 +29,14 @@ int launch_wilson_f64(lmx_context* ctx, const double2* U, const double2* clover,
     F64Clover F{clover};
     EpiArgs epi{e.partials, 0, e.st, e.gate};
     const NoEx none{};
+    // one field, or clover fields (one at a time): the eight-wavefront kernel
+    // where it is the faster one; a gated launch, which mostly only finds its
+    // gate off, keeps the smaller grids
+    const bool hops = (nrhs == 1 || clover != nullptr) && e.gate == nullptr && hops_f64(ctx, clover != nullptr);
+    if (hops) {
+        LMX_TRY(launch_hops_f64(ctx, out, in, U, clover, e.aux, kappa, csw, nrhs, flags, e));
+        return e.kind == 1 ? launch_finalize(ctx, nblocks(ctx->V), FIN_PAP, false, e.st, nullptr, true) : LMX_OK;
+    }
     if (e.kind == 1) {
         LMX_CHECK(nrhs == 1, LMX_ERR_UNSUPPORTED, "fused p.Ap needs a single right-hand side");
         SpF64In aux{e.aux, V};

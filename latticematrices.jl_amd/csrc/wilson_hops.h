@@ -1,0 +1,364 @@
+// wilson_hops.h -- the Wilson(-clover) stencil with the eight hops of a site
+// on eight wavefronts (FP64 and FP32 fields, one right-hand side per
+// workgroup).
+//
+// A workgroup of 512 work items owns 64 consecutive sites: lane i of every
+// wavefront is site i, wavefront 2 mu the forward and 2 mu + 1 the backward
+// hop of direction mu.  Each wavefront loads one neighbour spinor and one
+// link, forms its half-spinor U P psi and leaves it in LDS; after one barrier
+// wavefronts 0-5 each sum two of the site's twelve components over the eight
+// hops, in the reference's order, and write them (results bit-identical to
+// k_site's and k_stream's).
+//
+// Why: with the hops one after the other in one work item (k_site, k_stream)
+// a site waits for nine loads in turn, at 230-256 VGPRs and one or two
+// wavefronts per SIMD.  Here it waits for one, at 128 VGPRs and four per SIMD
+// (two workgroups per CU; 60 KB of LDS each in FP64), at the price of 1.5 KB
+// of LDS traffic per site and of the neighbours in t read again.  To keep
+// those in L2 the blocks are ordered slab by slab: an eighth of the 3-D
+// volume, which is one XCD's share, for t = 0, 1, ... (lattice order instead:
+// 174 against 148 us at 24^3 x 48, 3400 against 2650 us at 48^3 x 96; tiles in
+// y and z, nontemporal loads of links and a walk over t within the workgroup
+// were no faster).
+//
+#pragma once
+
+#include "wilson_kernels.h"
+
+namespace lmx {
+
+constexpr int kHopSites = 64;
+
+// Element s of the uniform base, the base held in scalar registers and the
+// lane's part a 32-bit offset: with the addresses left to the compiler, the 21
+// loads of a hop keep as many 64-bit lane addresses, and the kernel spills.
+template <typename V2, typename T>
+__device__ __forceinline__ V2 ld_sbase(const T* base, int s) {
+    using G = __attribute__((address_space(1))) const char*;
+    G b = (G)base;
+    asm("" : "+s"(b));
+    return *(__attribute__((address_space(1))) const V2*)(b + (unsigned)s * (unsigned)sizeof(V2));
+}
+// n components of stride V at site s
+template <int N, typename R, typename T>
+__device__ __forceinline__ void ld_comps(const T* base, int V, int s, cx<R> (&z)[N]) {
+    using V2 = R __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const V2 v = ld_sbase<V2>(base + (size_t)k * V, s);
+        z[k] = mk<R>(v.x, v.y);
+    }
+}
+
+// U P psi of one hop (the reference's half-spin order), the boundary phase
+// applied where the neighbour wraps.
+template <int MU, int PM, bool FWD, bool GP, typename R>
+__device__ __forceinline__ void hop_product(cx<R> (&psi)[12], const cx<R> (&u)[9], bool w, const Geom& g,
+                                            cx<R> (&o)[6]) {
+    cx<R> h[6];
+    if (GP) {
+        if (w && !g.phase_one[MU]) {
+            if (FWD)
+                phase_spinor(psi, g.ph_re[MU], g.ph_im[MU]);
+            else
+                phase_spinor(psi, g.iph_re[MU], g.iph_im[MU]);
+        }
+    }
+    half_project<PM, MU>(psi, h);
+    if (!GP) neg_select(h, w && g.phase_neg[MU]);
+    if (FWD)
+        matvec_fwd(u, h, o);
+    else
+        matvec_bwd(u, h, o);
+}
+
+// Add one hop's half-spinor (h1, h2) of a colour to spins (0, 1) or (2, 3) of
+// that colour's accumulator: the pair's share of reconstruct_add.
+template <int PM, int MU, bool HIGH, typename R>
+__device__ __forceinline__ void reconstruct_pair(cx<R>& a, cx<R>& b, cx<R> h1, cx<R> h2) {
+    if (!HIGH) {
+        a = cadd(a, h1);
+        b = cadd(b, h2);
+    } else if (MU == 0) {
+        a = cadd(a, pmi<PM>(h2));
+        b = cadd(b, pmi<PM>(h1));
+    } else if (MU == 1) {
+        a = cadd(a, pmr<PM>(h2));
+        b = csub(b, pmr<PM>(h1));
+    } else if (MU == 2) {
+        a = cadd(a, pmi<PM>(h1));
+        b = csub(b, pmi<PM>(h2));
+    } else {
+        a = csub(a, pmr<PM>(h1));
+        b = csub(b, pmr<PM>(h2));
+    }
+}
+
+// A complex number in LDS as one aligned word, so that a lane moves it whole.
+template <typename R>
+struct alignas(2 * sizeof(R)) LdsCx {
+    R re, im;
+    __device__ __forceinline__ LdsCx& operator=(cx<R> z) {
+        using V2 = R __attribute__((ext_vector_type(2)));
+        *reinterpret_cast<V2*>(this) = V2{z.re, z.im};
+        return *this;
+    }
+    __device__ __forceinline__ operator cx<R>() const {
+        using V2 = R __attribute__((ext_vector_type(2)));
+        const V2 v = *reinterpret_cast<const V2*>(this);
+        return mk<R>(v.x, v.y);
+    }
+};
+template <typename R>
+struct HopLds {
+    LdsCx<R> hop[8][6][kHopSites];  // U P psi of each hop: [hop][2 colour + half-spin][site]
+    LdsCx<R> psi[12][kHopSites];    // the site's own spinor
+};
+
+template <int FPM, bool HIGH, typename R>
+__device__ __forceinline__ void sum_hops(const LdsCx<R> (&hop)[8][6][kHopSites], int c, int lane, cx<R>& a, cx<R>& b) {
+    a = mk<R>(R(0), R(0));
+    b = a;
+#define LMX_HOP_ADD(H, PM, MU) \
+    reconstruct_pair<PM, MU, HIGH, R>(a, b, hop[H][2 * c][lane], hop[H][2 * c + 1][lane])
+    LMX_HOP_ADD(0, FPM, 0);
+    LMX_HOP_ADD(1, -FPM, 0);
+    LMX_HOP_ADD(2, FPM, 1);
+    LMX_HOP_ADD(3, -FPM, 1);
+    LMX_HOP_ADD(4, FPM, 2);
+    LMX_HOP_ADD(5, -FPM, 2);
+    LMX_HOP_ADD(6, FPM, 3);
+    LMX_HOP_ADD(7, -FPM, 3);
+#undef LMX_HOP_ADD
+}
+
+// The clover term of colour C's spins (0, 1) or (2, 3): that pair's share of
+// clover_add, in its order, from the site's own spinor in LDS.
+template <int C, bool HIGH, typename R, class Acc>
+__device__ __forceinline__ void clover_pair(const Acc& F, int s, int V, const LdsCx<R> (&psi)[12][kHopSites], int lane,
+                                            R coefficient, cx<R>& ra, cx<R>& rb) {
+    cx<R> v1 = mk<R>(R(0), R(0)), v2 = v1;
+    R d[6];
+    cx<R> u[6][2];
+#pragma unroll
+    for (int pl = 0; pl < 6; ++pl) {
+        const int q = 3 * pl + C;
+        const cx<R> v = F.ld((long)(q / 2) * V + s);
+        d[pl] = (q & 1) ? v.im : v.re;
+        // the row's two off-diagonal entries, by their column: 0 and 1 of the other two
+        constexpr int j0 = C == 0 ? 0 : (C == 1 ? 0 : 1), j1 = C == 0 ? 1 : 2;
+        u[pl][0] = F.ld((long)(9 + 3 * pl + j0) * V + s);
+        u[pl][1] = F.ld((long)(9 + 3 * pl + j1) * V + s);
+    }
+#pragma unroll
+    for (int ic = 0; ic < 3; ++ic) {
+        cx<R> f[6];
+#pragma unroll
+        for (int pl = 0; pl < 6; ++pl) {
+            if (ic == C)
+                f[pl] = mk<R>(R(0), d[pl]);
+            else if (C < ic)
+                f[pl] = u[pl][C == 0 ? ic - 1 : 1];
+            else
+                f[pl] = cneg(cconj(u[pl][C == 1 ? 0 : ic]));
+        }
+        const cx<R> f12 = f[0], f13 = f[1], f14 = f[2], f23 = f[3], f24 = f[4], f34 = f[5];
+        if (!HIGH) {
+            const cx<R> s1 = cadd(f12, f34), s3 = cadd(f14, f23);
+            const cx<R> dp = mk<R>(-s1.im, s1.re), odp = mk<R>(-s3.im, s3.re);
+            const cx<R> p1 = psi[ic][lane], p2 = psi[3 + ic][lane];
+            v1 = cadd(v1, cadd(cmul(dp, p1), cmul(cadd(cadd(cneg(f13), odp), f24), p2)));
+            v2 = cadd(v2, cadd(cmul(cneg(dp), p2), cmul(csub(cadd(f13, odp), f24), p1)));
+        } else {
+            const cx<R> s2 = csub(f12, f34), s4 = csub(f23, f14);
+            const cx<R> dm = mk<R>(-s2.im, s2.re), odm = mk<R>(-s4.im, s4.re);
+            const cx<R> p3 = psi[6 + ic][lane], p4 = psi[9 + ic][lane];
+            v1 = cadd(v1, cadd(cmul(dm, p3), cmul(csub(cadd(cneg(f13), odm), f24), p4)));
+            v2 = cadd(v2, cadd(cmul(cneg(dm), p4), cmul(cadd(cadd(f13, odm), f24), p3)));
+        }
+    }
+    ra = cadd(ra, rmul(coefficient, v1));
+    rb = cadd(rb, rmul(coefficient, v2));
+}
+
+template <class In, class Lk, class Out, class Cl>
+struct HopArgs {
+    Out out;
+    In in;
+    Lk U;
+    Cl F;
+    In aux;  // p of EPI_PAP
+    typename In::R kappa, ccoef;
+    int r;
+    double* partials;
+};
+
+// Wavefront W's part of the workgroup (hop W; the sum of two components for W < 6).
+template <int W, int FPM, int MODE, int EPI, bool GP, class In, class Lk, class Out, class Cl>
+__device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopLds<typename In::R>& sh,
+                                         double (*pap)[kHopSites], const Geom& g, int s0, int lane, int end) {
+    using R = typename In::R;
+    constexpr int MU = W >> 1;
+    constexpr bool FWD = (W & 1) == 0;
+    constexpr int PM = FWD ? FPM : -FPM;
+    const auto* spin = a.in.p + (size_t)a.r * 12 * g.V;
+    const auto* link = a.U.p + (size_t)MU * 9 * g.V;
+    int s = s0 + lane;
+    const bool live = s < end;
+    if (!live) s = end - 1;  // a ragged last block: recompute, do not store
+    int x[4];
+    site_coords(s, g, x);
+    bool w;
+    cx<R> psi[12], u[9];
+    {
+        const int t = FWD ? nbr_fwd(s, x, MU, g, w) : nbr_bwd(s, x, MU, g, w);
+        ld_comps(link, g.V, FWD ? s : t, u);
+        ld_comps(spin, g.V, t, psi);
+        if constexpr (W == 6) {  // the site's own spinor
+            cx<R> p[12];
+            ld_comps(spin, g.V, s, p);
+#pragma unroll
+            for (int k = 0; k < 12; ++k) sh.psi[k][lane] = p[k];
+        }
+    }
+    cx<R> o[6];
+    hop_product<MU, PM, FWD, GP>(psi, u, w, g, o);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sh.hop[W][k][lane] = o[k];
+    __syncthreads();
+    if constexpr (W < 6) {
+        constexpr int c = W >> 1;
+        constexpr bool kHigh = (W & 1) != 0;
+        constexpr int ka = (kHigh ? 6 : 0) + c, kb = ka + 3;
+        cx<R> ra, rb;
+        sum_hops<FPM, kHigh>(sh.hop, c, lane, ra, rb);
+        if (MODE == MODE_DONLY) {
+            const R half = R(1) / R(2);
+            ra = cadd(mk<R>(R(0), R(0)), rmul(half, ra));
+            rb = cadd(mk<R>(R(0), R(0)), rmul(half, rb));
+        } else {
+            ra = cadd(cx<R>(sh.psi[ka][lane]), rmul(-a.kappa, ra));
+            rb = cadd(cx<R>(sh.psi[kb][lane]), rmul(-a.kappa, rb));
+            if constexpr (MODE == MODE_CLOVER)
+                clover_pair<c, kHigh>(a.F, s, g.V, sh.psi, lane, a.ccoef, ra, rb);
+        }
+        if (live) {
+            a.out.st1(a.r, ka, s, ra);
+            a.out.st1(a.r, kb, s, rb);
+        }
+        if constexpr (EPI == EPI_PAP) {
+            // the terms of Re sum conj(p) Ap, summed per site in kernel_dot_D order by wavefront 7
+            const cx<R> pa = a.aux.ld1(a.r, ka, s), pb = a.aux.ld1(a.r, kb, s);
+            pap[ka][lane] = live ? cmul(cconj(pa), ra).re : 0.0;
+            pap[kb][lane] = live ? cmul(cconj(pb), rb).re : 0.0;
+        }
+    }
+    if constexpr (EPI == EPI_PAP) {
+        __syncthreads();
+        if constexpr (W == 7) {
+            double v = 0.0;
+#pragma unroll
+            for (int k = 0; k < 12; ++k) v = v + pap[k][lane];
+            v = wave_halve(v);
+            if (lane == 0) a.partials[s0 / kHopSites] = v;
+        }
+    }
+}
+
+template <class In, class Lk, class Out, class Cl, int FPM, int MODE, int EPI, bool GP>
+__global__ void __launch_bounds__(512, sizeof(typename In::R) == 8 ? 4 : 6) k_hops(Out out, In in, Lk U, Cl F, In aux, Geom g, double kappa_d,
+                                                 double ccoef_d, int nrhs, int slab, EpiArgs epi) {
+    using R = typename In::R;
+    if (epi.st != nullptr && epi.st->done) return;
+    if (epi.gate != nullptr && *epi.gate == 0) return;
+    __shared__ HopLds<R> sh;
+    __shared__ double pap[EPI == EPI_PAP ? 12 : 1][kHopSites];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int r = lb % nrhs;
+    lb /= nrhs;
+    int s0 = lb * kHopSites, end = g.V;
+    if (slab > 0) {
+        // `slab` 64-site blocks of a t-slice, then the same blocks of the next slice
+        const int V3 = g.stride[3], n3 = (V3 + kHopSites - 1) / kHopSites;
+        const int full = n3 / slab * slab * g.L[3];  // blocks in whole slabs
+        const bool tail = lb >= full;
+        const int n = tail ? n3 % slab : slab;
+        const int q = tail ? lb - full : lb % (slab * g.L[3]);
+        const int first = tail ? n3 / slab * slab : lb / (slab * g.L[3]) * slab;
+        const int t = q / n;
+        s0 = V3 * t + (first + q % n) * kHopSites;
+        end = V3 * (t + 1);
+    }
+    const HopArgs<In, Lk, Out, Cl> a{out, in, U, F, aux, R(kappa_d), R(ccoef_d), r, epi.partials};
+    switch (wave) {
+#define LMX_HOP_WAVE(W)                                                                   \
+    case W:                                                                               \
+        hop_wave<W, FPM, MODE, EPI, GP, In, Lk, Out, Cl>(a, sh, pap, g, s0, lane, end);   \
+        break
+        LMX_HOP_WAVE(0);
+        LMX_HOP_WAVE(1);
+        LMX_HOP_WAVE(2);
+        LMX_HOP_WAVE(3);
+        LMX_HOP_WAVE(4);
+        LMX_HOP_WAVE(5);
+        LMX_HOP_WAVE(6);
+        LMX_HOP_WAVE(7);
+#undef LMX_HOP_WAVE
+    }
+}
+
+// Launch over nrhs fields; flags LMX_DAGGER / LMX_DONLY.  EPI_PAP (on
+// D^dagger, one field): partials gets one sum per 64 consecutive sites.
+template <class In, class Lk, class Out, class Cl, int EPI>
+int launch_hops(lmx_context* ctx, Out out, In in, Lk U, Cl F, In aux, double kappa, double ccoef, int nrhs, int flags,
+                bool clover, const EpiArgs& epi) {
+    const bool dag = (flags & LMX_DAGGER) != 0, donly = (flags & LMX_DONLY) != 0;
+    const Geom& g = ctx->g;
+    const int V3 = g.stride[3], n3 = (V3 + kHopSites - 1) / kHopSites;
+    // slab order needs blocks that end with the slice: idle lanes where V3 is
+    // no multiple of 64 (at most 1/32 of them here; fewer blocks than XCDs are
+    // no slabs), and the 64-site sums of EPI_PAP need full blocks
+    const bool slabs = n3 >= 8 && (V3 % kHopSites == 0 || (EPI != EPI_PAP && n3 >= 32));
+    const int slab = slabs ? (n3 + 7) / 8 : 0;
+    const long nb = (slabs ? (long)n3 * g.L[3] : (ctx->V + kHopSites - 1) / kHopSites) * nrhs;
+    LMX_CHECK(nb < (1L << 31), LMX_ERR_ARG, "too many right-hand sides (%d)", nrhs);
+#define LMX_HOPS(FPM, MODE, GP)                                                                                    \
+    hipLaunchKernelGGL((k_hops<In, Lk, Out, Cl, FPM, MODE, EPI, GP>), dim3((unsigned)nb), dim3(512), 0, ctx->stream, \
+                       out, in, U, F, aux, g, kappa, ccoef, nrhs, slab, epi)
+#define LMX_HOPS_GP(FPM, MODE)            \
+    do {                                  \
+        if (g.general)                    \
+            LMX_HOPS(FPM, MODE, true);    \
+        else                              \
+            LMX_HOPS(FPM, MODE, false);   \
+    } while (0)
+#define LMX_HOPS_MODE(FPM)                          \
+    do {                                            \
+        if (clover)                                 \
+            LMX_HOPS_GP(FPM, MODE_CLOVER);          \
+        else                                        \
+            LMX_HOPS_GP(FPM, MODE_WILSON);          \
+    } while (0)
+    if constexpr (EPI == EPI_PAP) {
+        LMX_CHECK(dag && !donly && nrhs == 1, LMX_ERR_UNSUPPORTED, "fused p.Ap is built for one field on D^dagger");
+        LMX_HOPS_MODE(1);
+    } else if (donly) {
+        if (dag)
+            LMX_HOPS_GP(1, MODE_DONLY);
+        else
+            LMX_HOPS_GP(-1, MODE_DONLY);
+    } else if (dag) {
+        LMX_HOPS_MODE(1);
+    } else {
+        LMX_HOPS_MODE(-1);
+    }
+#undef LMX_HOPS_MODE
+#undef LMX_HOPS_GP
+#undef LMX_HOPS
+    LMX_HIP(hipGetLastError());
+    return LMX_OK;
+}
+
+}  // namespace lmx

@@ -1,0 +1,70 @@
+"""The eight-wavefront stencil (FP64, one field or clover fields) against the
+oracle, bit for bit, at the sizes where its blocks can go wrong: fewer sites
+than a block, a last block cut by the lattice, slabs that divide the slice and
+that do not, slices that end inside a block, complex phases; and the p.Ap sums
+that it leaves per 64 sites through whole CG solves."""
+import numpy as np
+import pytest
+
+import oracle as orc
+import lmx
+from lmx import generators as gen
+
+pytestmark = pytest.mark.gpu
+
+ANTI = (1, 1, 1, -1)
+SHAPES = [
+    ((2, 2, 2, 2), ANTI),                          # 16 sites: one block, 48 idle lanes
+    ((3, 5, 3, 3), ANTI),                          # 135 sites: a cut last block, lattice order
+    ((8, 8, 4, 3), ANTI),                          # slices of 4 whole blocks, no slabs
+    ((8, 8, 8, 4), ANTI),                          # 8 blocks a slice: slabs of one block
+    ((8, 8, 9, 4), ANTI),                          # 9 blocks: slabs of two and a tail slab of one
+    ((13, 13, 13, 3), ANTI),                       # 2197 sites a slice: slices end inside a block, tail slab
+    ((13, 13, 13, 2), (np.exp(0.3j), 1, -1j, -1)),  # the same with complex phases
+]
+
+
+@pytest.mark.parametrize("L,phases", SHAPES)
+@pytest.mark.parametrize("flags", [0, 1, 2, 3])
+def test_wilson(gpu, L, phases, flags):
+    print(f"blocks L={L} flags={flags}", flush=True)
+    U = gen.links(L, "haar", 31)
+    psi = gen.gaussian_spinor(L, 32)
+    lat = lmx.Lattice(L, phases)
+    Ug = lat.gauge_from_numpy(U)
+    A = lmx.WilsonDiracOperator4D_Donly(Ug) if flags & 2 else lmx.WilsonDiracOperator4D(Ug, 0.117)
+    y = lat.spinor()
+    lmx.mul_(y, lmx.adjoint(A) if flags & 1 else A, lat.spinor_from_numpy(psi))
+    ref = orc.wilson(U, psi, L, 0.117, phases, dagger=bool(flags & 1), donly=bool(flags & 2))
+    assert np.array_equal(y.to_numpy(), ref)
+
+
+@pytest.mark.parametrize("L", [(3, 5, 3, 3), (8, 8, 9, 4), (13, 13, 13, 3)])
+@pytest.mark.parametrize("dagger", [False, True])
+def test_clover_three_fields(gpu, L, dagger):
+    print(f"clover blocks L={L} dagger={dagger}", flush=True)
+    U = gen.links(L, "weak", 33, eps=0.15)
+    psi = gen.gaussian_spinor(L, 34, nrhs=3)
+    lat = lmx.Lattice(L, ANTI)
+    D = lmx.WilsonDiracCloverOperator4D(lat.gauge_from_numpy(U), 0.1235, 1.0)
+    y = lat.spinor(3)
+    lmx.mul_(y, lmx.adjoint(D) if dagger else D, lat.spinor_from_numpy(psi))
+    F = orc.clover_field_strength(U, L)
+    got = y.to_numpy()
+    for r in range(3):
+        assert np.array_equal(got[r], orc.wilson_clover(U, F, psi[r], L, 0.1235, 1.0, dagger=dagger))
+
+
+@pytest.mark.parametrize("L", [(2, 2, 2, 2), (3, 5, 3, 3), (8, 8, 9, 4), (13, 13, 13, 3)])
+def test_cg(gpu, L):
+    print(f"CG blocks L={L}", flush=True)
+    U = gen.links(L, "haar", 35)
+    b = gen.gaussian_spinor(L, 36)
+    xo, ro = orc.cg(orc.NormalOp(orc.OP_DDAGD_WILSON, L, U=U, kappa=0.12), b, rtol=1e-10, order=1)
+    lat = lmx.Lattice(L, ANTI)
+    D = lmx.WilsonDiracOperator4D(lat.gauge_from_numpy(U), 0.12)
+    x, r, p, Ap, tmp = (lat.spinor() for _ in range(5))
+    res = lmx.cg_(x, lmx.DdagDOp(D, tmp), lat.spinor_from_numpy(b), r, p, Ap, rtol=1e-10)
+    assert res.converged and res.iterations == ro.iterations
+    assert np.array_equal(x.to_numpy(), xo)
+    assert res.residual_norm == ro.residual_norm
