@@ -529,7 +529,7 @@ int lmx_wilson_destroy(lmx_wilson* op) {
     if (op->clover64) (void)hipFree(op->clover64);
     if (op->clover32) (void)hipFree(op->clover32);
     if (op->clover16) (void)hipFree(op->clover16);
-    if (op->clover_dF) (void)hipFree(op->clover_dF);
+    if (op->clover_dQ) (void)hipFree(op->clover_dQ);
     delete op;
     return LMX_OK;
 }
@@ -802,8 +802,8 @@ static int operator_pullback(lmx_wilson* op, double2* dU, const double2* dres, c
     }
     LMX_TRY(launch_pullback_f64(op->ctx, dU, dres, psi, coefficient));
     if (op->csw == 0.0) return LMX_OK;
-    if (!op->clover_dF) LMX_HIP(hipMalloc(&op->clover_dF, 6 * 9 * (size_t)op->ctx->V * sizeof(double2)));
-    return launch_clover_pullback(op->ctx, dU, op->links, op->clover_dF, dres, psi, coefficient * op->csw);
+    if (!op->clover_dQ) LMX_HIP(hipMalloc(&op->clover_dQ, 6 * 5 * (size_t)op->ctx->V * sizeof(double2)));
+    return launch_clover_pullback(op->ctx, dU, op->links, op->clover_dQ, dres, psi, coefficient * op->csw);
 }
 }  // namespace lmx
 

@@ -141,34 +141,82 @@ int launch_ta_project(lmx_context* ctx, double2* F, const double2* U, const doub
 // operation order follows the reference's loops (planes 12..34, leaves,
 // occurrences 1..4).
 // ---------------------------------------------------------------------------
-struct GammaProducts {
-    double2 g[6][4][4];
-};
 
-__device__ __forceinline__ void mat_mul_plain(const cx<double>* A, const cx<double>* B, cx<double>* out) {
-    cx<double> r[9];
+__device__ __forceinline__ void mat_mul_plain(const cx<double> A[9], const cx<double> B[9], cx<double> out[9]) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-            r[3 * i + j] =
+            out[3 * i + j] =
                 cadd(cadd(cmul(A[3 * i], B[j]), cmul(A[3 * i + 1], B[3 + j])), cmul(A[3 * i + 2], B[6 + j]));
-#pragma unroll
-    for (int k = 0; k < 9; ++k) out[k] = r[k];
 }
-__device__ __forceinline__ void mat_dag(const cx<double>* A, cx<double>* out) {
-    cx<double> r[9];
+__device__ __forceinline__ void mat_dag(const cx<double> A[9], cx<double> out[9]) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) r[3 * i + j] = cconj(A[3 * j + i]);
-#pragma unroll
-    for (int k = 0; k < 9; ++k) out[k] = r[k];
+        for (int j = 0; j < 3; ++j) out[3 * i + j] = cconj(A[3 * j + i]);
 }
 
-__global__ void __launch_bounds__(256) k_clover_cotangent(double2* __restrict__ dF, const double2* __restrict__ dres,
-                                                          const double2* __restrict__ psi, int V, double coefficient,
-                                                          GammaProducts gp) {
+// Row o of gamma_mu gamma_nu in the chiral basis (src/Operators/Operators.jl:44-67)
+// has one entry, a power of i: its column and that power.
+struct GammaEntry {
+    int col, pow;
+};
+constexpr GammaEntry gamma_entry(int mu, int row) {
+    constexpr int col[4][4] = {{3, 2, 1, 0}, {3, 2, 1, 0}, {2, 3, 0, 1}, {2, 3, 0, 1}};
+    constexpr int pw[4][4] = {{3, 3, 1, 1}, {2, 0, 0, 2}, {3, 1, 1, 3}, {2, 2, 2, 2}};
+    return {col[mu][row], pw[mu][row]};
+}
+constexpr GammaEntry gamma_product_entry(int mu, int nu, int row) {
+    const GammaEntry a = gamma_entry(mu, row), b = gamma_entry(nu, a.col);
+    return {b.col, (a.pow + b.pow) & 3};
+}
+template <int POW>
+__device__ __forceinline__ cx<double> i_pow(cx<double> z) {
+    return POW == 0 ? z : POW == 1 ? mk<double>(-z.im, z.re) : POW == 2 ? cneg(z) : mk<double>(z.im, -z.re);
+}
+
+// dF[c][ic] of plane (MU, NU): coefficient * sum_out dres[c,out] conj(sum_in g[out,in] psi[ic,in])
+template <int MU, int NU, int O>
+__device__ __forceinline__ void cotangent_add(const cx<double> d[12], const cx<double> p[12], cx<double> f[9]) {
+    constexpr GammaEntry e = gamma_product_entry(MU, NU, O);
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int ic = 0; ic < 3; ++ic)
+            f[3 * c + ic] = cadd(f[3 * c + ic], cmul(d[O * 3 + c], cconj(i_pow<e.pow>(p[e.col * 3 + ic]))));
+}
+template <int PL, int MU, int NU>
+__device__ __forceinline__ void cotangent_plane(double2* __restrict__ dQ, const cx<double> d[12], const cx<double> p[12],
+                                                int s, int V, double coefficient) {
+    cx<double> f[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) f[k] = mk<double>(0.0, 0.0);
+    cotangent_add<MU, NU, 0>(d, p, f);
+    cotangent_add<MU, NU, 1>(d, p, f);
+    cotangent_add<MU, NU, 2>(d, p, f);
+    cotangent_add<MU, NU, 3>(d, p, f);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) f[k] = rmul(coefficient, f[k]);
+    double2* q = dQ + (size_t)PL * 5 * V;
+    const double d0 = 0.125 * (f[0].im + f[0].im), d1 = 0.125 * (f[4].im + f[4].im), d2 = 0.125 * (f[8].im + f[8].im);
+    const cx<double> u0 = rmul(0.125, csub(f[1], cconj(f[3]))), u1 = rmul(0.125, csub(f[2], cconj(f[6]))),
+                     u2 = rmul(0.125, csub(f[5], cconj(f[7])));
+    q[s] = make_double2(d0, d1);
+    q[(size_t)V + s] = make_double2(d2, 0.0);
+    q[(size_t)2 * V + s] = make_double2(u0.re, u0.im);
+    q[(size_t)3 * V + s] = make_double2(u1.re, u1.im);
+    q[(size_t)4 * V + s] = make_double2(u2.re, u2.im);
+}
+
+// dQ = (dF - dF^dagger) / 8 of the six planes.  It is anti-Hermitian exactly
+// (the differences negate and the sums commute), so five words per plane hold
+// it: the three imaginary diagonals and the upper entries.  That is all the
+// links' chain rule reads; the products with gamma_mu gamma_nu are one term
+// each.  Bound by its 384 B read and 480 B written per site: 16^3 x 32 in
+// 21 us, against 17 + 59 us for a zero fill and full planes read and written.
+__global__ void __launch_bounds__(256) k_clover_cotangent(double2* __restrict__ dQ, const double2* __restrict__ dres,
+                                                          const double2* __restrict__ psi, int V, double coefficient) {
     const int s = blockIdx.x * 256 + threadIdx.x;
     if (s >= V) return;
     cx<double> d[12], p[12];
@@ -178,205 +226,180 @@ __global__ void __launch_bounds__(256) k_clover_cotangent(double2* __restrict__ 
         d[k] = mk<double>(a.x, a.y);
         p[k] = mk<double>(b.x, b.y);
     }
-    for (int pl = 0; pl < 6; ++pl)
-        for (int ic = 0; ic < 3; ++ic)
-            for (int c = 0; c < 3; ++c) {
-                cx<double> value = mk<double>(0.0, 0.0);
-                for (int o = 0; o < 4; ++o) {
-                    cx<double> tp = mk<double>(0.0, 0.0);
-                    for (int i = 0; i < 4; ++i) {
-                        const double2 gg = gp.g[pl][o][i];
-                        tp = cadd(tp, cmul(mk<double>(gg.x, gg.y), p[i * 3 + ic]));
-                    }
-                    value = cadd(value, cmul(d[o * 3 + c], cconj(tp)));
-                }
-                const long e = ((long)pl * 9 + c * 3 + ic) * V + s;
-                double2 cur = dF[e];
-                cx<double> nv = cadd(mk<double>(cur.x, cur.y), rmul(coefficient, value));
-                dF[e] = make_double2(nv.re, nv.im);
-            }
+    cotangent_plane<0, 0, 1>(dQ, d, p, s, V, coefficient);
+    cotangent_plane<1, 0, 2>(dQ, d, p, s, V, coefficient);
+    cotangent_plane<2, 0, 3>(dQ, d, p, s, V, coefficient);
+    cotangent_plane<3, 1, 2>(dQ, d, p, s, V, coefficient);
+    cotangent_plane<4, 1, 3>(dQ, d, p, s, V, coefficient);
+    cotangent_plane<5, 2, 3>(dQ, d, p, s, V, coefficient);
 }
 
-// leaf p of plane (mu, nu): (mu,nu,-mu,-nu), (nu,-mu,-nu,mu), (-mu,-nu,mu,nu), (-nu,mu,nu,-mu)
-// (_clover_path_descriptor, :140-159): factor origins relative to the anchor,
-// directions and adjoint flags.
-struct LeafPath {
-    int origin[4][4];
-    int dir[4];
-    int dag[4];
-};
-__device__ __forceinline__ void make_leaf(int mu, int nu, int p, LeafPath& lp) {
-    const int m = mu + 1, n = nu + 1;
-    int sd[4];
-    if (p == 0) { sd[0] = m; sd[1] = n; sd[2] = -m; sd[3] = -n; }
-    else if (p == 1) { sd[0] = n; sd[1] = -m; sd[2] = -n; sd[3] = m; }
-    else if (p == 2) { sd[0] = -m; sd[1] = -n; sd[2] = m; sd[3] = n; }
-    else { sd[0] = -n; sd[1] = m; sd[2] = n; sd[3] = -m; }
-    int pos[4] = {0, 0, 0, 0};
-    for (int k = 0; k < 4; ++k) {
-        const int d = (sd[k] > 0 ? sd[k] : -sd[k]) - 1;
-        if (sd[k] < 0) pos[d] -= 1;
-        for (int e = 0; e < 4; ++e) lp.origin[k][e] = pos[e];
-        lp.dir[k] = d;
-        lp.dag[k] = sd[k] < 0;
-        if (sd[k] > 0) pos[d] += 1;
-    }
-}
-
-__device__ __forceinline__ int site_of(const Geom& g, const int x[4], const int* off, int sign) {
-    int s = 0;
-    for (int d = 0; d < 4; ++d) {
-        int c = x[d] + sign * off[d];
-        c = c < 0 ? c + g.L[d] : (c >= g.L[d] ? c - g.L[d] : c);
-        s += c * g.stride[d];
-    }
-    return s;
-}
-
-__device__ __forceinline__ void ld_link(const double2* __restrict__ U, int V, int mu, int s, cx<double>* u) {
+__device__ __forceinline__ void ld_link(const double2* __restrict__ U, int V, int mu, int s, bool dag, cx<double> u[9]) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        double2 v = U[(long)(mu * 9 + k) * V + s];
-        u[k] = mk<double>(v.x, v.y);
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const double2 v = ldv(U + (size_t)(mu * 9 + 3 * i + j) * V, s);
+            if (dag)
+                u[3 * j + i] = mk<double>(v.x, -v.y);
+            else
+                u[3 * i + j] = mk<double>(v.x, v.y);
+        }
+}
+// dQ of plane pl at s, or its adjoint (exactly -dQ)
+template <bool DAG>
+__device__ __forceinline__ void ld_dq(const double2* __restrict__ dQ, int V, int pl, int s, cx<double> q[9]) {
+    const double2* a = dQ + (size_t)pl * 5 * V;
+    const double2 d01 = ldv(a, s), d2 = ldv(a + (size_t)V, s), u0 = ldv(a + (size_t)2 * V, s),
+                  u1 = ldv(a + (size_t)3 * V, s), u2 = ldv(a + (size_t)4 * V, s);
+    q[0] = mk<double>(0.0, d01.x);
+    q[4] = mk<double>(0.0, d01.y);
+    q[8] = mk<double>(0.0, d2.x);
+    q[1] = mk<double>(u0.x, u0.y);
+    q[2] = mk<double>(u1.x, u1.y);
+    q[5] = mk<double>(u2.x, u2.y);
+    q[3] = cneg(cconj(q[1]));
+    q[6] = cneg(cconj(q[2]));
+    q[7] = cneg(cconj(q[5]));
+    if (DAG) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) q[k] = cneg(q[k]);
+    }
+}
+__device__ __forceinline__ void mat_add(cx<double> a[9], const cx<double> b[9], bool first) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) a[k] = first ? b[k] : cadd(a[k], b[k]);
+}
+
+// The terms of one plaquette loop through a link L at y: L A B C (DAG false)
+// or L^dagger A B C, leaf number p of the plane being the loop begun at
+// another corner.  Begun at L the cotangent enters before L (site s0), at C
+// before C (s3), at B before B (s2), at A before A (s1); with X Y the factors
+// to its left and right in the leaf, the term is X^dagger dQ Y^dagger, or
+// Y dQ^dagger X.  H[p] sums the two terms a leaf has for this link (two terms
+// and a zero: any order), P0..P3 the leaves of the loops begun at L, C, B, A.
+template <bool DAG, bool DA, bool DB, bool DC, int P0, int P1, int P2, int P3, bool FIRST>
+__device__ __forceinline__ void plaquette_terms(const double2* __restrict__ U, const double2* __restrict__ dQ, int V,
+                                                int pl, int mA, int sA, int mB, int sB, int mC, int sC, int s0, int s1,
+                                                int s2, int s3, cx<double> (&H)[4][9]) {
+    cx<double> A[9], B[9], C[9], AB[9], X[9], t[9], h[9], q[9], y[9];
+    ld_link(U, V, mA, sA, DA, A);
+    ld_link(U, V, mB, sB, DB, B);
+    ld_link(U, V, mC, sC, DC, C);
+    mat_mul_plain(B, C, X);  // B C
+    ld_dq<DAG>(dQ, V, pl, s2, q);
+    if (!DAG) {
+        mat_dag(X, t);
+        mat_mul_plain(t, q, y);
+        mat_dag(A, t);
+        mat_mul_plain(y, t, h);
+    } else {
+        mat_mul_plain(A, q, t);
+        mat_mul_plain(t, X, h);
+    }
+    mat_add(H[P2], h, FIRST);
+    mat_mul_plain(A, B, AB);
+    ld_dq<DAG>(dQ, V, pl, s3, q);
+    if (!DAG) {
+        mat_dag(C, t);
+        mat_mul_plain(t, q, y);
+        mat_dag(AB, t);
+        mat_mul_plain(y, t, h);
+    } else {
+        mat_mul_plain(AB, q, t);
+        mat_mul_plain(t, C, h);
+    }
+    mat_add(H[P1], h, FIRST);
+    mat_mul_plain(AB, C, X);  // (A B) C
+    if (!DAG) {
+        mat_dag(X, t);
+        ld_dq<DAG>(dQ, V, pl, s0, q);
+        mat_mul_plain(q, t, h);
+        mat_add(H[P0], h, FIRST);
+        ld_dq<DAG>(dQ, V, pl, s1, q);
+        mat_mul_plain(t, q, h);
+        mat_add(H[P3], h, FIRST);
+    } else {
+        ld_dq<DAG>(dQ, V, pl, s0, q);
+        mat_mul_plain(X, q, h);
+        mat_add(H[P0], h, FIRST);
+        ld_dq<DAG>(dQ, V, pl, s1, q);
+        mat_mul_plain(q, X, h);
+        mat_add(H[P3], h, FIRST);
     }
 }
 
-__global__ void __launch_bounds__(256) k_clover_links_pullback(double2* __restrict__ dU, const double2* __restrict__ U,
-                                                               const double2* __restrict__ dF, Geom g) {
-    const int y = blockIdx.x * 256 + threadIdx.x;
+// Neighbour of a site (with its coordinates) one step along +-mu.
+__device__ __forceinline__ int step_site(const Geom& g, int s, const int x[4], int mu, bool fwd) {
+    bool w;
+    return fwd ? nbr_fwd(s, x, mu, g, w) : nbr_bwd(s, x, mu, g, w);
+}
+
+// Chain rule of the six planes onto the links: wavefront a of a workgroup
+// takes U_a of 64 sites, with the three planes that hold direction a and in
+// each the plaquette on either side.  The four leaves that share a plaquette
+// share its partial products (three products and six with dQ where the leaves
+// one by one take twelve), and the four wavefronts share their links in L1.
+// Bound by the unfused FP64 products (the operation order is the reference's):
+// 216 3x3 products or 43k operations per site, 148 us at 16^3 x 32 with every
+// lane busy; measured 324 us there, against 1142 us for one work item per
+// site that walked the paths through arrays in scratch.
+__global__ void __launch_bounds__(256, 1) k_clover_links_pullback(double2* __restrict__ dU,
+                                                                  const double2* __restrict__ U,
+                                                                  const double2* __restrict__ dQ, Geom g) {
+    const int y = xcd_block(blockIdx.x, gridDim.x) * 64 + (threadIdx.x & 63);
+    const int a = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (y >= g.V) return;
     const int V = g.V;
-    int xy[4];
-    site_coords(y, g, xy);
-    const int pmu[6] = {0, 0, 0, 1, 1, 2}, pnu[6] = {1, 2, 3, 2, 3, 3};
-    for (int pl = 0; pl < 6; ++pl) {
-        const int mu = pmu[pl], nu = pnu[pl];
-        cx<double> dmu[9], dnu[9];
-        for (int k = 0; k < 9; ++k) dmu[k] = dnu[k] = mk<double>(0.0, 0.0);
-        for (int p = 0; p < 4; ++p) {
-            LeafPath lp;
-            make_leaf(mu, nu, p, lp);
-            cx<double> hmu[9], hnu[9];
-            for (int k = 0; k < 9; ++k) hmu[k] = hnu[k] = mk<double>(0.0, 0.0);
-            for (int K = 0; K < 4; ++K) {
-                // anchor = y - origin_K; factor j at anchor + origin_j
-                const int anchor = site_of(g, xy, lp.origin[K], -1);
-                int xa[4];
-                site_coords(anchor, g, xa);
-                cx<double> left[9], right[9], t[9], m[9];
-                const bool has_left = K > 0, has_right = K < 3;
-                // left = M1 ... M_{K-1}
-                for (int j = 0; j < K; ++j) {
-                    ld_link(U, V, lp.dir[j], site_of(g, xa, lp.origin[j], 1), m);
-                    if (lp.dag[j]) mat_dag(m, m);
-                    if (j == 0) {
-                        for (int k = 0; k < 9; ++k) left[k] = m[k];
-                    } else {
-                        mat_mul_plain(left, m, left);
-                    }
-                }
-                // right = M_{K+1} ... M4
-                for (int j = K + 1; j < 4; ++j) {
-                    ld_link(U, V, lp.dir[j], site_of(g, xa, lp.origin[j], 1), m);
-                    if (lp.dag[j]) mat_dag(m, m);
-                    if (j == K + 1) {
-                        for (int k = 0; k < 9; ++k) right[k] = m[k];
-                    } else {
-                        mat_mul_plain(right, m, right);
-                    }
-                }
-                cx<double> f[9], dq[9];
+    int x[4];
+    site_coords(y, g, x);
+    cx<double> out[9];
 #pragma unroll
-                for (int k = 0; k < 9; ++k) {
-                    double2 v = dF[((long)pl * 9 + k) * V + anchor];
-                    f[k] = mk<double>(v.x, v.y);
-                }
-#pragma unroll
-                for (int r = 0; r < 3; ++r)
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) dq[3 * r + c] = rmul(0.125, csub(f[3 * r + c], cconj(f[3 * c + r])));
-                cx<double> h[9];
-                if (lp.dag[K]) {  // right * dQ^dagger * left
-                    mat_dag(dq, dq);
-                    if (has_right)
-                        mat_mul_plain(right, dq, t);
-                    else
-                        for (int k = 0; k < 9; ++k) t[k] = dq[k];
-                    if (has_left)
-                        mat_mul_plain(t, left, h);
-                    else
-                        for (int k = 0; k < 9; ++k) h[k] = t[k];
-                } else {  // left^dagger * dQ * right^dagger
-                    if (has_left) {
-                        mat_dag(left, left);
-                        mat_mul_plain(left, dq, t);
-                    } else {
-                        for (int k = 0; k < 9; ++k) t[k] = dq[k];
-                    }
-                    if (has_right) {
-                        mat_dag(right, right);
-                        mat_mul_plain(t, right, h);
-                    } else {
-                        for (int k = 0; k < 9; ++k) h[k] = t[k];
-                    }
-                }
-                cx<double>* acc = lp.dir[K] == mu ? hmu : hnu;
-                for (int k = 0; k < 9; ++k) acc[k] = cadd(acc[k], h[k]);
-            }
-            for (int k = 0; k < 9; ++k) {
-                dmu[k] = cadd(dmu[k], hmu[k]);
-                dnu[k] = cadd(dnu[k], hnu[k]);
-            }
-        }
-        for (int k = 0; k < 9; ++k) {
-            const long em = (long)(mu * 9 + k) * V + y, en = (long)(nu * 9 + k) * V + y;
-            double2 a = dU[em];
-            cx<double> na = cadd(mk<double>(a.x, a.y), dmu[k]);
-            dU[em] = make_double2(na.re, na.im);
-            double2 b = dU[en];
-            cx<double> nb = cadd(mk<double>(b.x, b.y), dnu[k]);
-            dU[en] = make_double2(nb.re, nb.im);
-        }
+    for (int k = 0; k < 9; ++k) {
+        const double2 v = ldv(dU + (size_t)(a * 9 + k) * V, y);
+        out[k] = mk<double>(v.x, v.y);
     }
+    const int ya = step_site(g, y, x, a, true);
+    int xa[4] = {x[0], x[1], x[2], x[3]};
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+        if (d == a) xa[d] = x[d] + 1 == g.L[d] ? 0 : x[d] + 1;
+#pragma unroll 1
+    for (int b = 0; b < 4; ++b) {
+        if (b == a) continue;
+        const int lo = a < b ? a : b, hi = a < b ? b : a;
+        const int pl = lo == 0 ? hi - 1 : lo + hi;  // (01,02,03,12,13,23)
+        const int yb = step_site(g, y, x, b, true), ymb = step_site(g, y, x, b, false);
+        const int yab = step_site(g, ya, xa, b, true), yamb = step_site(g, ya, xa, b, false);
+        cx<double> H[4][9];
+        if (a < b) {
+            // U_a is the plane's first direction: L U_b(y+a) U_a(y+b)^+ U_b(y)^+ and
+            // L^+ U_b(y-b)^+ U_a(y-b) U_b(y-b+a)
+            plaquette_terms<false, false, true, true, 0, 3, 2, 1, true>(U, dQ, V, pl, b, ya, a, yb, b, y, y, ya, yab, yb,
+                                                                       H);
+            plaquette_terms<true, true, false, false, 2, 1, 0, 3, false>(U, dQ, V, pl, b, ymb, a, ymb, b, yamb, ya, y, ymb,
+                                                                        yamb, H);
+        } else {
+            // the second: L U_b(y-b+a)^+ U_a(y-b)^+ U_b(y-b) and L^+ U_b(y) U_a(y+b) U_b(y+a)^+
+            plaquette_terms<false, true, true, false, 1, 0, 3, 2, true>(U, dQ, V, pl, b, yamb, a, ymb, b, ymb, y, ya, yamb,
+                                                                       ymb, H);
+            plaquette_terms<true, false, false, true, 3, 2, 1, 0, false>(U, dQ, V, pl, b, y, a, yb, b, ya, ya, y, yb, yab,
+                                                                        H);
+        }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) out[k] = cadd(out[k], cadd(cadd(cadd(H[0][k], H[1][k]), H[2][k]), H[3][k]));
+    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) dU[(size_t)(a * 9 + k) * V + y] = make_double2(out[k].re, out[k].im);
 }
 
-// gamma_mu gamma_nu of the chiral gamma matrices (src/Operators/Operators.jl:44-67),
-// exact (entries 0, +-1, +-i), summed as the oracle does
-static GammaProducts gamma_products() {
-    struct C2 {
-        double re, im;
-    };
-    C2 gm[4][4][4] = {};
-    gm[0][0][3] = {0, -1}; gm[0][1][2] = {0, -1}; gm[0][2][1] = {0, 1}; gm[0][3][0] = {0, 1};
-    gm[1][0][3] = {-1, 0}; gm[1][1][2] = {1, 0}; gm[1][2][1] = {1, 0}; gm[1][3][0] = {-1, 0};
-    gm[2][0][2] = {0, -1}; gm[2][1][3] = {0, 1}; gm[2][2][0] = {0, 1}; gm[2][3][1] = {0, -1};
-    gm[3][0][2] = {-1, 0}; gm[3][1][3] = {-1, 0}; gm[3][2][0] = {-1, 0}; gm[3][3][1] = {-1, 0};
-    const int pmu[6] = {0, 0, 0, 1, 1, 2}, pnu[6] = {1, 2, 3, 2, 3, 3};
-    GammaProducts out;
-    for (int pl = 0; pl < 6; ++pl)
-        for (int i = 0; i < 4; ++i)
-            for (int j = 0; j < 4; ++j) {
-                double re = 0.0, im = 0.0;
-                for (int k = 0; k < 4; ++k) {
-                    const C2 a = gm[pmu[pl]][i][k], b = gm[pnu[pl]][k][j];
-                    const double pr = a.re * b.re - a.im * b.im, pi = a.re * b.im + a.im * b.re;
-                    re = re + pr;
-                    im = im + pi;
-                }
-                out.g[pl][i][j] = make_double2(re, im);
-            }
-    return out;
-}
-
-int launch_clover_pullback(lmx_context* ctx, double2* dU, const double2* U, double2* dF, const double2* dres,
+int launch_clover_pullback(lmx_context* ctx, double2* dU, const double2* U, double2* dQ, const double2* dres,
                            const double2* psi, double coefficient) {
     if (ctx->V == 0) return LMX_OK;
-    static const GammaProducts gp = gamma_products();
-    LMX_TRY(launch_zero(ctx, dF, 6 * 9 * (int64_t)ctx->V));
-    hipLaunchKernelGGL(k_clover_cotangent, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, dF, dres, psi,
-                       (int)ctx->V, coefficient, gp);
-    hipLaunchKernelGGL(k_clover_links_pullback, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, dU, U,
-                       (const double2*)dF, ctx->g);
+    hipLaunchKernelGGL(k_clover_cotangent, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, dQ, dres, psi,
+                       (int)ctx->V, coefficient);
+    hipLaunchKernelGGL(k_clover_links_pullback, dim3((unsigned)((ctx->V + 63) / 64)), dim3(256), 0, ctx->stream, dU, U,
+                       (const double2*)dQ, ctx->g);
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }

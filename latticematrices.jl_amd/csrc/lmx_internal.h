@@ -86,7 +86,7 @@ struct lmx_wilson {
     float2* clover32;
     __half2* clover16;
     bool lo_valid;
-    double2* clover_dF;  // scratch of the clover link pullback (6 planes), on first use
+    double2* clover_dQ;  // scratch of the clover link pullback (6 planes, 5 words each), on first use
     // Autotuned launch shape per (precision, nrhs); 0 = untuned.
     int tuned_block[4][65];
 };
@@ -243,7 +243,7 @@ int launch_cg_update_p_f32(lmx_context* ctx, const float2* r, float2* p, CGState
 // ---- pullback / TA (force.hip) ----
 int launch_pullback_f64(lmx_context* ctx, double2* dU, const double2* dres, const double2* psi, double coefficient);
 int launch_ta_project(lmx_context* ctx, double2* F, const double2* U, const double2* G);
-// clover part of the Wilson-clover link pullback (dF: 6*9*V scratch)
+// clover part of the Wilson-clover link pullback (dQ: 6*5*V scratch)
 // Boundary phases of a halo refill for fields of element type elem
 // (LMX_ELEM_*), exchange_dim_local! (src/LatticeMatrices_core.jl:707-723):
 // a plus ghost is the wrapped core value times the phase, a minus ghost times
@@ -268,7 +268,7 @@ int launch_randomize_padded(lmx_context* ctx, void* C, int elem, int nc1, int nc
                             const int32_t* gdims);
 int launch_spinor_randomize(lmx_context* ctx, void* dst, int nrhs, int dist, const lmx_rng_key* keys, double sigma,
                             int algorithm, const int32_t* goff, const int32_t* gdims);
-int launch_clover_pullback(lmx_context* ctx, double2* dU, const double2* U, double2* dF, const double2* dres,
+int launch_clover_pullback(lmx_context* ctx, double2* dU, const double2* U, double2* dQ, const double2* dres,
                            const double2* psi, double coefficient);
 
 // ---- batched / mixed CG (mixed.hip) ----

@@ -68,3 +68,20 @@ def test_cg(gpu, L):
     assert res.converged and res.iterations == ro.iterations
     assert np.array_equal(x.to_numpy(), xo)
     assert res.residual_norm == ro.residual_norm
+
+
+@pytest.mark.parametrize("L", [(2, 2, 2, 2), (3, 5, 3, 3), (1, 4, 5, 3), (8, 8, 4, 2)])
+def test_clover_link_pullback(gpu, L):
+    # blocks of 64 sites, a wavefront per link direction: fewer sites than a
+    # block, a cut last block, an extent of one (a neighbour is the site itself)
+    print(f"clover pullback L={L}", flush=True)
+    U = gen.links(L, "haar", 37)
+    psi, w = gen.gaussian_spinor(L, 38), gen.gaussian_spinor(L, 39)
+    lat = lmx.Lattice(L, ANTI)
+    D = lmx.WilsonDiracCloverOperator4D(lat.gauge_from_numpy(U), 0.12, 1.3)
+    dU = lmx.GaugeField(lat)
+    for _ in range(2):  # the second call adds to the first, and finds its scratch written
+        lmx.wilson_pullback_(dU, D, lat.spinor_from_numpy(w), lat.spinor_from_numpy(psi), -0.12)
+    ref = orc.clover_pullback(U, w, psi, L, -0.12, 1.3)
+    ref = orc.clover_pullback(U, w, psi, L, -0.12, 1.3, dU=ref)
+    assert np.array_equal(dU.to_numpy(), ref)
