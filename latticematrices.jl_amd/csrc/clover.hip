@@ -11,14 +11,16 @@
 
 namespace lmx {
 
-__device__ __forceinline__ void ld_link(const double2* __restrict__ U, int mu, int s, int V, cx<double> u[9]) {
+// A = A*B row by row with muladdmulti (_clover_mul_matrix3, :137-149)
+__device__ __forceinline__ void mul3(cx<double> (&A)[9], const cx<double> (&B)[9]) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        double2 v = U[(long)(mu * 9 + k) * V + s];
-        u[k] = mk<double>(v.x, v.y);
+    for (int i = 0; i < 3; ++i) {
+        const cx<double> a0 = A[3 * i], a1 = A[3 * i + 1], a2 = A[3 * i + 2];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) A[3 * i + j] = muladdmulti(a0, B[j], a1, B[3 + j], a2, B[6 + j]);
     }
 }
-__device__ __forceinline__ void dag3(cx<double> u[9]) {
+__device__ __forceinline__ void dag3(cx<double> (&u)[9]) {
     cx<double> t[9];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -27,81 +29,99 @@ __device__ __forceinline__ void dag3(cx<double> u[9]) {
 #pragma unroll
     for (int k = 0; k < 9; ++k) u[k] = t[k];
 }
-// _clover_mul_matrix3 (:137-149): C = A*B with muladdmulti rows
-__device__ __forceinline__ void mul3(const cx<double> A[9], const cx<double> B[9], cx<double> out[9]) {
-    cx<double> r[9];
+
+// keep a product in registers here: the loads that follow are not hoisted above it
+__device__ __forceinline__ void pin9(cx<double> (&a)[9]) {
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            r[3 * i + j] = muladdmulti(A[3 * i], B[j], A[3 * i + 1], B[3 + j], A[3 * i + 2], B[6 + j]);
-#pragma unroll
-    for (int k = 0; k < 9; ++k) out[k] = r[k];
+    for (int k = 0; k < 9; ++k) asm volatile("" : "+v"(a[k].re), "+v"(a[k].im)::"memory");
 }
 
-__device__ __forceinline__ int shift(int s, int mu, int dir, const Geom& g) {
+// U_mu(s) or its adjoint, mu the same in the whole wavefront
+template <bool DAG>
+__device__ __forceinline__ void ld_factor(const double2* __restrict__ U, int V, int mu, int s, cx<double> (&u)[9]) {
+    ld_comps(U + (size_t)mu * 9 * V, V, s, u);
+    if (DAG) dag3(u);
+}
+
+// a <- ((a*B)*C)*d with B, C loaded (each U or U^dagger), d given
+template <bool DB, bool DC>
+__device__ __forceinline__ void leaf(const double2* __restrict__ U, int V, cx<double> (&a)[9], int mb, int sb, int mc,
+                                     int sc, const cx<double> (&d)[9]) {
+    cx<double> b[9];
+    ld_factor<DB>(U, V, mb, sb, b);
+    mul3(a, b);
+    pin9(a);
+    ld_factor<DC>(U, V, mc, sc, b);
+    mul3(a, b);
+    mul3(a, d);
+    pin9(a);
+}
+
+// A wavefront of a workgroup takes one plane of the workgroup's 64 sites: the
+// six share their links in L1, a leaf's last link is the next leaf's first,
+// and blocks follow slab_block's order.  Bound by the 78 link loads (11.2 KB)
+// per site that pass through L1 (19 TB/s over the chip at 24^3 x 48; its 72
+// products are 131 us there with every lane busy); 400 us there and 76 us at
+// 16^3 x 32, against 868 and 155 us for one work item per site that kept all
+// planes' results in scratch, in lattice order over all XCDs.  Without pin9
+// the loads are hoisted and spilled (690 us), at 4 wavefronts per SIMD it
+// spills (1180), at 2 it waits (430).
+__global__ void __launch_bounds__(384, 3) k_clover_build(const double2* __restrict__ U, double2* __restrict__ F, Geom g,
+                                                         int slab) {
+    int s0, end;
+    slab_block(xcd_block(blockIdx.x, gridDim.x), slab, g, s0, end);
+    const int s = s0 + (threadIdx.x & 63);
+    if (s >= end) return;
+    const int pl = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int V = g.V;
+    const int mu = pl < 3 ? 0 : (pl < 5 ? 1 : 2), nu = pl < 3 ? pl + 1 : (pl < 5 ? pl - 1 : 3);
     int x[4];
     site_coords(s, g, x);
-    bool w;
-    return dir > 0 ? nbr_fwd(s, x, mu, g, w) : nbr_bwd(s, x, mu, g, w);
-}
-
-// leaf = ((A*B)*C)*D, with optional daggers on each factor
-__device__ __forceinline__ void leaf(const double2* __restrict__ U, int V, int ma, int sa, bool da, int mb, int sb,
-                                     bool db, int mc, int sc, bool dc, int md, int sd, bool dd, cx<double> out[9]) {
-    cx<double> a[9], b[9];
-    ld_link(U, ma, sa, V, a);
-    if (da) dag3(a);
-    ld_link(U, mb, sb, V, b);
-    if (db) dag3(b);
-    mul3(a, b, a);
-    ld_link(U, mc, sc, V, b);
-    if (dc) dag3(b);
-    mul3(a, b, a);
-    ld_link(U, md, sd, V, b);
-    if (dd) dag3(b);
-    mul3(a, b, out);
-}
-
-__global__ void __launch_bounds__(256) k_clover_build(const double2* __restrict__ U, double2* __restrict__ F, Geom g) {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= g.V) return;
-    const int V = g.V;
-    const int pmu[6] = {0, 0, 0, 1, 1, 2};
-    const int pnu[6] = {1, 2, 3, 2, 3, 3};
-    double dg[18];
-    cx<double> up[18];
-#pragma unroll 1
-    for (int pl = 0; pl < 6; ++pl) {
-        const int mu = pmu[pl], nu = pnu[pl];
-        const int xpmu = shift(s, mu, 1, g), xpnu = shift(s, nu, 1, g);
-        const int xmmu = shift(s, mu, -1, g), xmnu = shift(s, nu, -1, g);
-        const int xpnu_mmu = shift(xpnu, mu, -1, g);
-        const int xmmu_mnu = shift(xmmu, nu, -1, g);
-        const int xpmu_mnu = shift(xmnu, mu, 1, g);
-        cx<double> q[9], t[9];
-        leaf(U, V, mu, s, false, nu, xpmu, false, mu, xpnu, true, nu, s, true, q);
-        leaf(U, V, nu, s, false, mu, xpnu_mmu, true, nu, xmmu, true, mu, xmmu, false, t);
+    const int xm = mu == 0 ? x[0] : (mu == 1 ? x[1] : x[2]), xn = nu == 1 ? x[1] : (nu == 2 ? x[2] : x[3]);
+    // offsets of one step along each direction of the plane (they commute)
+    const int fm = xm == g.L[mu] - 1 ? -(g.L[mu] - 1) * g.stride[mu] : g.stride[mu];
+    const int bm = xm == 0 ? (g.L[mu] - 1) * g.stride[mu] : -g.stride[mu];
+    const int fn = xn == g.L[nu] - 1 ? -(g.L[nu] - 1) * g.stride[nu] : g.stride[nu];
+    const int bn = xn == 0 ? (g.L[nu] - 1) * g.stride[nu] : -g.stride[nu];
+    // each leaf's last factor is the next one's first, adjointed
+    cx<double> q[9], a[9], d[9];
+    ld_factor<false>(U, V, mu, s, q);
+    ld_factor<true>(U, V, nu, s, d);
+    leaf<false, true>(U, V, q, nu, s + fm, mu, s + fn, d);
+    dag3(d);
 #pragma unroll
-        for (int k = 0; k < 9; ++k) q[k] = cadd(q[k], t[k]);
-        leaf(U, V, mu, xmmu, true, nu, xmmu_mnu, true, mu, xmmu_mnu, false, nu, xmnu, false, t);
+    for (int k = 0; k < 9; ++k) a[k] = d[k];
+    ld_factor<false>(U, V, mu, s + bm, d);
+    leaf<true, true>(U, V, a, mu, s + fn + bm, nu, s + bm, d);
 #pragma unroll
-        for (int k = 0; k < 9; ++k) q[k] = cadd(q[k], t[k]);
-        leaf(U, V, nu, xmnu, true, mu, xmnu, false, nu, xpmu_mnu, false, mu, s, true, t);
+    for (int k = 0; k < 9; ++k) q[k] = cadd(q[k], a[k]);
+    dag3(d);
 #pragma unroll
-        for (int k = 0; k < 9; ++k) q[k] = cadd(q[k], t[k]);
-        const double f = 1.0 / 8.0;
-        dg[3 * pl + 0] = rmul(f, csub(q[0], cconj(q[0]))).im;
-        dg[3 * pl + 1] = rmul(f, csub(q[4], cconj(q[4]))).im;
-        dg[3 * pl + 2] = rmul(f, csub(q[8], cconj(q[8]))).im;
-        up[3 * pl + 0] = rmul(f, csub(q[1], cconj(q[3])));
-        up[3 * pl + 1] = rmul(f, csub(q[2], cconj(q[6])));
-        up[3 * pl + 2] = rmul(f, csub(q[5], cconj(q[7])));
+    for (int k = 0; k < 9; ++k) a[k] = d[k];
+    ld_factor<false>(U, V, nu, s + bn, d);
+    leaf<true, false>(U, V, a, nu, s + bm + bn, mu, s + bm + bn, d);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) q[k] = cadd(q[k], a[k]);
+    dag3(d);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) a[k] = d[k];
+    ld_factor<true>(U, V, mu, s, d);
+    leaf<false, false>(U, V, a, mu, s + bn, nu, s + bn + fm, d);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) q[k] = cadd(q[k], a[k]);
+    const double f = 1.0 / 8.0;
+    // diagonal i is half of slot (3 pl + i) / 2
+    double* diag = reinterpret_cast<double*>(F);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int e = 3 * pl + i;
+        diag[2 * ((size_t)(e >> 1) * V + s) + (e & 1)] = rmul(f, csub(q[4 * i], cconj(q[4 * i]))).im;
     }
-#pragma unroll
-    for (int qd = 0; qd < 9; ++qd) F[(long)qd * V + s] = make_double2(dg[2 * qd], dg[2 * qd + 1]);
-#pragma unroll
-    for (int qd = 0; qd < 18; ++qd) F[(long)(9 + qd) * V + s] = make_double2(up[qd].re, up[qd].im);
+    const cx<double> u0 = rmul(f, csub(q[1], cconj(q[3]))), u1 = rmul(f, csub(q[2], cconj(q[6]))),
+                     u2 = rmul(f, csub(q[5], cconj(q[7])));
+    F[(size_t)(9 + 3 * pl) * V + s] = make_double2(u0.re, u0.im);
+    F[(size_t)(10 + 3 * pl) * V + s] = make_double2(u1.re, u1.im);
+    F[(size_t)(11 + 3 * pl) * V + s] = make_double2(u2.re, u2.im);
 }
 
 // compact cache -> full planes [6][V][3][3] complex
@@ -143,7 +163,8 @@ __global__ void __launch_bounds__(256) k_convert(const double2* __restrict__ in,
 
 int launch_clover_build_f64(lmx_context* ctx, const double2* U, double2* clover) {
     if (ctx->V == 0) return LMX_OK;
-    hipLaunchKernelGGL(k_clover_build, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, U, clover, ctx->g);
+    const SlabOrder so = slab_order(ctx->g, false);
+    hipLaunchKernelGGL(k_clover_build, dim3((unsigned)so.blocks), dim3(384), 0, ctx->stream, U, clover, ctx->g, so.slab);
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }

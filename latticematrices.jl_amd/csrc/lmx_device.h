@@ -113,6 +113,41 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
     return (k < rem) ? k * (per + 1) + j : rem * (per + 1) + (k - rem) * per + j;
 }
 
+// Blocks of 64 consecutive sites, ordered slab by slab: `slab` blocks of a
+// t-slice, then the same blocks of the next slice, through all slices; then
+// the next slab.  With xcd_block and slabs of an eighth of the 3-D volume each
+// XCD keeps one slab, whose neighbours in t come round again while they are
+// still in its L2.  slab == 0: lattice order.
+constexpr int kSlabSites = 64;
+struct SlabOrder {
+    int slab;
+    long blocks;
+};
+// whole: blocks must not be cut by the end of a slice (else at most 1/32 of
+// the lanes idle there); slices of fewer blocks than XCDs make no slabs
+inline SlabOrder slab_order(const Geom& g, bool whole) {
+    const int V3 = g.stride[3], n3 = (V3 + kSlabSites - 1) / kSlabSites;
+    if (n3 >= 8 && (V3 % kSlabSites == 0 || (!whole && n3 >= 32))) return {(n3 + 7) / 8, (long)n3 * g.L[3]};
+    return {0, ((long)g.V + kSlabSites - 1) / kSlabSites};
+}
+// First site of block lb and the end of the sites it may take.
+__device__ __forceinline__ void slab_block(int lb, int slab, const Geom& g, int& s0, int& end) {
+    if (slab == 0) {
+        s0 = lb * kSlabSites;
+        end = g.V;
+        return;
+    }
+    const int V3 = g.stride[3], n3 = (V3 + kSlabSites - 1) / kSlabSites;
+    const int full = n3 / slab * slab * g.L[3];  // blocks in whole slabs
+    const bool tail = lb >= full;
+    const int n = tail ? n3 % slab : slab;
+    const int q = tail ? lb - full : lb % (slab * g.L[3]);
+    const int first = tail ? n3 / slab * slab : lb / (slab * g.L[3]) * slab;
+    const int t = q / n;
+    s0 = V3 * t + (first + q % n) * kSlabSites;
+    end = V3 * (t + 1);
+}
+
 // ---------------------------------------------------------------------------
 // Field accessors.  A spinor accessor moves the 12 colour-spin components
 // (k = spin*3 + colour) of right-hand side r at site s; a link accessor the
@@ -241,6 +276,27 @@ __device__ __forceinline__ float4 ldg_stream(const float4* base, int s) {
 __device__ __forceinline__ double2 ldg_stream(const double2* base, int s) {
     const lmx_dv2 v = ldg_raw<double2, lmx_dv2, LMX_NT_STREAM != 0>(base, s);
     return make_double2(v.x, v.y);
+}
+
+// Element s of the uniform base, the base held in scalar registers and the
+// lane's part a 32-bit offset: with the addresses left to the compiler, the 21
+// loads of a hop keep as many 64-bit lane addresses, and the kernel spills.
+template <typename V2, typename T>
+__device__ __forceinline__ V2 ld_sbase(const T* base, int s) {
+    using G = __attribute__((address_space(1))) const char*;
+    G b = (G)base;
+    asm("" : "+s"(b));
+    return *(__attribute__((address_space(1))) const V2*)(b + (unsigned)s * (unsigned)sizeof(V2));
+}
+// n components of stride V at site s
+template <int N, typename R, typename T>
+__device__ __forceinline__ void ld_comps(const T* base, int V, int s, cx<R> (&z)[N]) {
+    using V2 = R __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const V2 v = ld_sbase<V2>(base + (size_t)k * V, s);
+        z[k] = mk<R>(v.x, v.y);
+    }
 }
 
 struct SpF64In {

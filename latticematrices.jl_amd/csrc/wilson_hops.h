@@ -27,28 +27,7 @@
 
 namespace lmx {
 
-constexpr int kHopSites = 64;
-
-// Element s of the uniform base, the base held in scalar registers and the
-// lane's part a 32-bit offset: with the addresses left to the compiler, the 21
-// loads of a hop keep as many 64-bit lane addresses, and the kernel spills.
-template <typename V2, typename T>
-__device__ __forceinline__ V2 ld_sbase(const T* base, int s) {
-    using G = __attribute__((address_space(1))) const char*;
-    G b = (G)base;
-    asm("" : "+s"(b));
-    return *(__attribute__((address_space(1))) const V2*)(b + (unsigned)s * (unsigned)sizeof(V2));
-}
-// n components of stride V at site s
-template <int N, typename R, typename T>
-__device__ __forceinline__ void ld_comps(const T* base, int V, int s, cx<R> (&z)[N]) {
-    using V2 = R __attribute__((ext_vector_type(2)));
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const V2 v = ld_sbase<V2>(base + (size_t)k * V, s);
-        z[k] = mk<R>(v.x, v.y);
-    }
-}
+constexpr int kHopSites = kSlabSites;
 
 // U P psi of one hop (the reference's half-spin order), the boundary phase
 // applied where the neighbour wraps.
@@ -278,19 +257,8 @@ __global__ void __launch_bounds__(512, sizeof(typename In::R) == 8 ? 4 : 6) k_ho
     int lb = xcd_block(blockIdx.x, gridDim.x);
     const int r = lb % nrhs;
     lb /= nrhs;
-    int s0 = lb * kHopSites, end = g.V;
-    if (slab > 0) {
-        // `slab` 64-site blocks of a t-slice, then the same blocks of the next slice
-        const int V3 = g.stride[3], n3 = (V3 + kHopSites - 1) / kHopSites;
-        const int full = n3 / slab * slab * g.L[3];  // blocks in whole slabs
-        const bool tail = lb >= full;
-        const int n = tail ? n3 % slab : slab;
-        const int q = tail ? lb - full : lb % (slab * g.L[3]);
-        const int first = tail ? n3 / slab * slab : lb / (slab * g.L[3]) * slab;
-        const int t = q / n;
-        s0 = V3 * t + (first + q % n) * kHopSites;
-        end = V3 * (t + 1);
-    }
+    int s0, end;
+    slab_block(lb, slab, g, s0, end);
     const HopArgs<In, Lk, Out, Cl> a{out, in, U, F, aux, R(kappa_d), R(ccoef_d), r, epi.partials};
     switch (wave) {
 #define LMX_HOP_WAVE(W)                                                                   \
@@ -316,13 +284,9 @@ int launch_hops(lmx_context* ctx, Out out, In in, Lk U, Cl F, In aux, double kap
                 bool clover, const EpiArgs& epi) {
     const bool dag = (flags & LMX_DAGGER) != 0, donly = (flags & LMX_DONLY) != 0;
     const Geom& g = ctx->g;
-    const int V3 = g.stride[3], n3 = (V3 + kHopSites - 1) / kHopSites;
-    // slab order needs blocks that end with the slice: idle lanes where V3 is
-    // no multiple of 64 (at most 1/32 of them here; fewer blocks than XCDs are
-    // no slabs), and the 64-site sums of EPI_PAP need full blocks
-    const bool slabs = n3 >= 8 && (V3 % kHopSites == 0 || (EPI != EPI_PAP && n3 >= 32));
-    const int slab = slabs ? (n3 + 7) / 8 : 0;
-    const long nb = (slabs ? (long)n3 * g.L[3] : (ctx->V + kHopSites - 1) / kHopSites) * nrhs;
+    const SlabOrder so = slab_order(g, EPI == EPI_PAP);  // the sums of EPI_PAP need whole blocks
+    const int slab = so.slab;
+    const long nb = so.blocks * nrhs;
     LMX_CHECK(nb < (1L << 31), LMX_ERR_ARG, "too many right-hand sides (%d)", nrhs);
 #define LMX_HOPS(FPM, MODE, GP)                                                                                    \
     hipLaunchKernelGGL((k_hops<In, Lk, Out, Cl, FPM, MODE, EPI, GP>), dim3((unsigned)nb), dim3(512), 0, ctx->stream, \

@@ -85,3 +85,13 @@ def test_clover_link_pullback(gpu, L):
     ref = orc.clover_pullback(U, w, psi, L, -0.12, 1.3)
     ref = orc.clover_pullback(U, w, psi, L, -0.12, 1.3, dU=ref)
     assert np.array_equal(dU.to_numpy(), ref)
+
+
+@pytest.mark.parametrize("L", [(2, 2, 2, 2), (3, 5, 3, 3), (1, 4, 5, 3), (8, 8, 9, 4), (13, 13, 13, 3)])
+def test_field_strength(gpu, L):
+    # a wavefront per plane over the same blocks and slabs as the stencil
+    print(f"field strength L={L}", flush=True)
+    U = gen.links(L, "haar", 40)
+    lat = lmx.Lattice(L, ANTI)
+    D = lmx.WilsonDiracCloverOperator4D(lat.gauge_from_numpy(U), 0.12, 1.0)
+    assert np.array_equal(D.clover_planes(), orc.clover_field_strength(U, L))
