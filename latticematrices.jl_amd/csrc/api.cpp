@@ -152,6 +152,15 @@ static int noalloc_scratch_address(int device, void** out) {
     return LMX_OK;
 }
 
+// Lattices up to this volume take the small-lattice iteration (four launches
+// instead of six): 8^3 x 16 22 us an iteration against 34, 16^4 56 against 67,
+// but 16^3 x 32 112 against 104, where every block summing all partials costs
+// more than the two launches it saves.
+constexpr int64_t kSmallCgVolume = 1 << 16;
+static int small_cg_n64(const lmx_context* c) { return (int)((c->V + 63) / 64); }
+// Its second state record lies after the two rows of 64-site sums.
+static CGState* small_cg_state2(const lmx_context* c) { return (CGState*)(c->partials + 2 * small_cg_n64(c)); }
+
 // cg!(x, DdagDOp(D, tmp), b, r, p, Ap) in FP64 on the context c, whose
 // partials and state buffers the kernels use as their scratch.
 static int cg_ddagd_run(lmx_wilson* op, lmx_context* c, void* x, const void* b, void* r, void* p, void* Ap,
@@ -172,10 +181,30 @@ static int cg_ddagd_run(lmx_wilson* op, lmx_context* c, void* x, const void* b, 
     const int chunk = chunk_of(params);
     const long max_polls = (long)params->maxiter / chunk + 3;
     long polls = 0;
+    if (c->nc == 3 && c->V <= kSmallCgVolume) {
+        // small lattices (blas.hip): the state alternates between two records
+        CGState* st2 = small_cg_state2(c);
+        double *pap_w = c->partials, *rr_w = c->partials + small_cg_n64(c);
+        const Epilogue hop{0, nullptr, st, nullptr, nullptr}, hop_pap{1, P, st, pap_w, nullptr};
+        while (!c->host_state->done) {
+            LMX_CHECK(++polls <= max_polls, LMX_ERR_HIP, "CG state did not advance (iteration %d)",
+                      c->host_state->iteration);
+            for (int k = 0; k < chunk; ++k) {
+                LMX_TRY(launch_hops_f64(c, T, P, U, F, nullptr, op->kappa, op->csw, 1, 0, hop));
+                LMX_TRY(launch_hops_f64(c, AP, T, U, F, P, op->kappa, op->csw, 1, LMX_DAGGER, hop_pap));
+                LMX_TRY(launch_cg_small_r(c, R, AP, pap_w, rr_w, st, st2));
+                LMX_TRY(launch_cg_small_xp(c, X, R, P, rr_w, st2, st));
+            }
+            LMX_TRY(read_state(c, st, c->host_state));
+        }
+        fill_result(*c->host_state, result);
+        return LMX_OK;
+    }
+    int it = 0;
     while (!c->host_state->done) {
         LMX_CHECK(++polls <= max_polls, LMX_ERR_HIP, "CG state did not advance (iteration %d)",
                   c->host_state->iteration);
-        for (int k = 0; k < chunk; ++k) {
+        for (int k = 0; k < chunk; ++k, ++it) {
             LMX_TRY(launch_wilson_f64(c, U, F, op->kappa, op->csw, T, P, 1, 0, gate));
             if (c->nc == 3) {  // p.Ap fused into D^dagger's epilogue
                 LMX_TRY(launch_wilson_f64(c, U, F, op->kappa, op->csw, AP, T, 1, LMX_DAGGER, pap));
@@ -183,8 +212,8 @@ static int cg_ddagd_run(lmx_wilson* op, lmx_context* c, void* x, const void* b, 
                 LMX_TRY(launch_wilson_f64(c, U, F, op->kappa, op->csw, AP, T, 1, LMX_DAGGER, gate));
                 LMX_TRY(launch_dot(c, P, AP, FIN_PAP, st, nullptr));
             }
-            LMX_TRY(launch_cg_update_xr(c, X, R, P, AP, st));
-            LMX_TRY(launch_cg_update_p(c, R, P, st));
+            LMX_TRY(launch_cg_update_r(c, R, AP, st));
+            LMX_TRY(launch_cg_update_xp(c, X, R, P, st, it));
         }
         LMX_TRY(read_state(c, st, c->host_state));
     }
@@ -227,15 +256,16 @@ static int cg_ddagd_run_f32(lmx_wilson* op, lmx_context* c, float2* X, const flo
     const int chunk = chunk_of(params);
     const long max_polls = (long)params->maxiter / chunk + 3;
     long polls = 0;
+    int it = 0;
     while (!c->host_state->done) {
         LMX_CHECK(++polls <= max_polls, LMX_ERR_HIP, "CG state did not advance (iteration %d)",
                   c->host_state->iteration);
-        for (int k = 0; k < chunk; ++k) {
+        for (int k = 0; k < chunk; ++k, ++it) {
             LMX_TRY(apply_f32_gated(op, T, P, 0, st));
             LMX_TRY(apply_f32_gated(op, AP, T, LMX_DAGGER, st));
             LMX_TRY(launch_dot_f32(c, P, AP, FIN_PAP, st, nullptr));
-            LMX_TRY(launch_cg_update_xr_f32(c, X, R, P, AP, st));
-            LMX_TRY(launch_cg_update_p_f32(c, R, P, st));
+            LMX_TRY(launch_cg_update_r_f32(c, R, AP, st));
+            LMX_TRY(launch_cg_update_xp_f32(c, X, R, P, st, it));
         }
         LMX_TRY(read_state(c, st, c->host_state));
     }
@@ -756,13 +786,13 @@ int lmx_cg_generic(lmx_context* c, lmx_apply_fn A, void* A_user, void* x, const 
         LMX_TRY(read_state(c, st, c->host_state));
     }
     long polls = 0;
-    while (!c->host_state->done) {
+    for (int it = 0; !c->host_state->done; ++it) {
         LMX_CHECK(++polls <= (long)params->maxiter + 2, LMX_ERR_HIP, "CG state did not advance (iteration %d)",
                   c->host_state->iteration);
         LMX_CHECK(A(A_user, AP, P, c->stream) == 0, LMX_ERR_ARG, "operator callback failed");
         LMX_TRY(launch_dot(c, P, AP, 4, st, nullptr));
-        LMX_TRY(launch_cg_update_xr(c, X, R, P, AP, st));
-        LMX_TRY(launch_cg_update_p(c, R, P, st));
+        LMX_TRY(launch_cg_update_r(c, R, AP, st));
+        LMX_TRY(launch_cg_update_xp(c, X, R, P, st, it));
         LMX_TRY(read_state(c, st, c->host_state));
     }
     fill_result(*c->host_state, result);

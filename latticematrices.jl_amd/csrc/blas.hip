@@ -206,16 +206,13 @@ __global__ void __launch_bounds__(256) k_cg_setup_r(const typename Vec2<R>::T* _
     store_partials(re, 0.0, false, lb, partials);
 }
 
-// x = alpha*p + x; r = (-alpha)*Ap + r; rr_new = |r|^2  (cg.jl:116-120)
+// r = (-alpha)*Ap + r; rr_new = |r|^2  (cg.jl:117-120)
 template <int NCOMP, typename R = double>
-__global__ void __launch_bounds__(256) k_cg_update_xr(typename Vec2<R>::T* __restrict__ x,
-                                                      typename Vec2<R>::T* __restrict__ r,
-                                                      const typename Vec2<R>::T* __restrict__ p,
-                                                      const typename Vec2<R>::T* __restrict__ Ap, int V,
-                                                      double* partials, CGState* st) {
+__global__ void __launch_bounds__(256) k_cg_update_r(typename Vec2<R>::T* __restrict__ r,
+                                                     const typename Vec2<R>::T* __restrict__ Ap, int V,
+                                                     double* partials, CGState* st) {
     if (st->done) return;
-    const R alpha = R(st->alpha);
-    const R malpha = -alpha;
+    const R malpha = -R(st->alpha);
     const int lb = blockIdx.x;
     const int s = lb * 256 + threadIdx.x;
     double re = 0.0;
@@ -224,12 +221,9 @@ __global__ void __launch_bounds__(256) k_cg_update_xr(typename Vec2<R>::T* __res
 #pragma unroll
         for (int k = 0; k < NCOMP; ++k) {
             const long i = (long)k * V + s;
-            auto pv = p[i], xv = x[i], av = Ap[i], rv = r[i];
-            xv.x = alpha * pv.x + R(1) * xv.x;
-            xv.y = alpha * pv.y + R(1) * xv.y;
+            auto av = Ap[i], rv = r[i];
             rv.x = malpha * av.x + R(1) * rv.x;
             rv.y = malpha * av.y + R(1) * rv.y;
-            x[i] = xv;
             r[i] = rv;
             cx<R> rc = mk<R>(rv.x, rv.y);
             acc = cadd(acc, cmul(cconj(rc), rc));
@@ -239,21 +233,145 @@ __global__ void __launch_bounds__(256) k_cg_update_xr(typename Vec2<R>::T* __res
     store_partials(re, 0.0, false, lb, partials);
 }
 
-// p = 1*r + beta*p  (cg.jl:130-131)
+// x = alpha*p + x  (cg.jl:116), p = 1*r + beta*p  (cg.jl:130-131): one pass
+// reads p for both.  It runs after iteration `it` (from zero) has been counted,
+// so also on the one that ended the solve (x only), and not again after it.
 template <int NCOMP, typename R = double>
-__global__ void __launch_bounds__(256) k_cg_update_p(const typename Vec2<R>::T* __restrict__ r,
-                                                     typename Vec2<R>::T* __restrict__ p, int V, CGState* st) {
-    if (st->done) return;
-    const R beta = R(st->beta);
+__global__ void __launch_bounds__(256) k_cg_update_xp(typename Vec2<R>::T* __restrict__ x,
+                                                      const typename Vec2<R>::T* __restrict__ r,
+                                                      typename Vec2<R>::T* __restrict__ p, int V, const CGState* st,
+                                                      int it) {
+    if (st->iteration != it + 1) return;
+    const R alpha = R(st->alpha), beta = R(st->beta);
+    const bool more = !st->done;
     const int s = blockIdx.x * 256 + threadIdx.x;
     if (s < V) {
 #pragma unroll
         for (int k = 0; k < NCOMP; ++k) {
             const long i = (long)k * V + s;
-            auto rv = r[i], pv = p[i];
-            pv.x = R(1) * rv.x + beta * pv.x;
-            pv.y = R(1) * rv.y + beta * pv.y;
-            p[i] = pv;
+            auto xv = x[i], pv = p[i];
+            xv.x = alpha * pv.x + R(1) * xv.x;
+            xv.y = alpha * pv.y + R(1) * xv.y;
+            x[i] = xv;
+            if (more) {
+                const auto rv = r[i];
+                pv.x = R(1) * rv.x + beta * pv.x;
+                pv.y = R(1) * rv.y + beta * pv.y;
+                p[i] = pv;
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The FP64 iteration of small lattices (NC = 3), where launches and latency
+// are what it costs.  The vector kernels sum the partials of the reduction
+// before them themselves (every block the same sum, in k_finalize's order),
+// and a block is 64 sites by four groups of three components, so a lattice
+// makes four times the blocks.  The state goes from one record to another: a
+// kernel reads the one and its block 0 writes the other, so no block reads
+// what another writes.
+// ---------------------------------------------------------------------------
+// The sum of n64 partials of 64 sites each, in all of the block's 256 threads.
+__device__ __forceinline__ double sum_wave_partials(const double* w, int n64, double* lds4) {
+    const int nb = (n64 + 3) / 4;
+    double acc = 0.0;
+    for (int b = threadIdx.x; b < nb; b += kRedBlock) acc = acc + wave_quad(w, b, n64);
+    acc = wave_halve(acc);
+    if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    return (lds4[0] + lds4[2]) + (lds4[1] + lds4[3]);
+}
+
+// p.Ap is known: alpha, and r = (-alpha)*Ap + r with |r|^2 per 64 sites.
+__global__ void __launch_bounds__(256) k_cg_small_r(double2* __restrict__ r, const double2* __restrict__ Ap, int V,
+                                                    const double* __restrict__ pap, double* __restrict__ rr, int n64,
+                                                    const CGState* __restrict__ in, CGState* __restrict__ out) {
+    __shared__ double lds4[4];
+    __shared__ double term[12][64];
+    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int s = blockIdx.x * 64 + lane;
+    const bool live = s < V;
+    double2 rv[3], av[3];
+    if (live) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            rv[k] = r[(size_t)(3 * grp + k) * V + s];
+            av[k] = Ap[(size_t)(3 * grp + k) * V + s];
+        }
+    }
+    const bool was_done = in->done != 0;
+    const double pAp = was_done ? 0.0 : sum_wave_partials(pap, n64, lds4);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *out = *in;
+        if (!was_done) finalize_scalar(FIN_PAP, out, pAp, 0.0, nullptr);
+    }
+    if (was_done || !isfinite(pAp) || pAp <= 0.0) return;  // as FIN_PAP ends the solve
+    const double malpha = -(in->rr / pAp);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        double t = 0.0;
+        if (live) {
+            double2 v;
+            v.x = malpha * av[k].x + 1.0 * rv[k].x;
+            v.y = malpha * av[k].y + 1.0 * rv[k].y;
+            r[(size_t)(3 * grp + k) * V + s] = v;
+            const cx<double> rc = mk<double>(v.x, v.y);
+            t = cmul(cconj(rc), rc).re;
+        }
+        term[3 * grp + k][lane] = t;
+    }
+    __syncthreads();
+    if (grp == 0) {
+        double v = 0.0;
+#pragma unroll
+        for (int k = 0; k < 12; ++k) v = v + term[k][lane];
+        v = wave_halve(v);
+        if (lane == 0) rr[blockIdx.x] = v;
+    }
+}
+
+// |r|^2 is known: beta and the stopping test; x = alpha*p + x and, unless the
+// solve has ended, p = r + beta*p.
+__global__ void __launch_bounds__(256) k_cg_small_xp(double2* __restrict__ x, const double2* __restrict__ r,
+                                                     double2* __restrict__ p, int V, const double* __restrict__ rr,
+                                                     int n64, const CGState* __restrict__ in,
+                                                     CGState* __restrict__ out) {
+    __shared__ double lds4[4];
+    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int s = blockIdx.x * 64 + lane;
+    const bool live = s < V;
+    double2 xv[3], pv[3], rv[3];
+    if (live) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const size_t i = (size_t)(3 * grp + k) * V + s;
+            xv[k] = x[i];
+            pv[k] = p[i];
+            rv[k] = r[i];
+        }
+    }
+    const bool was_done = in->done != 0;
+    const double rr_new = was_done ? 0.0 : sum_wave_partials(rr, n64, lds4);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *out = *in;
+        if (!was_done) finalize_scalar(FIN_RRNEW, out, rr_new, 0.0, nullptr);
+    }
+    if (was_done || !live) return;
+    const double alpha = in->alpha, beta = rr_new / in->rr;
+    // as FIN_RRNEW ends the solve
+    const bool ended = !isfinite(rr_new) || rr_new < 0.0 || sqrt(rr_new) <= in->tol || in->iteration + 1 >= in->maxiter;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const size_t i = (size_t)(3 * grp + k) * V + s;
+        double2 v;
+        v.x = alpha * pv[k].x + 1.0 * xv[k].x;
+        v.y = alpha * pv[k].y + 1.0 * xv[k].y;
+        x[i] = v;
+        if (!ended) {
+            v.x = 1.0 * rv[k].x + beta * pv[k].x;
+            v.y = 1.0 * rv[k].y + beta * pv[k].y;
+            p[i] = v;
         }
     }
 }
@@ -330,22 +448,42 @@ int launch_cg_setup_r(lmx_context* ctx, const double2* b, const double2* Ap, dou
     return launch_finalize(ctx, nblocks(ctx->V), FIN_RR0, false, st, nullptr);
 }
 
-int launch_cg_update_xr(lmx_context* ctx, double2* x, double2* r, const double2* p, const double2* Ap, CGState* st) {
+int launch_cg_update_r(lmx_context* ctx, double2* r, const double2* Ap, CGState* st) {
     if (ctx->nc == 3)
-        hipLaunchKernelGGL(k_cg_update_xr<12>, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, x, r, p, Ap,
-                           (int)ctx->V, ctx->partials, st);
+        hipLaunchKernelGGL(k_cg_update_r<12>, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, r, Ap, (int)ctx->V,
+                           ctx->partials, st);
     else
-        hipLaunchKernelGGL(k_cg_update_xr<8>, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, x, r, p, Ap,
-                           (int)ctx->V, ctx->partials, st);
+        hipLaunchKernelGGL(k_cg_update_r<8>, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, r, Ap, (int)ctx->V,
+                           ctx->partials, st);
     LMX_HIP(hipGetLastError());
     return launch_finalize(ctx, nblocks(ctx->V), FIN_RRNEW, false, st, nullptr);
 }
 
-int launch_cg_update_p(lmx_context* ctx, const double2* r, double2* p, CGState* st) {
+int launch_cg_update_xp(lmx_context* ctx, double2* x, const double2* r, double2* p, const CGState* st, int it) {
     if (ctx->nc == 3)
-        hipLaunchKernelGGL(k_cg_update_p<12>, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, r, p, (int)ctx->V, st);
+        hipLaunchKernelGGL(k_cg_update_xp<12>, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, x, r, p, (int)ctx->V,
+                           st, it);
     else
-        hipLaunchKernelGGL(k_cg_update_p<8>, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, r, p, (int)ctx->V, st);
+        hipLaunchKernelGGL(k_cg_update_xp<8>, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, x, r, p, (int)ctx->V,
+                           st, it);
+    LMX_HIP(hipGetLastError());
+    return LMX_OK;
+}
+
+static inline int n64_of(const lmx_context* ctx) { return (int)((ctx->V + 63) / 64); }
+
+int launch_cg_small_r(lmx_context* ctx, double2* r, const double2* Ap, const double* pap, double* rr, const CGState* in,
+                      CGState* out) {
+    const int n = n64_of(ctx);
+    hipLaunchKernelGGL(k_cg_small_r, dim3(n), dim3(256), 0, ctx->stream, r, Ap, (int)ctx->V, pap, rr, n, in, out);
+    LMX_HIP(hipGetLastError());
+    return LMX_OK;
+}
+
+int launch_cg_small_xp(lmx_context* ctx, double2* x, const double2* r, double2* p, const double* rr, const CGState* in,
+                       CGState* out) {
+    const int n = n64_of(ctx);
+    hipLaunchKernelGGL(k_cg_small_xp, dim3(n), dim3(256), 0, ctx->stream, x, r, p, (int)ctx->V, rr, n, in, out);
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }
@@ -367,16 +505,16 @@ int launch_cg_setup_r_f32(lmx_context* ctx, const float2* b, const float2* Ap, f
     return launch_finalize(ctx, nblocks(ctx->V), FIN_RR0, false, st, nullptr);
 }
 
-int launch_cg_update_xr_f32(lmx_context* ctx, float2* x, float2* r, const float2* p, const float2* Ap, CGState* st) {
-    hipLaunchKernelGGL((k_cg_update_xr<12, float>), dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, x, r, p, Ap,
+int launch_cg_update_r_f32(lmx_context* ctx, float2* r, const float2* Ap, CGState* st) {
+    hipLaunchKernelGGL((k_cg_update_r<12, float>), dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, r, Ap,
                        (int)ctx->V, ctx->partials, st);
     LMX_HIP(hipGetLastError());
     return launch_finalize(ctx, nblocks(ctx->V), FIN_RRNEW, false, st, nullptr);
 }
 
-int launch_cg_update_p_f32(lmx_context* ctx, const float2* r, float2* p, CGState* st) {
-    hipLaunchKernelGGL((k_cg_update_p<12, float>), dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, r, p,
-                       (int)ctx->V, st);
+int launch_cg_update_xp_f32(lmx_context* ctx, float2* x, const float2* r, float2* p, const CGState* st, int it) {
+    hipLaunchKernelGGL((k_cg_update_xp<12, float>), dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, x, r, p,
+                       (int)ctx->V, st, it);
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }

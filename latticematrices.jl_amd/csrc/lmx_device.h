@@ -969,16 +969,17 @@ __device__ __forceinline__ double finish_partials(const double* partials, int nb
     return block_tree(acc, lds4);
 }
 
-// The same from the sums of 64 consecutive sites (n64 of them; a block's
-// missing ones are zero, as block_tree finds its idle wavefronts).
+// The partial of 256-site block b from the sums w of 64 consecutive sites (n64
+// of them; missing ones are zero, as block_tree finds its idle wavefronts).
+__device__ __forceinline__ double wave_quad(const double* w, int b, int n64) {
+    const int k = 4 * b;
+    const double w0 = w[k], w1 = k + 1 < n64 ? w[k + 1] : 0.0, w2 = k + 2 < n64 ? w[k + 2] : 0.0,
+                 w3 = k + 3 < n64 ? w[k + 3] : 0.0;
+    return (w0 + w2) + (w1 + w3);
+}
 __device__ __forceinline__ double finish_wave_partials(const double* w, int nb, int n64, double* lds4) {
     double acc = 0.0;
-    for (int b = threadIdx.x; b < nb; b += kRedBlock) {
-        const int k = 4 * b;
-        const double w0 = w[k], w1 = k + 1 < n64 ? w[k + 1] : 0.0, w2 = k + 2 < n64 ? w[k + 2] : 0.0,
-                     w3 = k + 3 < n64 ? w[k + 3] : 0.0;
-        acc = acc + ((w0 + w2) + (w1 + w3));
-    }
+    for (int b = threadIdx.x; b < nb; b += kRedBlock) acc = acc + wave_quad(w, b, n64);
     return block_tree(acc, lds4);
 }
 

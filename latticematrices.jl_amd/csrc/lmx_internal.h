@@ -231,14 +231,19 @@ int launch_axpby(lmx_context* ctx, double a, const double2* X, double b, double2
 int launch_zero(lmx_context* ctx, double2* p, int64_t n);
 int launch_scale(lmx_context* ctx, double2* out, const double2* in, double sr, double si, int64_t n);
 int launch_cg_setup_r(lmx_context* ctx, const double2* b, const double2* Ap, double2* r, double2* p, CGState* st);
-int launch_cg_update_xr(lmx_context* ctx, double2* x, double2* r, const double2* p, const double2* Ap, CGState* st);
-int launch_cg_update_p(lmx_context* ctx, const double2* r, double2* p, CGState* st);
+int launch_cg_update_r(lmx_context* ctx, double2* r, const double2* Ap, CGState* st);
+int launch_cg_update_xp(lmx_context* ctx, double2* x, const double2* r, double2* p, const CGState* st, int it);
+// the small-lattice iteration: pap, rr one sum per 64 sites; in is read, out written
+int launch_cg_small_r(lmx_context* ctx, double2* r, const double2* Ap, const double* pap, double* rr, const CGState* in,
+                      CGState* out);
+int launch_cg_small_xp(lmx_context* ctx, double2* x, const double2* r, double2* p, const double* rr, const CGState* in,
+                       CGState* out);
 int launch_cg_init_state(lmx_context* ctx, CGState* st, double rtol, double atol, int maxiter);
 // the same on ComplexF32 fields (float2 [12][V]; NC = 3)
 int launch_dot_f32(lmx_context* ctx, const float2* A, const float2* B, int fin_kind, CGState* st, double* out2);
 int launch_cg_setup_r_f32(lmx_context* ctx, const float2* b, const float2* Ap, float2* r, float2* p, CGState* st);
-int launch_cg_update_xr_f32(lmx_context* ctx, float2* x, float2* r, const float2* p, const float2* Ap, CGState* st);
-int launch_cg_update_p_f32(lmx_context* ctx, const float2* r, float2* p, CGState* st);
+int launch_cg_update_r_f32(lmx_context* ctx, float2* r, const float2* Ap, CGState* st);
+int launch_cg_update_xp_f32(lmx_context* ctx, float2* x, const float2* r, float2* p, const CGState* st, int it);
 
 // ---- pullback / TA (force.hip) ----
 int launch_pullback_f64(lmx_context* ctx, double2* dU, const double2* dres, const double2* psi, double coefficient);

@@ -95,3 +95,34 @@ def test_field_strength(gpu, L):
     lat = lmx.Lattice(L, ANTI)
     D = lmx.WilsonDiracCloverOperator4D(lat.gauge_from_numpy(U), 0.12, 1.0)
     assert np.array_equal(D.clover_planes(), orc.clover_field_strength(U, L))
+
+
+@pytest.mark.parametrize("L", [(4, 4, 4, 4), (16, 16, 16, 17)])  # the small-lattice iteration and the general one
+@pytest.mark.parametrize("maxiter", [0, 1, 17])  # none, one, and one into the second batch of launches
+def test_cg_stops_at_maxiter(gpu, L, maxiter):
+    print(f"CG maxiter L={L} maxiter={maxiter}", flush=True)
+    U = gen.links(L, "weak", 41)
+    b, x0 = gen.gaussian_spinor(L, 42), gen.gaussian_spinor(L, 43)
+    xo, ro = orc.cg(orc.NormalOp(orc.OP_DDAGD_WILSON, L, U=U, kappa=0.12), b, x0=x0, rtol=1e-10, maxiter=maxiter,
+                    order=1)
+    lat = lmx.Lattice(L, ANTI)
+    D = lmx.WilsonDiracOperator4D(lat.gauge_from_numpy(U), 0.12)
+    r, p, Ap, tmp = (lat.spinor() for _ in range(4))
+    x = lat.spinor_from_numpy(x0)
+    res = lmx.cg_(x, lmx.DdagDOp(D, tmp), lat.spinor_from_numpy(b), r, p, Ap, rtol=1e-10, maxiter=maxiter)
+    assert not res.converged and res.reason == ro.reason and res.iterations == ro.iterations == maxiter
+    assert np.array_equal(x.to_numpy(), xo)
+    assert res.residual_norm == ro.residual_norm
+
+
+@pytest.mark.parametrize("L", [(4, 4, 4, 4), (16, 16, 16, 17)])
+def test_cg_first_iteration_converges(gpu, L):
+    # zero links: D = 1, so the solve ends in the iteration whose x update is still to come
+    print(f"CG one iteration L={L}", flush=True)
+    lat = lmx.Lattice(L, ANTI)
+    D = lmx.WilsonDiracOperator4D(lmx.GaugeField(lat), 0.12)
+    b = lat.spinor_from_numpy(gen.gaussian_spinor(L, 44))
+    x, r, p, Ap, tmp = (lat.spinor() for _ in range(5))
+    res = lmx.cg_(x, lmx.DdagDOp(D, tmp), b, r, p, Ap, rtol=1e-10)
+    assert res.converged and res.iterations == 1 and res.residual_norm == 0.0
+    assert np.array_equal(x.to_numpy(), b.to_numpy())
