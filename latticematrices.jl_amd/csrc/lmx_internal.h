@@ -114,7 +114,7 @@ int launch_wilson_f64(lmx_context* ctx, const double2* U, const double2* clover,
 // The same by the eight-wavefront kernel (wilson_hops.hip), and whether it is
 // the faster one on this lattice.  Epilogue kind 1 leaves one p.Ap sum per 64
 // consecutive sites in e.partials (for launch_finalize's `waves`).
-bool hops_f64(const lmx_context* ctx, bool clover);
+bool hops_f64(const lmx_context* ctx, int nrhs, bool clover);
 int launch_hops_f64(lmx_context* ctx, double2* out, const double2* in, const double2* U, const double2* clover,
                     const double2* p, double kappa, double csw, int nrhs, int flags, const Epilogue& e);
 // FP64 D^dagger of the mixed solver's reliable update with the true residual
@@ -204,6 +204,9 @@ struct LoArgs {
     const CGState* st;
 };
 int launch_wilson_lo(lmx_context* ctx, const LoArgs& a);
+// The FP32 apply without an epilogue by the eight-wavefront kernel, and whether it is the faster one.
+bool hops_f32(const lmx_context* ctx, int nrhs, bool clover);
+int launch_hops_f32(lmx_context* ctx, const LoArgs& a);
 
 int launch_clover_build_f64(lmx_context* ctx, const double2* U, double2* clover);
 int launch_clover_export(lmx_context* ctx, const double2* clover, double2* F_out);

@@ -29,10 +29,9 @@ int launch_wilson_f64(lmx_context* ctx, const double2* U, const double2* clover,
     F64Clover F{clover};
     EpiArgs epi{e.partials, 0, e.st, e.gate};
     const NoEx none{};
-    // one field, or clover fields (one at a time): the eight-wavefront kernel
-    // where it is the faster one; a gated launch, which mostly only finds its
-    // gate off, keeps the smaller grids
-    const bool hops = (nrhs == 1 || clover != nullptr) && e.gate == nullptr && hops_f64(ctx, clover != nullptr);
+    // the eight-wavefront kernel where it is the faster one; a gated launch,
+    // which mostly only finds its gate off, keeps the smaller grids
+    const bool hops = e.gate == nullptr && hops_f64(ctx, nrhs, clover != nullptr);
     if (hops) {
         LMX_TRY(launch_hops_f64(ctx, out, in, U, clover, e.aux, kappa, csw, nrhs, flags, e));
         return e.kind == 1 ? launch_finalize(ctx, nblocks(ctx->V), FIN_PAP, false, e.st, nullptr, true) : LMX_OK;
@@ -116,6 +115,8 @@ int launch_wilson_lo(lmx_context* ctx, const LoArgs& a) {
     if (ctx->V == 0 || a.nrhs == 0) return LMX_OK;
     const bool cl = a.clover != nullptr;
     const int V = (int)ctx->V;
+    if (a.link_prec == LMX_F32 && a.spinor_prec == LMX_F32 && a.epi == EPI_NONE && hops_f32(ctx, a.nrhs, cl))
+        return launch_hops_f32(ctx, a);
     if (a.link_prec == LMX_F32 && a.spinor_prec == LMX_F32)
         return launch_lo_sp<SpF32In, SpF32Out>(ctx, a, LinkF32{(const float2*)a.links, V},
                                                F32Clover{(const float2*)a.clover}, cl);

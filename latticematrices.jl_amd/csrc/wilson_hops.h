@@ -1,6 +1,5 @@
 // wilson_hops.h -- the Wilson(-clover) stencil with the eight hops of a site
-// on eight wavefronts (FP64 and FP32 fields, one right-hand side per
-// workgroup).
+// on eight wavefronts (FP64 and FP32 fields).
 //
 // A workgroup of 512 work items owns 64 consecutive sites: lane i of every
 // wavefront is site i, wavefront 2 mu the forward and 2 mu + 1 the backward
@@ -8,18 +7,21 @@
 // link, forms its half-spinor U P psi and leaves it in LDS; after one barrier
 // wavefronts 0-5 each sum two of the site's twelve components over the eight
 // hops, in the reference's order, and write them (results bit-identical to
-// k_site's and k_stream's).
+// k_site's and k_stream's).  Several right-hand sides take their turns in the
+// workgroup with the links kept in registers, the next one's spinors in
+// flight while the last one's components are summed.
 //
 // Why: with the hops one after the other in one work item (k_site, k_stream)
 // a site waits for nine loads in turn, at 230-256 VGPRs and one or two
-// wavefronts per SIMD.  Here it waits for one, at 128 VGPRs and four per SIMD
-// (two workgroups per CU; 60 KB of LDS each in FP64), at the price of 1.5 KB
-// of LDS traffic per site and of the neighbours in t read again.  To keep
-// those in L2 the blocks are ordered slab by slab: an eighth of the 3-D
-// volume, which is one XCD's share, for t = 0, 1, ... (lattice order instead:
-// 174 against 148 us at 24^3 x 48, 3400 against 2650 us at 48^3 x 96; tiles in
-// y and z, nontemporal loads of links and a walk over t within the workgroup
-// were no faster).
+// wavefronts per SIMD in FP64.  Here it waits for one, at 88 VGPRs and five
+// wavefronts per SIMD, at the price of 1.5 KB of LDS traffic per site and of
+// the neighbours in t read again.  To keep those in L2 the blocks are ordered
+// slab by slab: an eighth of the 3-D volume, which is one XCD's share, for
+// t = 0, 1, ... (lattice order instead: 174 against 148 us at 24^3 x 48, 3400
+// against 2650 us at 48^3 x 96; tiles in y and z, nontemporal loads of links
+// and a walk over t within the workgroup were no faster).  Bound by the L2
+// misses that remain (24^3 x 48: 0.79 GB moved at 5.3 TB/s, 1.23x the fields
+// themselves).
 //
 #pragma once
 
@@ -88,11 +90,19 @@ struct alignas(2 * sizeof(R)) LdsCx {
         return mk<R>(v.x, v.y);
     }
 };
-template <typename R>
+template <typename R, int MODE>
 struct HopLds {
-    LdsCx<R> hop[8][6][kHopSites];  // U P psi of each hop: [hop][2 colour + half-spin][site]
-    LdsCx<R> psi[12][kHopSites];    // the site's own spinor
+    LdsCx<R> hop[8][6][kHopSites];                            // U P psi of each hop: [hop][2 colour + half-spin][site]
+    LdsCx<R> psi[MODE == MODE_CLOVER ? 12 : 1][kHopSites];  // the site's own spinor, for the clover term
 };
+// two components of the site's own spinor
+template <typename R, typename T>
+__device__ __forceinline__ void ld_own(const T* spin, int V, int ka, int kb, int s, cx<R> (&z)[2]) {
+    using V2 = R __attribute__((ext_vector_type(2)));
+    const V2 a = ld_sbase<V2>(spin + (size_t)ka * V, s), b = ld_sbase<V2>(spin + (size_t)kb * V, s);
+    z[0] = mk<R>(a.x, a.y);
+    z[1] = mk<R>(b.x, b.y);
+}
 
 template <int FPM, bool HIGH, typename R>
 __device__ __forceinline__ void sum_hops(const LdsCx<R> (&hop)[8][6][kHopSites], int c, int lane, cx<R>& a, cx<R>& b) {
@@ -168,73 +178,80 @@ struct HopArgs {
     Cl F;
     In aux;  // p of EPI_PAP
     typename In::R kappa, ccoef;
-    int r;
+    int r0, r1;  // the workgroup's right-hand sides
     double* partials;
 };
 
 // Wavefront W's part of the workgroup (hop W; the sum of two components for W < 6).
-template <int W, int FPM, int MODE, int EPI, bool GP, class In, class Lk, class Out, class Cl>
-__device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopLds<typename In::R>& sh,
+template <int W, int FPM, int MODE, int EPI, bool GP, bool LOOP, class In, class Lk, class Out, class Cl>
+__device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopLds<typename In::R, MODE>& sh,
                                          double (*pap)[kHopSites], const Geom& g, int s0, int lane, int end) {
     using R = typename In::R;
     constexpr int MU = W >> 1;
     constexpr bool FWD = (W & 1) == 0;
     constexpr int PM = FWD ? FPM : -FPM;
-    const auto* spin = a.in.p + (size_t)a.r * 12 * g.V;
-    const auto* link = a.U.p + (size_t)MU * 9 * g.V;
+    // the summed components: colour c, spins (0, 1) or (2, 3)
+    constexpr int c = W >> 1;
+    constexpr bool kHigh = (W & 1) != 0;
+    constexpr int ka = (kHigh ? 6 : 0) + c, kb = ka + 3;
     int s = s0 + lane;
     const bool live = s < end;
     if (!live) s = end - 1;  // a ragged last block: recompute, do not store
     int x[4];
     site_coords(s, g, x);
     bool w;
-    cx<R> psi[12], u[9];
-    {
-        const int t = FWD ? nbr_fwd(s, x, MU, g, w) : nbr_bwd(s, x, MU, g, w);
-        ld_comps(link, g.V, FWD ? s : t, u);
-        ld_comps(spin, g.V, t, psi);
-        if constexpr (W == 6) {  // the site's own spinor
-            cx<R> p[12];
-            ld_comps(spin, g.V, s, p);
+    const int t = FWD ? nbr_fwd(s, x, MU, g, w) : nbr_bwd(s, x, MU, g, w);
+    cx<R> psi[12], u[9], own[2];
+    const auto* spin = a.in.p + (size_t)a.r0 * 12 * g.V;
+    ld_comps(a.U.p + (size_t)MU * 9 * g.V, g.V, FWD ? s : t, u);
+    ld_comps(spin, g.V, t, psi);
+    if constexpr (W < 6 && MODE != MODE_DONLY) ld_own(spin, g.V, ka, kb, s, own);
+    const int r1 = LOOP ? a.r1 : a.r0 + 1;
+    for (int r = a.r0; r < r1; ++r) {
+        cx<R> o[6], mine[2];
+        hop_product<MU, PM, FWD, GP>(psi, u, w, g, o);
 #pragma unroll
-            for (int k = 0; k < 12; ++k) sh.psi[k][lane] = p[k];
+        for (int k = 0; k < 6; ++k) sh.hop[W][k][lane] = o[k];
+        if constexpr (W < 6 && MODE != MODE_DONLY) {
+            mine[0] = own[0];
+            mine[1] = own[1];
+            if constexpr (MODE == MODE_CLOVER) {
+                sh.psi[ka][lane] = mine[0];
+                sh.psi[kb][lane] = mine[1];
+            }
         }
-    }
-    cx<R> o[6];
-    hop_product<MU, PM, FWD, GP>(psi, u, w, g, o);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) sh.hop[W][k][lane] = o[k];
-    __syncthreads();
-    if constexpr (W < 6) {
-        constexpr int c = W >> 1;
-        constexpr bool kHigh = (W & 1) != 0;
-        constexpr int ka = (kHigh ? 6 : 0) + c, kb = ka + 3;
-        cx<R> ra, rb;
-        sum_hops<FPM, kHigh>(sh.hop, c, lane, ra, rb);
-        if (MODE == MODE_DONLY) {
-            const R half = R(1) / R(2);
-            ra = cadd(mk<R>(R(0), R(0)), rmul(half, ra));
-            rb = cadd(mk<R>(R(0), R(0)), rmul(half, rb));
-        } else {
-            ra = cadd(cx<R>(sh.psi[ka][lane]), rmul(-a.kappa, ra));
-            rb = cadd(cx<R>(sh.psi[kb][lane]), rmul(-a.kappa, rb));
-            if constexpr (MODE == MODE_CLOVER)
-                clover_pair<c, kHigh>(a.F, s, g.V, sh.psi, lane, a.ccoef, ra, rb);
+        if (LOOP && r + 1 < r1) {  // the next field's, in flight while this one is summed
+            spin += (size_t)12 * g.V;
+            ld_comps(spin, g.V, t, psi);
+            if constexpr (W < 6 && MODE != MODE_DONLY) ld_own(spin, g.V, ka, kb, s, own);
         }
-        if (live) {
-            a.out.st1(a.r, ka, s, ra);
-            a.out.st1(a.r, kb, s, rb);
-        }
-        if constexpr (EPI == EPI_PAP) {
-            // the terms of Re sum conj(p) Ap, summed per site in kernel_dot_D order by wavefront 7
-            const cx<R> pa = a.aux.ld1(a.r, ka, s), pb = a.aux.ld1(a.r, kb, s);
-            pap[ka][lane] = live ? cmul(cconj(pa), ra).re : 0.0;
-            pap[kb][lane] = live ? cmul(cconj(pb), rb).re : 0.0;
-        }
-    }
-    if constexpr (EPI == EPI_PAP) {
         __syncthreads();
-        if constexpr (W == 7) {
+        if constexpr (W < 6) {
+            cx<R> ra, rb;
+            sum_hops<FPM, kHigh>(sh.hop, c, lane, ra, rb);
+            if (MODE == MODE_DONLY) {
+                const R half = R(1) / R(2);
+                ra = cadd(mk<R>(R(0), R(0)), rmul(half, ra));
+                rb = cadd(mk<R>(R(0), R(0)), rmul(half, rb));
+            } else {
+                ra = cadd(mine[0], rmul(-a.kappa, ra));
+                rb = cadd(mine[1], rmul(-a.kappa, rb));
+                if constexpr (MODE == MODE_CLOVER)
+                    clover_pair<c, kHigh>(a.F, s, g.V, sh.psi, lane, a.ccoef, ra, rb);
+            }
+            if (live) {
+                a.out.st1(r, ka, s, ra);
+                a.out.st1(r, kb, s, rb);
+            }
+            if constexpr (EPI == EPI_PAP) {
+                // the terms of Re sum conj(p) Ap, summed per site in kernel_dot_D order by wavefront 7
+                const cx<R> pa = a.aux.ld1(r, ka, s), pb = a.aux.ld1(r, kb, s);
+                pap[ka][lane] = live ? cmul(cconj(pa), ra).re : 0.0;
+                pap[kb][lane] = live ? cmul(cconj(pb), rb).re : 0.0;
+            }
+        }
+        if (LOOP || EPI == EPI_PAP) __syncthreads();
+        if constexpr (EPI == EPI_PAP && W == 7) {
             double v = 0.0;
 #pragma unroll
             for (int k = 0; k < 12; ++k) v = v + pap[k][lane];
@@ -244,26 +261,35 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
     }
 }
 
-template <class In, class Lk, class Out, class Cl, int FPM, int MODE, int EPI, bool GP>
-__global__ void __launch_bounds__(512, sizeof(typename In::R) == 8 ? 4 : 6) k_hops(Out out, In in, Lk U, Cl F, In aux, Geom g, double kappa_d,
-                                                 double ccoef_d, int nrhs, int slab, EpiArgs epi) {
+// Wavefronts per SIMD to compile for: one field, all that LDS admits; several,
+// where the next field's operands stay in registers across the sum, half (FP64
+// at 4: spills, 24^3 x 48 x 4 597 us against 471).
+template <typename R>
+constexpr int hop_waves(bool loop) {
+    return sizeof(R) == 8 ? (loop ? 2 : 4) : (loop ? 4 : 6);
+}
+
+// Block lb is RHS group lb % ngroups (per fields each) of site block lb / ngroups.
+template <class In, class Lk, class Out, class Cl, int FPM, int MODE, int EPI, bool GP, bool LOOP>
+__global__ void __launch_bounds__(512, hop_waves<typename In::R>(LOOP))
+    k_hops(Out out, In in, Lk U, Cl F, In aux, Geom g, double kappa_d, double ccoef_d, int ngroups, int per, int nrhs,
+           int slab, EpiArgs epi) {
     using R = typename In::R;
     if (epi.st != nullptr && epi.st->done) return;
     if (epi.gate != nullptr && *epi.gate == 0) return;
-    __shared__ HopLds<R> sh;
+    __shared__ HopLds<R, MODE> sh;
     __shared__ double pap[EPI == EPI_PAP ? 12 : 1][kHopSites];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int lb = xcd_block(blockIdx.x, gridDim.x);
-    const int r = lb % nrhs;
-    lb /= nrhs;
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int r0 = lb % ngroups * per;
     int s0, end;
-    slab_block(lb, slab, g, s0, end);
-    const HopArgs<In, Lk, Out, Cl> a{out, in, U, F, aux, R(kappa_d), R(ccoef_d), r, epi.partials};
+    slab_block(lb / ngroups, slab, g, s0, end);
+    const HopArgs<In, Lk, Out, Cl> a{out, in, U, F, aux, R(kappa_d), R(ccoef_d), r0, min(r0 + per, nrhs), epi.partials};
     switch (wave) {
-#define LMX_HOP_WAVE(W)                                                                   \
-    case W:                                                                               \
-        hop_wave<W, FPM, MODE, EPI, GP, In, Lk, Out, Cl>(a, sh, pap, g, s0, lane, end);   \
+#define LMX_HOP_WAVE(W)                                                                       \
+    case W:                                                                                   \
+        hop_wave<W, FPM, MODE, EPI, GP, LOOP, In, Lk, Out, Cl>(a, sh, pap, g, s0, lane, end); \
         break
         LMX_HOP_WAVE(0);
         LMX_HOP_WAVE(1);
@@ -277,20 +303,31 @@ __global__ void __launch_bounds__(512, sizeof(typename In::R) == 8 ? 4 : 6) k_ho
     }
 }
 
-// Launch over nrhs fields; flags LMX_DAGGER / LMX_DONLY.  EPI_PAP (on
+// Launch over nrhs fields, up to per_hint of them in a workgroup; flags LMX_DAGGER / LMX_DONLY.  EPI_PAP (on
 // D^dagger, one field): partials gets one sum per 64 consecutive sites.
 template <class In, class Lk, class Out, class Cl, int EPI>
-int launch_hops(lmx_context* ctx, Out out, In in, Lk U, Cl F, In aux, double kappa, double ccoef, int nrhs, int flags,
-                bool clover, const EpiArgs& epi) {
+int launch_hops(lmx_context* ctx, Out out, In in, Lk U, Cl F, In aux, double kappa, double ccoef, int nrhs, int per_hint,
+                int flags, bool clover, const EpiArgs& epi) {
     const bool dag = (flags & LMX_DAGGER) != 0, donly = (flags & LMX_DONLY) != 0;
     const Geom& g = ctx->g;
     const SlabOrder so = slab_order(g, EPI == EPI_PAP);  // the sums of EPI_PAP need whole blocks
-    const int slab = so.slab;
-    const long nb = so.blocks * nrhs;
+    // clover fields one by one: a loop over them would hold the planes' entries too
+    const int per = clover || EPI != EPI_NONE ? 1 : std::min(std::max(per_hint, 1), nrhs);
+    const int ngroups = (nrhs + per - 1) / per;
+    const long nb = so.blocks * ngroups;
     LMX_CHECK(nb < (1L << 31), LMX_ERR_ARG, "too many right-hand sides (%d)", nrhs);
-#define LMX_HOPS(FPM, MODE, GP)                                                                                    \
-    hipLaunchKernelGGL((k_hops<In, Lk, Out, Cl, FPM, MODE, EPI, GP>), dim3((unsigned)nb), dim3(512), 0, ctx->stream, \
-                       out, in, U, F, aux, g, kappa, ccoef, nrhs, slab, epi)
+#define LMX_HOPS(FPM, MODE, GP)                                                                                     \
+    do {                                                                                                            \
+        if constexpr (EPI == EPI_NONE && MODE != MODE_CLOVER) {                                                     \
+            if (per > 1) {                                                                                          \
+                hipLaunchKernelGGL((k_hops<In, Lk, Out, Cl, FPM, MODE, EPI, GP, true>), dim3((unsigned)nb), dim3(512), 0, \
+                                   ctx->stream, out, in, U, F, aux, g, kappa, ccoef, ngroups, per, nrhs, so.slab, epi); \
+                break;                                                                                              \
+            }                                                                                                       \
+        }                                                                                                           \
+        hipLaunchKernelGGL((k_hops<In, Lk, Out, Cl, FPM, MODE, EPI, GP, false>), dim3((unsigned)nb), dim3(512), 0,  \
+                           ctx->stream, out, in, U, F, aux, g, kappa, ccoef, ngroups, per, nrhs, so.slab, epi);     \
+    } while (0)
 #define LMX_HOPS_GP(FPM, MODE)            \
     do {                                  \
         if (g.general)                    \
