@@ -684,25 +684,28 @@ __device__ __forceinline__ void pin_acc(cx<R> (&a)[12]) {
 //   _wilson_reconstruct_add3  src/Operators/WilsonDiracOperator.jl:231-263
 // psi is indexed [spin*3 + colour]; h[2*colour + {0,1}]; acc[colour*4 + spin].
 // ---------------------------------------------------------------------------
+// one colour's half-spinor from its four spins
+template <int PM, int MU, typename R>
+__device__ __forceinline__ void half_project1(cx<R> p1, cx<R> p2, cx<R> p3, cx<R> p4, cx<R>& h1, cx<R>& h2) {
+    if (MU == 0) {
+        h1 = csub(p1, pmi<PM>(p4));
+        h2 = csub(p2, pmi<PM>(p3));
+    } else if (MU == 1) {
+        h1 = csub(p1, pmr<PM>(p4));
+        h2 = cadd(p2, pmr<PM>(p3));
+    } else if (MU == 2) {
+        h1 = csub(p1, pmi<PM>(p3));
+        h2 = cadd(p2, pmi<PM>(p4));
+    } else {
+        h1 = csub(p1, pmr<PM>(p3));
+        h2 = csub(p2, pmr<PM>(p4));
+    }
+}
 template <int PM, int MU, typename R>
 __device__ __forceinline__ void half_project(const cx<R> psi[12], cx<R> h[6]) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        cx<R> p1 = psi[c], p2 = psi[3 + c], p3 = psi[6 + c], p4 = psi[9 + c];
-        if (MU == 0) {
-            h[2 * c] = csub(p1, pmi<PM>(p4));
-            h[2 * c + 1] = csub(p2, pmi<PM>(p3));
-        } else if (MU == 1) {
-            h[2 * c] = csub(p1, pmr<PM>(p4));
-            h[2 * c + 1] = cadd(p2, pmr<PM>(p3));
-        } else if (MU == 2) {
-            h[2 * c] = csub(p1, pmi<PM>(p3));
-            h[2 * c + 1] = cadd(p2, pmi<PM>(p4));
-        } else {
-            h[2 * c] = csub(p1, pmr<PM>(p3));
-            h[2 * c + 1] = csub(p2, pmr<PM>(p4));
-        }
-    }
+    for (int c = 0; c < 3; ++c)
+        half_project1<PM, MU>(psi[c], psi[3 + c], psi[6 + c], psi[9 + c], h[2 * c], h[2 * c + 1]);
 }
 
 template <int PM, int MU, typename R>

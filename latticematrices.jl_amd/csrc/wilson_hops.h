@@ -123,8 +123,8 @@ __device__ __forceinline__ void sum_hops(const LdsCx<R> (&hop)[8][6][kHopSites],
 
 // The clover term of colour C's spins (0, 1) or (2, 3): that pair's share of
 // clover_add, in its order, from the site's own spinor in LDS.
-template <int C, bool HIGH, typename R, class Acc>
-__device__ __forceinline__ void clover_pair(const Acc& F, int s, int V, const LdsCx<R> (&psi)[12][kHopSites], int lane,
+template <int C, bool HIGH, int P, typename R, class Acc>
+__device__ __forceinline__ void clover_pair(const Acc& F, int s, int V, const LdsCx<R> (&psi)[12][P], int lane,
                                             R coefficient, cx<R>& ra, cx<R>& rb) {
     cx<R> v1 = mk<R>(R(0), R(0)), v2 = v1;
     R d[6];
@@ -237,7 +237,7 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
                 ra = cadd(mine[0], rmul(-a.kappa, ra));
                 rb = cadd(mine[1], rmul(-a.kappa, rb));
                 if constexpr (MODE == MODE_CLOVER)
-                    clover_pair<c, kHigh>(a.F, s, g.V, sh.psi, lane, a.ccoef, ra, rb);
+                    clover_pair<c, kHigh, kHopSites>(a.F, s, g.V, sh.psi, lane, a.ccoef, ra, rb);
             }
             if (live) {
                 a.out.st1(r, ka, s, ra);
@@ -358,6 +358,245 @@ int launch_hops(lmx_context* ctx, Out out, In in, Lk U, Cl F, In aux, double kap
 #undef LMX_HOPS_MODE
 #undef LMX_HOPS_GP
 #undef LMX_HOPS
+    LMX_HIP(hipGetLastError());
+    return LMX_OK;
+}
+
+// ---------------------------------------------------------------------------
+// The same stencil on the reference's own storage (LatticeMatrix.A: component
+// spin*3 + colour of padded site p at p*12 + k; halo not read, only core sites
+// written).  A wavefront loads its 64 neighbours' spinors as they lie, 16 (8)
+// consecutive bytes per lane across a row of sites, and turns them to one site
+// per lane in its own 6 (3) KB of LDS, 32 sites at a time, projecting colour by
+// colour as it reads; the results leave the same way.  One site per lane
+// straight from memory touches a line per lane and load, twelve times over, and
+// takes the hops in turn: 24^3 x 48 276 us against 168 here, in ComplexF32
+// 126 against 89, 32^4 392 against 288.  Bound by L2 misses, as above.
+// ---------------------------------------------------------------------------
+struct PadGeom {
+    int PS[4];  // padded strides (1, P1, P1 P2, P1 P2 P3)
+    int nw;
+    long Vp;    // padded volume
+};
+constexpr int kPadPitch = kHopSites + 1;  // a site's twelve components lie in different banks
+
+template <typename R>
+struct PadLds {
+    LdsCx<R> hop[8][6][kHopSites];
+    LdsCx<R> psi[12][kPadPitch];  // the site's own spinor, then the results
+    int site[kHopSites];          // padded index of the workgroup's sites
+};
+
+// N consecutive components of a site as one word (16 bytes; 8 for a FP32 array
+// that is not 16-byte aligned)
+template <typename E, int N>
+struct alignas(N * sizeof(E)) PadWord {
+    E e[N];
+};
+
+template <typename E, class Lk, class Cl>
+struct PadArgs {
+    E* out;
+    const E* in;
+    Lk U;
+    Cl F;
+    double kappa, ccoef;
+};
+
+template <int W, int FPM, int MODE, bool GP, int N, typename R, typename E, class Lk, class Cl>
+__device__ __forceinline__ void pad_wave(const PadArgs<E, Lk, Cl>& a, PadLds<R>& sh, const Geom& g, const PadGeom& pg,
+                                         int s0, int lane, int end) {
+    constexpr int MU = W >> 1;
+    constexpr bool FWD = (W & 1) == 0;
+    constexpr int PM = FWD ? FPM : -FPM;
+    constexpr int c = W >> 1;
+    constexpr bool kHigh = (W & 1) != 0;
+    constexpr int ka = (kHigh ? 6 : 0) + c, kb = ka + 3;
+    int s = s0 + lane;
+    if (s >= end) s = end - 1;
+    int x[4];
+    site_coords(s, g, x);
+    bool w;
+    const int t = FWD ? nbr_fwd(s, x, MU, g, w) : nbr_bwd(s, x, MU, g, w);
+    const int sp = (x[0] + pg.nw) + pg.PS[1] * (x[1] + pg.nw) + pg.PS[2] * (x[2] + pg.nw) + pg.PS[3] * (x[3] + pg.nw);
+    const int step = FWD ? (w ? -(g.L[MU] - 1) : 1) : (w ? g.L[MU] - 1 : -1);
+    const int tp = sp + step * pg.PS[MU];
+    // word 64 j + lane of the 64 spinors end to end, M words a site
+    using Word = PadWord<E, N>;
+    constexpr int M = 12 / N;
+    Word land[M];
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        const int e = 64 * j + lane, i = e / M;
+        land[j] = reinterpret_cast<const Word*>(a.in)[(long)__shfl(tp, i, 64) * M + (e - M * i)];
+    }
+    cx<R> u[9];
+    ld_comps(a.U.p + (size_t)MU * 9 * g.V, g.V, FWD ? s : t, u);
+    if constexpr (W == 0) sh.site[lane] = sp;
+    LdsCx<R>* mine = &sh.hop[W][0][0];
+    cx<R> h[6];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int j = 0; j < M / 2; ++j)
+#pragma unroll
+            for (int n = 0; n < N; ++n) {
+                const E v = land[M / 2 * half + j].e[n];
+                mine[N * (64 * j + lane) + n] = mk<R>(v.x, v.y);
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if ((lane >> 5) == half) {
+            const LdsCx<R>* q = mine + 12 * (lane & 31);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                cx<R> p[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    p[d] = q[3 * d + k];
+                    if (GP && w && !g.phase_one[MU])
+                        p[d] = cmul(p[d], FWD ? mk<R>(R(g.ph_re[MU]), R(g.ph_im[MU]))
+                                              : mk<R>(R(g.iph_re[MU]), R(g.iph_im[MU])));
+                }
+                half_project1<PM, MU>(p[0], p[1], p[2], p[3], h[2 * k], h[2 * k + 1]);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (!GP) neg_select(h, w && g.phase_neg[MU]);
+    cx<R> o[6];
+    if (FWD)
+        matvec_fwd(u, h, o);
+    else
+        matvec_bwd(u, h, o);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sh.hop[W][k][lane] = o[k];
+    __syncthreads();
+    cx<R> ra, rb;
+    if constexpr (W < 6) {
+        const R kappa = R(a.kappa);
+        sum_hops<FPM, kHigh>(sh.hop, c, lane, ra, rb);
+        if (MODE == MODE_DONLY) {
+            const R half = R(1) / R(2);
+            ra = cadd(mk<R>(R(0), R(0)), rmul(half, ra));
+            rb = cadd(mk<R>(R(0), R(0)), rmul(half, rb));
+        } else {
+            ra = cadd(cx<R>(sh.psi[ka][lane]), rmul(-kappa, ra));
+            rb = cadd(cx<R>(sh.psi[kb][lane]), rmul(-kappa, rb));
+            if constexpr (MODE == MODE_CLOVER)
+                clover_pair<c, kHigh, kPadPitch>(a.F, s, g.V, sh.psi, lane, R(a.ccoef), ra, rb);
+        }
+    }
+    __syncthreads();  // the own spinors have been read: results take their place
+    if constexpr (W < 6) {
+        sh.psi[ka][lane] = ra;
+        sh.psi[kb][lane] = rb;
+    }
+}
+
+template <int FPM, int MODE, bool GP, int N, typename E, class Lk, class Cl>
+__global__ void __launch_bounds__(512, sizeof(E) == 16 ? 4 : 6)
+    k_hops_pad(E* __restrict__ C, const E* __restrict__ psi, Lk U, Cl F, Geom g, PadGeom pg, double kappa,
+               double ccoef, int nrhs, int slab) {
+    using R = typename std::conditional<std::is_same<E, float2>::value, float, double>::type;
+    __shared__ PadLds<R> sh;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const long field = (long)(lb % nrhs) * pg.Vp * 12;
+    int s0, end;
+    slab_block(lb / nrhs, slab, g, s0, end);
+    const PadArgs<E, Lk, Cl> a{C + field, psi + field, U, F, kappa, ccoef};
+    const int n = min(kHopSites, end - s0);
+    using Word = PadWord<E, N>;
+    constexpr int M = 12 / N;
+    if (MODE != MODE_DONLY) {  // the sites' own spinors, word after word
+        for (int e = threadIdx.x; e < M * n; e += 512) {
+            const int i = e / M, k = N * (e - M * i);
+            int x[4];
+            site_coords(s0 + i, g, x);
+            const long sp = (x[0] + pg.nw) + (long)pg.PS[1] * (x[1] + pg.nw) + (long)pg.PS[2] * (x[2] + pg.nw) +
+                            (long)pg.PS[3] * (x[3] + pg.nw);
+            const Word v = reinterpret_cast<const Word*>(a.in)[sp * M + k / N];
+#pragma unroll
+            for (int c = 0; c < N; ++c) sh.psi[k + c][i] = mk<R>(v.e[c].x, v.e[c].y);
+        }
+    }
+    switch (wave) {
+#define LMX_PAD_WAVE(W)                                                                    \
+    case W:                                                                                \
+        pad_wave<W, FPM, MODE, GP, N, R, E, Lk, Cl>(a, sh, g, pg, s0, lane, end);          \
+        break
+        LMX_PAD_WAVE(0);
+        LMX_PAD_WAVE(1);
+        LMX_PAD_WAVE(2);
+        LMX_PAD_WAVE(3);
+        LMX_PAD_WAVE(4);
+        LMX_PAD_WAVE(5);
+        LMX_PAD_WAVE(6);
+        LMX_PAD_WAVE(7);
+#undef LMX_PAD_WAVE
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < M * n; e += 512) {
+        const int i = e / M, k = N * (e - M * i);
+        Word v;
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            const cx<R> z = sh.psi[k + c][i];
+            v.e[c].x = z.re;
+            v.e[c].y = z.im;
+        }
+        reinterpret_cast<Word*>(a.out)[(long)sh.site[i] * M + k / N] = v;
+    }
+}
+
+template <int N, typename E, class Lk, class Cl>
+int launch_hops_pad(lmx_context* ctx, Lk l, Cl F, bool clover, double kappa, double csw, E* C, const E* psi, int nw,
+                    int nrhs, int flags) {
+    if (ctx->V == 0 || nrhs == 0) return LMX_OK;
+    const Geom& g = ctx->g;
+    PadGeom pg;
+    pg.nw = nw;
+    long st = 1;
+    for (int d = 0; d < 4; ++d) {
+        pg.PS[d] = (int)st;
+        st *= g.L[d] + 2 * nw;
+    }
+    pg.Vp = st;
+    LMX_CHECK(st < (1L << 31), LMX_ERR_ARG, "padded volume too large");
+    const double ccoef = (-kappa) * csw;
+    const SlabOrder so = slab_order(g, false);
+    const long nb = so.blocks * nrhs;
+    LMX_CHECK(nb < (1L << 31), LMX_ERR_ARG, "too many right-hand sides (%d)", nrhs);
+    const bool dag = (flags & LMX_DAGGER) != 0, donly = (flags & LMX_DONLY) != 0;
+#define LMX_PAD(FPM, MODE)                                                                                       \
+    do {                                                                                                         \
+        if (g.general)                                                                                           \
+            hipLaunchKernelGGL((k_hops_pad<FPM, MODE, true, N, E, Lk, Cl>), dim3((unsigned)nb), dim3(512), 0,       \
+                               ctx->stream, C, psi, l, F, g, pg, kappa, ccoef, nrhs, so.slab);                   \
+        else                                                                                                     \
+            hipLaunchKernelGGL((k_hops_pad<FPM, MODE, false, N, E, Lk, Cl>), dim3((unsigned)nb), dim3(512), 0,      \
+                               ctx->stream, C, psi, l, F, g, pg, kappa, ccoef, nrhs, so.slab);                   \
+    } while (0)
+    if (donly) {
+        if (dag)
+            LMX_PAD(1, MODE_DONLY);
+        else
+            LMX_PAD(-1, MODE_DONLY);
+    } else if (clover) {
+        if (dag)
+            LMX_PAD(1, MODE_CLOVER);
+        else
+            LMX_PAD(-1, MODE_CLOVER);
+    } else {
+        if (dag)
+            LMX_PAD(1, MODE_WILSON);
+        else
+            LMX_PAD(-1, MODE_WILSON);
+    }
+#undef LMX_PAD
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }

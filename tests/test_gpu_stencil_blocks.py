@@ -5,6 +5,7 @@ that do not, slices that end inside a block, complex phases; and the p.Ap sums
 that it leaves per 64 sites through whole CG solves."""
 import numpy as np
 import pytest
+import torch
 
 import oracle as orc
 import lmx
@@ -126,3 +127,42 @@ def test_cg_first_iteration_converges(gpu, L):
     res = lmx.cg_(x, lmx.DdagDOp(D, tmp), b, r, p, Ap, rtol=1e-10)
     assert res.converged and res.iterations == 1 and res.residual_norm == 0.0
     assert np.array_equal(x.to_numpy(), b.to_numpy())
+
+
+def _padded(L, nw, nrhs, rng):
+    P = [d + 2 * nw for d in L]
+    shape = (nrhs, P[3], P[2], P[1], P[0], 4, 3)
+    a = rng.standard_normal(shape) + 1j * rng.standard_normal(shape)  # the halo: garbage
+    core = (slice(None),) + tuple(slice(nw, nw + d) for d in reversed(L)) + (slice(None), slice(None))
+    return a, core
+
+
+@pytest.mark.parametrize("L,nw,phases", [((2, 2, 2, 2), 1, ANTI), ((3, 5, 3, 3), 0, ANTI), ((3, 5, 3, 3), 2, (-1, 1j, 1, -1)),
+                                         ((8, 8, 9, 4), 1, ANTI), ((13, 13, 13, 2), 1, ANTI)])
+@pytest.mark.parametrize("csw", [0.0, 1.0])
+@pytest.mark.parametrize("dt", [torch.complex128, torch.complex64])
+@pytest.mark.parametrize("offset", [0, 1])  # in elements: at 1 a complex64 array is not 16-byte aligned
+def test_reference_storage(gpu, L, nw, phases, csw, dt, offset):
+    print(f"padded blocks L={L} nw={nw} csw={csw} {dt} offset={offset}", flush=True)
+    U = gen.links(L, "haar", 49)
+    a, core = _padded(L, nw, 2, np.random.default_rng(50))
+    lat = lmx.Lattice(L, phases)
+    D = lmx.WilsonDiracOperator4D(lat.gauge_from_numpy(U), 0.117, csw)
+    store = torch.empty(a.size + offset, dtype=dt, device="cuda")
+    psi = store[offset:].view(a.shape).copy_(torch.from_numpy(a))
+    C = torch.full((a.size + offset,), 3.0, dtype=dt, device="cuda")[offset:].view(a.shape)
+    lmx.mul_padded_(C, lmx.adjoint(D), psi, nw=nw)
+    got = C.cpu().numpy()
+    outside = np.ones(a.shape, dtype=bool)
+    outside[core] = False
+    assert np.all(got[outside] == 3.0)  # only core sites are written
+    F = orc.clover_field_strength(U, L) if csw else None
+    for r in range(2):
+        p = np.ascontiguousarray(a[core][r]).reshape(-1, 4, 3)
+        ref = (orc.wilson_clover(U, F, p, L, 0.117, csw, phases, dagger=True) if csw
+               else orc.wilson(U, p, L, 0.117, phases, dagger=True))
+        mine = got[core][r].reshape(-1, 4, 3)
+        if dt == torch.complex128:
+            assert np.array_equal(mine, ref)
+        else:  # a few dozen roundings of 6e-8 on values of order one
+            assert np.max(np.abs(mine - ref)) <= 64 * 6e-8 * np.max(np.abs(ref))
