@@ -525,10 +525,28 @@ int lmx_cg_ddagd_internal(lmx_wilson* op, double2* x, const double2* b, double2*
 static int default_rhs_block(lmx_wilson* op, int prec, int nrhs) {
     const int t = (prec >= 0 && prec < 4 && nrhs >= 0 && nrhs <= 64) ? op->tuned_block[prec][nrhs] : 0;
     if (t > 0) return t;
-    // all RHS in one launch, two per work item when that divides evenly
+    // all RHS in one launch.  D + D^dagger of one inner iteration, us, by shape:
+    const lmx_context* c = op->ctx;
     const int per = std::min(nrhs, 12);
-    const int nr = (per % 2 == 0) ? 2 : 1;
-    return (per << 4) | nr;
+    const long n = (long)c->V * per;
+    const bool clover = op->csw != 0.0;
+    if (lds_ok(c)) {
+        // LDS-staged, four t-slices per workgroup where that leaves two
+        // workgroups per CU (24^3 x 48 x 4: f16 615 against 793 streaming two per
+        // work item, h16 clover 497 / 944; 32^4 x 12: h16 1499 / 1824, f32
+        // 3048 / 3584), else as few as fill the chip (16^3 x 32 x 2 f32 78 / 116);
+        // one z-range, so that no z-halo crosses XCDs
+        const bool four = c->g.L[3] % 4 == 0 && n / 1024 >= 512;
+        // too little work to repay the staging in 16 bits: 16^3 x 32 x 1 33 / 35
+        if (!four && prec == LMX_H16) return (1 << 20) | (per << 4) | 1;
+        return kLdsStage | (1 << 20) | ((four ? 4 : 0) << 12) | (per << 4) | 1;
+    }
+    // no streaming there: two per work item share the links where there is
+    // work enough (27x29x31x35 x 4 f32 1210 against 1335 one by one, but
+    // 9x10x11x12 x 4 47 / 32); in 16 bits the second one's registers cost more
+    // (18x20x22x30 x 4 160 / 145, clover 223 / 184)
+    const bool two = per % 2 == 0 && (prec == LMX_H16 ? !clover && n > 3000000 : n > 1000000);
+    return (per << 4) | (two ? 2 : 1);
 }
 
 int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void* work, size_t bytes,
