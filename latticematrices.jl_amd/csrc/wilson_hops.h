@@ -7,7 +7,9 @@
 // link, forms its half-spinor U P psi and leaves it in LDS; after one barrier
 // wavefronts 0-5 each sum two of the site's twelve components over the eight
 // hops, in the reference's order, and write them (results bit-identical to
-// k_site's and k_stream's).  Several right-hand sides take their turns in the
+// k_site's and k_stream's).  The clover planes' words are loaded once by all
+// eight, an eighth each, and wait in LDS (read by each wavefront that needs
+// them instead: 48^3 x 96 3850 us against 3500).  Several right-hand sides take their turns in the
 // workgroup with the links kept in registers, the next one's spinors in
 // flight while the last one's components are summed.
 //
@@ -90,9 +92,33 @@ struct alignas(2 * sizeof(R)) LdsCx {
         return mk<R>(v.x, v.y);
     }
 };
+// U P psi of each hop: [hop][2 colour + half-spin][site]; the clover planes
+// take their place once they are summed.
+template <typename R>
+union HopBuf {
+    LdsCx<R> hop[8][6][kHopSites];
+    LdsCx<R> F[27][kHopSites];
+    __device__ HopBuf() {}
+};
+// Wavefront W's share of the 27 clover words of the workgroup's sites: into
+// registers before the hops are summed, into LDS after.
+template <int W>
+struct CloverShare {
+    static constexpr int kFirst = W < 3 ? 4 * W : 3 * W + 3, kNum = W < 3 ? 4 : 3;
+};
+template <int W, typename R, class Cl>
+__device__ __forceinline__ void ld_clover_share(const Cl& F, int V, int s, cx<R> (&f)[CloverShare<W>::kNum]) {
+    ld_comps(F.p + (size_t)CloverShare<W>::kFirst * V, V, s, f);
+}
+template <int W, typename R>
+__device__ __forceinline__ void put_clover_share(LdsCx<R> (&F)[27][kHopSites], int lane,
+                                                 const cx<R> (&f)[CloverShare<W>::kNum]) {
+#pragma unroll
+    for (int k = 0; k < CloverShare<W>::kNum; ++k) F[CloverShare<W>::kFirst + k][lane] = f[k];
+}
 template <typename R, int MODE>
 struct HopLds {
-    LdsCx<R> hop[8][6][kHopSites];                            // U P psi of each hop: [hop][2 colour + half-spin][site]
+    HopBuf<R> b;
     LdsCx<R> psi[MODE == MODE_CLOVER ? 12 : 1][kHopSites];  // the site's own spinor, for the clover term
 };
 // two components of the site's own spinor
@@ -123,8 +149,8 @@ __device__ __forceinline__ void sum_hops(const LdsCx<R> (&hop)[8][6][kHopSites],
 
 // The clover term of colour C's spins (0, 1) or (2, 3): that pair's share of
 // clover_add, in its order, from the site's own spinor in LDS.
-template <int C, bool HIGH, int P, typename R, class Acc>
-__device__ __forceinline__ void clover_pair(const Acc& F, int s, int V, const LdsCx<R> (&psi)[12][P], int lane,
+template <int C, bool HIGH, int P, typename R>
+__device__ __forceinline__ void clover_pair(const LdsCx<R> (&F)[27][kHopSites], const LdsCx<R> (&psi)[12][P], int lane,
                                             R coefficient, cx<R>& ra, cx<R>& rb) {
     cx<R> v1 = mk<R>(R(0), R(0)), v2 = v1;
     R d[6];
@@ -132,12 +158,12 @@ __device__ __forceinline__ void clover_pair(const Acc& F, int s, int V, const Ld
 #pragma unroll
     for (int pl = 0; pl < 6; ++pl) {
         const int q = 3 * pl + C;
-        const cx<R> v = F.ld((long)(q / 2) * V + s);
+        const cx<R> v = F[q / 2][lane];
         d[pl] = (q & 1) ? v.im : v.re;
         // the row's two off-diagonal entries, by their column: 0 and 1 of the other two
         constexpr int j0 = C == 0 ? 0 : (C == 1 ? 0 : 1), j1 = C == 0 ? 1 : 2;
-        u[pl][0] = F.ld((long)(9 + 3 * pl + j0) * V + s);
-        u[pl][1] = F.ld((long)(9 + 3 * pl + j1) * V + s);
+        u[pl][0] = F[9 + 3 * pl + j0][lane];
+        u[pl][1] = F[9 + 3 * pl + j1][lane];
     }
 #pragma unroll
     for (int ic = 0; ic < 3; ++ic) {
@@ -211,7 +237,7 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
         cx<R> o[6], mine[2];
         hop_product<MU, PM, FWD, GP>(psi, u, w, g, o);
 #pragma unroll
-        for (int k = 0; k < 6; ++k) sh.hop[W][k][lane] = o[k];
+        for (int k = 0; k < 6; ++k) sh.b.hop[W][k][lane] = o[k];
         if constexpr (W < 6 && MODE != MODE_DONLY) {
             mine[0] = own[0];
             mine[1] = own[1];
@@ -225,10 +251,17 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
             ld_comps(spin, g.V, t, psi);
             if constexpr (W < 6 && MODE != MODE_DONLY) ld_own(spin, g.V, ka, kb, s, own);
         }
+        cx<R> f[MODE == MODE_CLOVER ? CloverShare<W>::kNum : 1];
+        if constexpr (MODE == MODE_CLOVER) ld_clover_share<W>(a.F, g.V, s, f);
         __syncthreads();
+        cx<R> ra, rb;
+        if constexpr (W < 6) sum_hops<FPM, kHigh>(sh.b.hop, c, lane, ra, rb);
+        if constexpr (MODE == MODE_CLOVER) {
+            __syncthreads();
+            put_clover_share<W>(sh.b.F, lane, f);
+            __syncthreads();
+        }
         if constexpr (W < 6) {
-            cx<R> ra, rb;
-            sum_hops<FPM, kHigh>(sh.hop, c, lane, ra, rb);
             if (MODE == MODE_DONLY) {
                 const R half = R(1) / R(2);
                 ra = cadd(mk<R>(R(0), R(0)), rmul(half, ra));
@@ -237,7 +270,7 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
                 ra = cadd(mine[0], rmul(-a.kappa, ra));
                 rb = cadd(mine[1], rmul(-a.kappa, rb));
                 if constexpr (MODE == MODE_CLOVER)
-                    clover_pair<c, kHigh, kHopSites>(a.F, s, g.V, sh.psi, lane, a.ccoef, ra, rb);
+                    clover_pair<c, kHigh>(sh.b.F, sh.psi, lane, a.ccoef, ra, rb);
             }
             if (live) {
                 a.out.st1(r, ka, s, ra);
@@ -382,7 +415,7 @@ constexpr int kPadPitch = kHopSites + 1;  // a site's twelve components lie in d
 
 template <typename R>
 struct PadLds {
-    LdsCx<R> hop[8][6][kHopSites];
+    HopBuf<R> b;
     LdsCx<R> psi[12][kPadPitch];  // the site's own spinor, then the results
     int site[kHopSites];          // padded index of the workgroup's sites
 };
@@ -433,7 +466,7 @@ __device__ __forceinline__ void pad_wave(const PadArgs<E, Lk, Cl>& a, PadLds<R>&
     cx<R> u[9];
     ld_comps(a.U.p + (size_t)MU * 9 * g.V, g.V, FWD ? s : t, u);
     if constexpr (W == 0) sh.site[lane] = sp;
-    LdsCx<R>* mine = &sh.hop[W][0][0];
+    LdsCx<R>* mine = &sh.b.hop[W][0][0];
     cx<R> h[6];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -471,12 +504,19 @@ __device__ __forceinline__ void pad_wave(const PadArgs<E, Lk, Cl>& a, PadLds<R>&
     else
         matvec_bwd(u, h, o);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) sh.hop[W][k][lane] = o[k];
+    for (int k = 0; k < 6; ++k) sh.b.hop[W][k][lane] = o[k];
+    cx<R> f[MODE == MODE_CLOVER ? CloverShare<W>::kNum : 1];
+    if constexpr (MODE == MODE_CLOVER) ld_clover_share<W>(a.F, g.V, s, f);
     __syncthreads();
     cx<R> ra, rb;
+    if constexpr (W < 6) sum_hops<FPM, kHigh>(sh.b.hop, c, lane, ra, rb);
+    if constexpr (MODE == MODE_CLOVER) {
+        __syncthreads();
+        put_clover_share<W>(sh.b.F, lane, f);
+        __syncthreads();
+    }
     if constexpr (W < 6) {
         const R kappa = R(a.kappa);
-        sum_hops<FPM, kHigh>(sh.hop, c, lane, ra, rb);
         if (MODE == MODE_DONLY) {
             const R half = R(1) / R(2);
             ra = cadd(mk<R>(R(0), R(0)), rmul(half, ra));
@@ -485,7 +525,7 @@ __device__ __forceinline__ void pad_wave(const PadArgs<E, Lk, Cl>& a, PadLds<R>&
             ra = cadd(cx<R>(sh.psi[ka][lane]), rmul(-kappa, ra));
             rb = cadd(cx<R>(sh.psi[kb][lane]), rmul(-kappa, rb));
             if constexpr (MODE == MODE_CLOVER)
-                clover_pair<c, kHigh, kPadPitch>(a.F, s, g.V, sh.psi, lane, R(a.ccoef), ra, rb);
+                clover_pair<c, kHigh>(sh.b.F, sh.psi, lane, R(a.ccoef), ra, rb);
         }
     }
     __syncthreads();  // the own spinors have been read: results take their place

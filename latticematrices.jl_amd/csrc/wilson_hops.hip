@@ -29,32 +29,35 @@ static int rhs_per_block(const lmx_context* ctx, int nrhs) {
 
 // Measured, us, this kernel / the other.
 bool hops_f64(const lmx_context* ctx, int nrhs, bool clover) {
-    // several clover fields: the planes are read for each (16^4 x 4 59 / 50,
-    // 24^3 x 48 x 4 690 / 699, but 8^3 x 16 x 4 9 / 12)
-    if (clover && nrhs > 1) return ctx->V * nrhs <= 100000;
     const StreamUse st = stream_use(ctx, clover ? nrhs : (nrhs + 1) / 2, 256);
-    if (st.tl == 0 || ctx->g.general) return true;  // k_site: 18x20x22x30 42 / 80, four fields 173 / 252
+    // against k_site: 18x20x22x30 42 / 80, four fields 173 / 252; clover 65 / 93, 227 / 242
+    if (st.tl == 0 || ctx->g.general) return true;
     if (shape_forced(ctx)) return false;
-    // Clover: 16^3 x 32 36 / 39, 24^3 x 48 213 / 268 (k_stream fills 63%), but
-    // 32^4 365 / 321, 40^3 x 80 1740 / 1693, 48^3 x 96 3850 / 3867.
-    if (clover) return st.tl < 4 || st.fill < 0.8;
-    // One field: 16^3 x 32 26 / 31, 24^3 x 48 146 / 198, 40^3 x 80 1185 / 1310,
-    // 48^3 x 96 2610 / 2920; k_stream wins where its workgroups fill the 256
-    // CUs exactly once and walk far (32^3 x 16 122 / 115, 32^4 253 / 230).
-    // Several, two of them to its work item: 16^3 x 32 x 4 80 / 93, 24^3 x 48 x 4
-    // 471 / 598, but 32^4 x 4 798 / 684, 40^3 x 80 x 2 2270 / 1940.
+    // k_stream wins where its workgroups fill the 256 CUs an exact number of
+    // times and walk far.  Clover, one field per work item: 32^4 335 / 324, x 4
+    // 1055 / 981, 16^4 x 4 53 / 50, but 16^3 x 32 35 / 39, 24^3 x 48 192 / 270,
+    // 40^3 x 80 1560 / 1697, 48^3 x 96 3501 / 3866.
+    if (clover) return st.fill < 0.99 || st.tl < (nrhs >= 4 ? 4 : 8);
+    // One field: 32^3 x 16 122 / 115, 32^4 253 / 230, but 16^3 x 32 26 / 31,
+    // 24^3 x 48 146 / 198, 40^3 x 80 1185 / 1310, 48^3 x 96 2610 / 2920.
+    // Several, two of them to its work item: 32^4 x 4 798 / 684, 40^3 x 80 x 2
+    // 2270 / 1940, but 16^3 x 32 x 4 80 / 93, 24^3 x 48 x 4 471 / 598.
     return st.tl < 8 || st.fill < 0.8 || (nrhs == 1 && st.wgs > 256);
 }
 
 bool hops_f32(const lmx_context* ctx, int nrhs, bool clover) {
-    // clover, the planes read twice and more: 8^3 x 16 6 / 11, but 24^3 x 48 146 / 129
-    if (clover) return ctx->V * nrhs <= 50000;
-    // several fields share the links (24^3 x 48 x 4 266 / 341, 32^4 x 12 1246 / 1546);
-    // one: 24^3 x 48 63 / 79, 40^3 x 80 682 / 718, and as above 32^4 151 / 145
     const Geom& g = ctx->g;
-    if (nrhs > 1 || g.general || !(g.phase_one[0] && g.phase_one[1] && g.phase_one[2])) return true;
-    const StreamUse st = stream_use(ctx, 1, 512);
-    return st.tl < 8 || st.fill < 0.8 || st.wgs > 512;
+    const bool streams = !g.general && g.phase_one[0] && g.phase_one[1] && g.phase_one[2];
+    const StreamUse st = streams ? stream_use(ctx, nrhs, 512) : StreamUse{0, 0, 0.0};
+    // one field: 32^4 151 / 145, clover 200 / 189, but 24^3 x 48 63 / 79, clover
+    // 113 / 129, 40^3 x 80 682 / 718, clover 908 / 920
+    if (nrhs == 1) return st.tl < 8 || st.fill < 0.8 || st.wgs > 512;
+    // several share the links: 24^3 x 48 x 4 266 / 341, 32^4 x 12 1246 / 1546
+    if (!clover) return true;
+    // clover fields do not: 16^4 x 4 32 / 34, 24^3 x 48 x 4 371 / 417, 27x29x31x35
+    // x 12 1460 / 1546, but 16^3 x 32 x 12 195 / 176, 20^3 x 40 x 4 171 / 165,
+    // 32^4 x 4 612 / 589
+    return ctx->V * nrhs <= 550000 || (ctx->V >= 500000 && st.fill < 0.99);
 }
 
 int launch_hops_f64(lmx_context* ctx, double2* out, const double2* in, const double2* U, const double2* clover,
