@@ -100,6 +100,42 @@ def test_spinor_fill_matches_padded_fill_and_oracle(gpu):
     assert np.array_equal(u.to_numpy(), o.reshape(-1, 4, 3))
 
 
+@pytest.mark.parametrize("dims,n,alg", [((4, 4, 4, 4), 1, "philox4x32"), ((5, 3, 7, 5), 17, "philox4x32"),
+                                        ((4, 6, 5, 9), 16, "xoshiro256++"), ((3, 3, 3, 3), 33, "pcg32")])
+def test_fields_of_a_batch_are_the_single_fields(gpu, dims, n, alg):
+    # several right-hand sides share a launch, sixteen at a time
+    lat = lmx.Lattice(dims)
+    keys = [lmx.RNGStreamKey(7 + r, r, 1) for r in range(n)]
+    psi, one = lat.spinor(n), lat.spinor(1)
+    for f, kw in ((lmx.randomize_matrix_, {}), (lmx.randomize_gaussian_matrix_, dict(sigma=0.75))):
+        f(psi, keys, rng_algorithm=alg, **kw)
+        got = psi.to_numpy().reshape(n, -1)
+        for r in range(n):
+            f(one, keys[r], rng_algorithm=alg, **kw)
+            assert np.array_equal(got[r], one.to_numpy().reshape(-1)), (r, f)
+
+
+@pytest.mark.parametrize("seed", [1, 987654321])
+def test_normals_against_extended_precision(gpu, seed):
+    # z = sqrt(-2 log u) (cos, sin)(2 pi v), u and v from the uniform fill of the same streams; the angle is rounded
+    # to 64 bits as the reference does.  Radius and sine or cosine each within 3/4 of a unit in their last place, the
+    # product rounded once: 3.5 units in the last place of z at most.
+    lat = lmx.Lattice((8, 8, 8, 16))
+    key = lmx.RNGStreamKey(seed)
+    z, u = lat.spinor(1), lat.spinor(1)
+    lmx.randomize_gaussian_matrix_(z, key, sigma=1.0)
+    lmx.randomize_matrix_(u, key)
+    zz, w = z.to_numpy().reshape(-1), u.to_numpy().reshape(-1)
+    uu = w.real + 0.5
+    uu = np.where(uu == 0.0, 2.0 ** -54, uu).astype(np.longdouble)
+    angle = (6.283185307179586 * (w.imag + 0.5)).astype(np.longdouble)
+    radius = np.sqrt(-2 * np.log(uu))
+    for got, want in ((zz.real, radius * np.cos(angle)), (zz.imag, radius * np.sin(angle))):
+        err = np.abs(got - want) / np.spacing(np.abs(want.astype(np.float64)))
+        print(f"  max {float(err.max()):.2f} units in the last place", flush=True)
+        assert float(err.max()) <= 3.5
+
+
 def test_box_fills_are_slices_of_the_global_fill(gpu):
     G, box = (8, 4, 4, 8), (4, 4, 2, 4)
     key = lmx.RNGStreamKey(123, 9, 2)
