@@ -14,8 +14,11 @@
 //   last update), after reliable_maxiter iterations, or when the inner
 //   residual reaches the tolerance.  Convergence is declared only on the
 //   FP64 true residual.  The update decision is a device flag that gates the
-//   FP64 kernels, so one iteration is a fixed sequence of launches that can be
-//   captured once in a hipGraph and replayed.
+//   FP64 kernels: a group of kXBatch iterations and one gated update is a fixed
+//   sequence of launches that can be captured once in a hipGraph and replayed.
+//   The iteration that requests an update is the last of its group to run (the
+//   rest find their gate off), so an update still follows the iteration that
+//   asked for it.
 // The reference solver this replaces is cg! (src/LinearAlgebras/cg.jl:73-137)
 // on DdagDOp (src/Operators/DiracOperators.jl:104-121).
 #include <algorithm>
@@ -39,8 +42,11 @@ struct MixRhs {
     int fold;
 };
 struct MixBatch {
-    int do_update;  // reliable update requested this iteration
+    int do_update;  // reliable update requested in this group
     int n_active;   // RHS still iterating
+    int go;         // iterations run: an RHS is active and no update is pending
+    int live;       // go as the current iteration began
+    int ticket;     // RHS whose update has ended
     double delta;
     int rmax;
     int maxiter;    // an RHS stops once its inner iteration count reaches it
@@ -121,7 +127,7 @@ __device__ __forceinline__ void retire(MixRhs* st, MixBatch* batch, int reason, 
     st->reason = reason;
     st->converged = converged;
     st->fold = fold;
-    atomicSub(&batch->n_active, 1);
+    if (atomicSub(&batch->n_active, 1) == 1) batch->go = 0;
 }
 
 enum { MX_INIT = 0, MX_PAP = 1, MX_RR = 2, MX_TRUE = 3 };
@@ -134,12 +140,10 @@ enum { MX_INIT = 0, MX_PAP = 1, MX_RR = 2, MX_TRUE = 3 };
 // (cg!, src/LinearAlgebras/cg.jl:105,135-136), in the iteration's own
 // finalize, so a graph replay that runs past maxiter leaves it untouched.
 template <int KIND>
-__global__ void __launch_bounds__(256) k_mx_fin(const double* __restrict__ partials, int nb, MixRhs* rhs,
-                                                MixBatch* batch, double rtol, double atol, int flag) {
+__device__ __forceinline__ void mx_finish(const double* __restrict__ partials, int nb, MixRhs* rhs, MixBatch* batch,
+                                          double rtol, double atol, int flag) {
     const int i = blockIdx.x;
     MixRhs* st = rhs + i;
-    if (KIND == MX_PAP && i == 0 && threadIdx.x == 0) batch->do_update = 0;
-    if (KIND == MX_TRUE && !flag && !batch->do_update) return;
     const bool final_fold = KIND == MX_TRUE && flag && st->done && st->fold;
     if (st->done && !final_fold) return;
     if (threadIdx.x == 0) {
@@ -200,7 +204,10 @@ __global__ void __launch_bounds__(256) k_mx_fin(const double* __restrict__ parti
             retire(st, batch, LMX_CG_MAXITER, 0, 1);
             return;
         }
-        if (rn < batch->delta * st->rref || st->since >= batch->rmax || rn <= st->tol) atomicOr(&batch->do_update, 1);
+        if (rn < batch->delta * st->rref || st->since >= batch->rmax || rn <= st->tol) {
+            atomicOr(&batch->do_update, 1);
+            batch->go = 0;
+        }
     } else if (final_fold) {  // MX_TRUE on a retired RHS: A = |b - A x|^2 after its fold
         st->rtrue = sqrt(A);
         st->updates += 1;
@@ -221,6 +228,30 @@ __global__ void __launch_bounds__(256) k_mx_fin(const double* __restrict__ parti
             st->rr = A;
             st->rref = st->rtrue;
             st->since = 0;
+        }
+    }
+}
+
+// The iterations after an update request do nothing: MX_PAP keeps what go was
+// as the iteration began, since MX_RR itself may clear it.  The last RHS of an
+// update (MX_TRUE) lets the next group run.
+template <int KIND>
+__global__ void __launch_bounds__(256) k_mx_fin(const double* __restrict__ partials, int nb, MixRhs* rhs,
+                                                MixBatch* batch, double rtol, double atol, int flag) {
+    if (KIND == MX_PAP) {
+        const int go = batch->go;
+        if (blockIdx.x == 0 && threadIdx.x == 0) batch->live = go;
+        if (!go) return;
+    }
+    if (KIND == MX_RR && !batch->live) return;
+    if (KIND == MX_TRUE && !flag && !batch->do_update) return;
+    mx_finish<KIND>(partials, nb, rhs, batch, rtol, atol, flag);
+    if (KIND == MX_TRUE && !flag && threadIdx.x == 0) {
+        __threadfence();
+        if (atomicAdd(&batch->ticket, 1) == (int)gridDim.x - 1) {
+            batch->ticket = 0;
+            batch->do_update = 0;
+            batch->go = atomicAdd(&batch->n_active, 0) > 0;
         }
     }
 }
@@ -270,6 +301,9 @@ __global__ void k_mx_reset(MixRhs* rhs, MixBatch* batch, int nrhs, double delta,
     if (t == 0) {
         batch->do_update = 0;
         batch->n_active = nrhs;
+        batch->go = 1;
+        batch->live = 0;
+        batch->ticket = 0;
         batch->delta = delta;
         batch->rmax = rmax;
         batch->maxiter = maxiter;
@@ -326,17 +360,38 @@ __device__ __forceinline__ bool update_runs(const MixRhs& st, const MixBatch* ba
     return force ? (!st.done || st.fold) : (batch->do_update && !st.done);
 }
 
+// site s of an inner vector of RHS i, bit for bit
+__device__ __forceinline__ void copy_site(const SpF32In& from, const InnerVec& to, int V, int i, int s) {
+    const size_t o = (size_t)i * 12 * V + s;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) ((float2*)to.p)[o + (size_t)k * V] = from.p[o + (size_t)k * V];
+}
+__device__ __forceinline__ void copy_site(const SpH16In& from, const InnerVec& to, int V, int i, int s) {
+    const size_t o = (size_t)i * 3 * V + s;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) ((int4*)to.p)[o + (size_t)k * V] = from.p[o + (size_t)k * V];
+    to.n[(size_t)i * V + s] = from.scale[(size_t)i * V + s];
+}
+
+// An update that cuts a group short also puts the newest p where the next
+// group's first iteration reads it, in the ring's last slot.
 // (grid-stride over the sites: a small grid, so that the launch costs little
-// on the iterations where the update is gated off)
+// on the groups where the update is gated off)
 template <class SI>
 __global__ void __launch_bounds__(256) k_mx_accum(double2* __restrict__ x, float4* __restrict__ xlo, RingSlots<SI> ring,
-                                                  int V, const MixRhs* rhs, const MixBatch* batch, int force) {
+                                                  InnerVec last, int V, const MixRhs* rhs, const MixBatch* batch,
+                                                  int force) {
     const int i = blockIdx.y;
     if (!update_runs(rhs[i], batch, force)) return;
     const size_t o = (size_t)i * 12 * V, o4 = (size_t)i * 6 * V;
     const int mask = rhs[i].pmask;  // slots not yet overwritten by a later p update
-    for (int s = blockIdx.x * 256 + threadIdx.x; s < V; s += gridDim.x * 256)
+    for (int s = blockIdx.x * 256 + threadIdx.x; s < V; s += gridDim.x * 256) {
         accum_site(x, xlo, ring, V, rhs[i], mask, o, o4, i, s);
+        if (force) continue;
+#pragma unroll
+        for (int j = 0; j < kXBatch - 1; ++j)
+            if (mask >> j == 1) copy_site(ring.p[j], last, V, i, s);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -352,6 +407,7 @@ struct MixRun {
     int link_prec;
     int spinor_prec;
     int rhs_block;
+    bool update_each;  // the gated update after every iteration, not every group
 };
 
 template <class SI>
@@ -393,14 +449,14 @@ static LoArgs lo_args(lmx_wilson* op, int link_prec, int spinor_prec) {
 //   alpha p (its p stays in ring slot j, the finalize records alpha and
 //   marks the slot), the group's last phase adds the marked terms and its own
 //   alpha p -- the x_inner traffic of one iteration for kXBatch.  A reliable
-//   update inside a group folds the marked terms into x in k_mx_accum.
+//   update that ends a group early folds the marked terms into x in k_mx_accum.
 static_assert(sizeof(MixRhs) % sizeof(double) == 0, "MixRhs is addressed in doubles and ints");
 
 static int apply_d_tp(MixRun& R, int e) {
     LoArgs a = lo_args(R.op, R.link_prec, R.spinor_prec);
     a.nrhs = R.nrhs;
     a.rhs_block = R.rhs_block;
-    a.gate = &R.w.batch->n_active;
+    a.gate = &R.w.batch->go;
     a.out = R.w.t.p;
     a.out_norm = R.w.t.n;
     a.in = R.w.r.p;
@@ -425,7 +481,7 @@ static int apply_ddag_xr(MixRun& R, int e) {
     LoArgs a = lo_args(R.op, R.link_prec, R.spinor_prec);
     a.nrhs = R.nrhs;
     a.rhs_block = R.rhs_block;
-    a.gate = &R.w.batch->n_active;
+    a.gate = &R.w.batch->go;
     a.out = nullptr;  // Ap is consumed in registers
     a.in = R.w.t.p;
     a.in_norm = R.w.t.n;
@@ -452,7 +508,7 @@ static int apply_ddag_xr(MixRun& R, int e) {
     return launch_wilson_lo(R.ctx, a);
 }
 
-// The reliable-update kernels run on most iterations only to find their gate
+// The reliable-update kernels run after most groups only to find their gate
 // off; they stride over the lattice with at most this many workgroups per RHS.
 constexpr unsigned kUpdateBlocks = 256;
 
@@ -487,13 +543,18 @@ static void enqueue_accum(MixRun& R, dim3 grid, int force) {
     grid.x = std::min(grid.x, kUpdateBlocks);
     if (R.spinor_prec == LMX_H16)
         hipLaunchKernelGGL((k_mx_accum<SpH16In>), grid, dim3(256), 0, R.ctx->stream, R.x, R.w.xlo, ring_of<SpH16In>(R),
-                           V, R.w.rhs, R.w.batch, force);
+                           R.w.p[kXBatch - 1], V, R.w.rhs, R.w.batch, force);
     else
         hipLaunchKernelGGL((k_mx_accum<SpF32In>), grid, dim3(256), 0, R.ctx->stream, R.x, R.w.xlo, ring_of<SpF32In>(R),
-                           V, R.w.rhs, R.w.batch, force);
+                           R.w.p[kXBatch - 1], V, R.w.rhs, R.w.batch, force);
 }
 
-// One iteration with phase e (iteration k has e = k % kXBatch).
+// One iteration with phase e in its group, and after the group's last one the
+// gated update.  A launch that finds its gate off still costs 1.5 us, and only
+// one iteration in 18 (8^3 x 16) to 35 (24^3 x 48) asks for an update: with the
+// update's four launches after every iteration one right-hand side in 16 bits
+// took 33.9 us an iteration at 8^3 x 16 against 28.8, four with FP16 links
+// 93.2 at 16^4 against 89.3.
 static int enqueue_iteration(MixRun& R, int e) {
     lmx_context* c = R.ctx;
     dim3 grid(nblocks(c->V), R.nrhs), blk(256);
@@ -504,9 +565,11 @@ static int enqueue_iteration(MixRun& R, int e) {
     hipLaunchKernelGGL(k_mx_fin<MX_PAP>, dim3(R.nrhs), blk, 0, c->stream, R.w.partials, nb, rhs, bt, 0.0, 0.0, 0);
     LMX_TRY(apply_ddag_xr(R, e));
     hipLaunchKernelGGL(k_mx_fin<MX_RR>, dim3(R.nrhs), blk, 0, c->stream, R.w.partials, nb, rhs, bt, 0.0, 0.0, e);
-    enqueue_accum(R, grid, 0);
-    LMX_TRY(enqueue_true_ddagd(R, R.x, &bt->do_update, 0));
-    hipLaunchKernelGGL(k_mx_fin<MX_TRUE>, dim3(R.nrhs), blk, 0, c->stream, R.w.partials, nb, rhs, bt, 0.0, 0.0, 0);
+    if (R.update_each || e == kXBatch - 1) {
+        enqueue_accum(R, grid, 0);
+        LMX_TRY(enqueue_true_ddagd(R, R.x, &bt->do_update, 0));
+        hipLaunchKernelGGL(k_mx_fin<MX_TRUE>, dim3(R.nrhs), blk, 0, c->stream, R.w.partials, nb, rhs, bt, 0.0, 0.0, 0);
+    }
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }
@@ -583,6 +646,7 @@ int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void
     R.rhs_block = params->rhs_block > 0 ? params->rhs_block : default_rhs_block(op, params->precision, nrhs);
     dim3 grid(nblocks(c->V), nrhs), blk(256);
     const int rmax = params->reliable_maxiter > 0 ? params->reliable_maxiter : 100;
+    R.update_each = rmax < 2 * kXBatch;  // updates so dense that most groups would be cut short
     hipLaunchKernelGGL(k_mx_reset, dim3(1), dim3(64), 0, c->stream, R.w.rhs, R.w.batch, nrhs, params->reliable_delta,
                        rmax, params->maxiter);
     LMX_TRY(apply_ddagd64(R, R.w.r64, x, R.w.t64, nullptr));
@@ -594,8 +658,8 @@ int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void
                        R.w.batch, params->rtol, params->atol, 0);
     LMX_HIP(hipGetLastError());
 
-    // iterations between host polls; a multiple of kXBatch with a graph, so
-    // every replay starts a group (the x_inner batching groups iterations)
+    // iterations enqueued between host polls; a multiple of kXBatch with a
+    // graph, so every replay starts a group
     int chunk = params->check_every > 0 ? params->check_every : 10;
     if (params->use_graph) chunk = (chunk + kXBatch - 1) / kXBatch * kXBatch;
     hipGraphExec_t exec = nullptr;
@@ -620,12 +684,15 @@ int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void
     }
     std::vector<MixRhs> hs(nrhs);
     MixBatch hb;
-    int launched = 0;
+    // every group runs at least one of its iterations, so the device has
+    // retired all RHS by maxiter at the latest after maxiter groups
+    const int64_t most = (int64_t)kXBatch * params->maxiter;
+    int64_t launched = 0;
     int rc = LMX_OK;
     while (true) {
         LMX_HIP(hipMemcpyAsync(&hb, R.w.batch, sizeof(MixBatch), hipMemcpyDeviceToHost, c->stream));
         LMX_HIP(hipStreamSynchronize(c->stream));
-        if (hb.n_active <= 0 || launched >= params->maxiter) break;
+        if (hb.n_active <= 0 || launched >= most) break;
         if (exec) {
             if (hipGraphLaunch(exec, c->stream) != hipSuccess) {
                 rc = LMX_ERR_HIP;
@@ -634,10 +701,9 @@ int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void
             }
             launched += chunk;
         } else {
-            const int n = std::min(chunk, params->maxiter - launched);
-            for (int k = 0; k < n && rc == LMX_OK; ++k) rc = enqueue_iteration(R, (launched + k) % kXBatch);
+            for (int k = 0; k < chunk && rc == LMX_OK; ++k) rc = enqueue_iteration(R, (int)((launched + k) % kXBatch));
             if (rc != LMX_OK) break;
-            launched += n;
+            launched += chunk;
         }
     }
     if (exec) (void)hipGraphExecDestroy(exec);

@@ -362,3 +362,30 @@ def test_lds_stage_shape(gpu, precision, csw, L):
         assert r.converged and tr <= rtol * 1.05 and err <= 1e-7
     t = lmx.inner_kernel_times(D, precision, 3, LDS_STAGE | shape, groups=1)
     assert t["D"] > 0 and t["Ddag"] > 0
+
+
+@pytest.mark.parametrize("precision", ["f32", "f16", "h16"])
+@pytest.mark.parametrize("reliable_maxiter", [1, 7, 8, 9, 10, 11])
+def test_updates_at_every_phase_of_a_group(gpu, precision, reliable_maxiter):
+    # iterations run in groups of four, and one that asks for a reliable update is the last of its group to run:
+    # periods of 8 to 11 end on each phase, below 8 the update follows every iteration.  The right-hand sides
+    # differ, one of them is zero (converged at once), and a period is never exceeded.
+    L, kappa, rtol = (8, 4, 4, 8), 0.12, 1e-10
+    U, b, lat, Ug, D = setup(L, "weak", 395, kappa, nrhs=3)
+    b = np.array(b)
+    b[1] = 0.0
+    bg = lat.spinor_from_numpy(b)
+    xs = []
+    for graph, every in ((False, 1), (False, 10), (True, 10)):
+        x = lat.spinor(3)
+        res = lmx.cg_batched_(x, D, bg, precision=precision, rtol=rtol, use_graph=graph, check_every=every,
+                              reliable_delta=1e-8, reliable_maxiter=reliable_maxiter)
+        assert all(r.converged for r in res) and res[1].iterations == 0
+        for r in (res[0], res[2]):
+            assert r.reliable_updates >= r.iterations // reliable_maxiter
+        xs.append((x.to_numpy(), [(r.iterations, r.reliable_updates) for r in res]))
+    assert xs[0][1] == xs[1][1] == xs[2][1]
+    assert np.array_equal(xs[0][0], xs[1][0]) and np.array_equal(xs[0][0], xs[2][0])
+    A = orc.NormalOp(orc.OP_DDAGD_WILSON, L, U=U, kappa=kappa)
+    for k in (0, 2):
+        assert np.linalg.norm(A.apply(xs[0][0][k]) - b[k]) <= 1.05 * rtol * np.linalg.norm(b[k])
