@@ -150,6 +150,10 @@ __device__ __forceinline__ void mat_mul_plain(const cx<double> A[9], const cx<do
             out[3 * i + j] =
                 cadd(cadd(cmul(A[3 * i], B[j]), cmul(A[3 * i + 1], B[3 + j])), cmul(A[3 * i + 2], B[6 + j]));
 }
+__device__ __forceinline__ void add9(cx<double> (&a)[9], const cx<double> (&b)[9]) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) a[k] = cadd(a[k], b[k]);
+}
 __device__ __forceinline__ void mat_dag(const cx<double> A[9], cx<double> out[9]) {
 #pragma unroll
     for (int i = 0; i < 3; ++i)
@@ -234,21 +238,17 @@ __global__ void __launch_bounds__(256) k_clover_cotangent(double2* __restrict__ 
     cotangent_plane<5, 2, 3>(dQ, d, p, s, V, coefficient);
 }
 
-__device__ __forceinline__ void ld_link(const double2* __restrict__ U, int V, int mu, int s, bool dag, cx<double> u[9]) {
+__device__ __forceinline__ void ld_link(const double2* U, int V, int mu, int s, bool dag, cx<double> (&u)[9]) {
+    cx<double> v[9];
+    ld_comps(U + (size_t)mu * 9 * V, V, s, v);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const double2 v = ldv(U + (size_t)(mu * 9 + 3 * i + j) * V, s);
-            if (dag)
-                u[3 * j + i] = mk<double>(v.x, -v.y);
-            else
-                u[3 * i + j] = mk<double>(v.x, v.y);
-        }
+        for (int j = 0; j < 3; ++j) u[3 * i + j] = dag ? cconj(v[3 * j + i]) : v[3 * i + j];
 }
 // dQ of plane pl at s, or its adjoint (exactly -dQ)
 template <bool DAG>
-__device__ __forceinline__ void ld_dq(const double2* __restrict__ dQ, int V, int pl, int s, cx<double> q[9]) {
+__device__ __forceinline__ void ld_dq(const double2* dQ, int V, int pl, int s, cx<double> q[9]) {
     const double2* a = dQ + (size_t)pl * 5 * V;
     const double2 d01 = ldv(a, s), d2 = ldv(a + (size_t)V, s), u0 = ldv(a + (size_t)2 * V, s),
                   u1 = ldv(a + (size_t)3 * V, s), u2 = ldv(a + (size_t)4 * V, s);
@@ -266,69 +266,117 @@ __device__ __forceinline__ void ld_dq(const double2* __restrict__ dQ, int V, int
         for (int k = 0; k < 9; ++k) q[k] = cneg(q[k]);
     }
 }
-__device__ __forceinline__ void mat_add(cx<double> a[9], const cx<double> b[9], bool first) {
+// keep a matrix in registers here: the loads that follow are not hoisted above it
+__device__ __forceinline__ void pin9(cx<double> (&a)[9]) {
 #pragma unroll
-    for (int k = 0; k < 9; ++k) a[k] = first ? b[k] : cadd(a[k], b[k]);
+    for (int k = 0; k < 9; ++k) asm volatile("" : "+v"(a[k].re), "+v"(a[k].im)::"memory");
 }
 
 // The terms of one plaquette loop through a link L at y: L A B C (DAG false)
-// or L^dagger A B C, leaf number p of the plane being the loop begun at
-// another corner.  Begun at L the cotangent enters before L (site s0), at C
-// before C (s3), at B before B (s2), at A before A (s1); with X Y the factors
-// to its left and right in the leaf, the term is X^dagger dQ Y^dagger, or
-// Y dQ^dagger X.  H[p] sums the two terms a leaf has for this link (two terms
-// and a zero: any order), P0..P3 the leaves of the loops begun at L, C, B, A.
-template <bool DAG, bool DA, bool DB, bool DC, int P0, int P1, int P2, int P3, bool FIRST>
-__device__ __forceinline__ void plaquette_terms(const double2* __restrict__ U, const double2* __restrict__ dQ, int V,
-                                                int pl, int mA, int sA, int mB, int sB, int mC, int sC, int s0, int s1,
-                                                int s2, int s3, cx<double> (&H)[4][9]) {
-    cx<double> A[9], B[9], C[9], AB[9], X[9], t[9], h[9], q[9], y[9];
-    ld_link(U, V, mA, sA, DA, A);
-    ld_link(U, V, mB, sB, DB, B);
-    ld_link(U, V, mC, sC, DC, C);
-    mat_mul_plain(B, C, X);  // B C
-    ld_dq<DAG>(dQ, V, pl, s2, q);
-    if (!DAG) {
-        mat_dag(X, t);
-        mat_mul_plain(t, q, y);
-        mat_dag(A, t);
-        mat_mul_plain(y, t, h);
-    } else {
-        mat_mul_plain(A, q, t);
-        mat_mul_plain(t, X, h);
-    }
-    mat_add(H[P2], h, FIRST);
-    mat_mul_plain(A, B, AB);
-    ld_dq<DAG>(dQ, V, pl, s3, q);
-    if (!DAG) {
-        mat_dag(C, t);
-        mat_mul_plain(t, q, y);
-        mat_dag(AB, t);
-        mat_mul_plain(y, t, h);
-    } else {
-        mat_mul_plain(AB, q, t);
-        mat_mul_plain(t, C, h);
-    }
-    mat_add(H[P1], h, FIRST);
-    mat_mul_plain(AB, C, X);  // (A B) C
-    if (!DAG) {
-        mat_dag(X, t);
-        ld_dq<DAG>(dQ, V, pl, s0, q);
-        mat_mul_plain(q, t, h);
-        mat_add(H[P0], h, FIRST);
-        ld_dq<DAG>(dQ, V, pl, s1, q);
-        mat_mul_plain(t, q, h);
-        mat_add(H[P3], h, FIRST);
-    } else {
-        ld_dq<DAG>(dQ, V, pl, s0, q);
-        mat_mul_plain(X, q, h);
-        mat_add(H[P0], h, FIRST);
-        ld_dq<DAG>(dQ, V, pl, s1, q);
-        mat_mul_plain(q, X, h);
-        mat_add(H[P3], h, FIRST);
-    }
-}
+// or L^dagger A B C, the leaves of the plane being the loop begun at its four
+// corners.  Begun at L the cotangent enters before L (site s0), at C before C
+// (s3), at B before B (s2), at A before A (s1); with X Y the factors to its
+// left and right in the leaf, the term is X^dagger dQ Y^dagger, or
+// Y dQ^dagger X.  Links are loaded where they are used, so that few matrices
+// are live at once.
+template <bool DAG, bool DA, bool DB, bool DC>
+struct Plaquette {
+    const double2 *U, *dQ;
+    int V, pl, mA, sA, mB, sB, mC, sC, s0, s1, s2, s3;
 
+    // (the pointer is made opaque, or a link that another term needs again would be kept, spilled, instead)
+    __device__ __forceinline__ void lnk(int mu, int s, bool dag, cx<double> (&u)[9]) const {
+        const double2* p = U;
+        asm volatile("" : "+s"(p));
+        ld_link(p, V, mu, s, dag, u);
+    }
+    __device__ __forceinline__ void link_b(cx<double> (&B)[9]) const { lnk(mB, sB, DB, B); }
+    // z = X^dagger dQ of site s (DAG false), or Y dQ^dagger
+    __device__ __forceinline__ void dq_left(const cx<double> (&X)[9], int s, cx<double> (&z)[9]) const {
+        cx<double> q[9], t[9];
+        ld_dq<DAG>(dQ, V, pl, s, q);
+        mat_dag(X, t);
+        mat_mul_plain(t, q, z);
+        pin9(z);
+    }
+    __device__ __forceinline__ void dq_right(const cx<double> (&Y)[9], int s, cx<double> (&z)[9]) const {
+        cx<double> q[9];
+        ld_dq<DAG>(dQ, V, pl, s, q);
+        mat_mul_plain(Y, q, z);
+        pin9(z);
+    }
+    // (B C)^dagger dQ A^dagger or A dQ^dagger (B C); A and B are given back
+    template <class F>
+    __device__ __forceinline__ void begun_at_b(cx<double> (&A)[9], cx<double> (&B)[9], F&& emit) const {
+        cx<double> X[9], z[9];
+        {
+            cx<double> C[9];
+            lnk(mB, sB, DB, B);
+            lnk(mC, sC, DC, C);
+            mat_mul_plain(B, C, X);
+        }
+        pin9(X);
+        lnk(mA, sA, DA, A);
+        if (!DAG) {
+            dq_left(X, s2, z);
+            cx<double> t[9];
+            mat_dag(A, t);
+            mul_emit(z, t, emit);
+        } else {
+            dq_right(A, s2, z);
+            mul_emit(z, X, emit);
+        }
+    }
+    // C^dagger dQ (A B)^dagger or (A B) dQ^dagger C; C is given back
+    template <class F>
+    __device__ __forceinline__ void begun_at_c(const cx<double> (&AB)[9], cx<double> (&C)[9], F&& emit) const {
+        cx<double> z[9];
+        lnk(mC, sC, DC, C);
+        if (!DAG) {
+            dq_left(C, s3, z);
+            cx<double> t[9];
+            mat_dag(AB, t);
+            mul_emit(z, t, emit);
+        } else {
+            dq_right(AB, s3, z);
+            mul_emit(z, C, emit);
+        }
+    }
+    // X = A B C: dQ X^dagger or X dQ^dagger
+    template <class F>
+    __device__ __forceinline__ void begun_at_l(const cx<double> (&X)[9], F&& emit) const {
+        cx<double> q[9], t[9];
+        ld_dq<DAG>(dQ, V, pl, s0, q);
+        if (!DAG) {
+            mat_dag(X, t);
+            mul_emit(q, t, emit);
+        } else {
+            mul_emit(X, q, emit);
+        }
+    }
+    // X^dagger dQ or dQ^dagger X
+    template <class F>
+    __device__ __forceinline__ void begun_at_a(const cx<double> (&X)[9], F&& emit) const {
+        cx<double> q[9], t[9];
+        ld_dq<DAG>(dQ, V, pl, s1, q);
+        if (!DAG) {
+            mat_dag(X, t);
+            mul_emit(t, q, emit);
+        } else {
+            mul_emit(q, X, emit);
+        }
+    }
+    // emit(k, entry k of a b)
+    template <class F>
+    static __device__ __forceinline__ void mul_emit(const cx<double> (&a)[9], const cx<double> (&b)[9], F&& emit) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                emit(3 * i + j,
+                     cadd(cadd(cmul(a[3 * i], b[j]), cmul(a[3 * i + 1], b[3 + j])), cmul(a[3 * i + 2], b[6 + j])));
+    }
+};
 // Neighbour of a site (with its coordinates) one step along +-mu.
 __device__ __forceinline__ int step_site(const Geom& g, int s, const int x[4], int mu, bool fwd) {
     bool w;
@@ -339,26 +387,28 @@ __device__ __forceinline__ int step_site(const Geom& g, int s, const int x[4], i
 // takes U_a of 64 sites, with the three planes that hold direction a and in
 // each the plaquette on either side.  The four leaves that share a plaquette
 // share its partial products (three products and six with dQ where the leaves
-// one by one take twelve), and the four wavefronts share their links in L1.
-// Bound by the unfused FP64 products (the operation order is the reference's):
-// 216 3x3 products or 43k operations per site, 148 us at 16^3 x 32 with every
-// lane busy; measured 324 us there, against 1142 us for one work item per
-// site that walked the paths through arrays in scratch.
-__global__ void __launch_bounds__(256, 1) k_clover_links_pullback(double2* __restrict__ dU,
-                                                                  const double2* __restrict__ U,
-                                                                  const double2* __restrict__ dQ, Geom g) {
-    const int y = xcd_block(blockIdx.x, gridDim.x) * 64 + (threadIdx.x & 63);
+// one by one take twelve).  Bound by the unfused FP64 products (the operation
+// order is the reference's): 216 3x3 products or 43k operations per site,
+// 148 us at 16^3 x 32 at the nominal rate with every lane busy, 190 us at the
+// 4.8 cycles an instruction that two wavefronts per SIMD reach.  A wavefront
+// alone issues an FP64 instruction every six cycles, so the terms come in an
+// order that keeps few matrices at once, two wait in LDS and one link is read
+// twice: 248 registers and two wavefronts per SIMD, 284 us against 324 with
+// everything in 460 registers at one.  (More links read again and less parked
+// loses it: 320 us at 1.4 times the loads.)  Blocks in the stencil's slab order.
+__global__ void __launch_bounds__(256, 2) k_clover_links_pullback(double2* dU,
+                                                                  const double2* U,
+                                                                  const double2* dQ, Geom g, int slab) {
+    // matrices that wait while others need the registers (each work item its own)
+    __shared__ double2 park[2][9][256];
+    int y0, end;
+    slab_block(xcd_block(blockIdx.x, gridDim.x), slab, g, y0, end);
+    const int y = y0 + (threadIdx.x & 63);
     const int a = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (y >= g.V) return;
+    if (y >= end) return;
     const int V = g.V;
     int x[4];
     site_coords(y, g, x);
-    cx<double> out[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-        const double2 v = ldv(dU + (size_t)(a * 9 + k) * V, y);
-        out[k] = mk<double>(v.x, v.y);
-    }
     const int ya = step_site(g, y, x, a, true);
     int xa[4] = {x[0], x[1], x[2], x[3]};
 #pragma unroll
@@ -371,26 +421,87 @@ __global__ void __launch_bounds__(256, 1) k_clover_links_pullback(double2* __res
         const int pl = lo == 0 ? hi - 1 : lo + hi;  // (01,02,03,12,13,23)
         const int yb = step_site(g, y, x, b, true), ymb = step_site(g, y, x, b, false);
         const int yab = step_site(g, ya, xa, b, true), yamb = step_site(g, ya, xa, b, false);
-        cx<double> H[4][9];
+        // h_p: the two terms of leaf p; h0 becomes ((h0 + h1) + h2) + h3
+        cx<double> h0[9], h1[9], A[9], B[9], AB[9], C[9], X[9];
+        const auto set = [](cx<double> (&h)[9]) { return [&h](int k, cx<double> v) { h[k] = v; }; };
+        const auto add = [](cx<double> (&h)[9]) { return [&h](int k, cx<double> v) { h[k] = cadd(h[k], v); }; };
+        const auto put = [&](int j) {
+            return [j](int k, cx<double> v) { park[j][k][threadIdx.x] = make_double2(v.re, v.im); };
+        };
+        // the parked term completes leaf j's two terms
+        const auto fetch_add = [&](int j, cx<double> (&h)[9]) {
+            return [&h, j](int k, cx<double> v) {
+                const double2 o = park[j][k][threadIdx.x];
+                h[k] = cadd(mk<double>(o.x, o.y), v);
+            };
+        };
         if (a < b) {
             // U_a is the plane's first direction: L U_b(y+a) U_a(y+b)^+ U_b(y)^+ and
             // L^+ U_b(y-b)^+ U_a(y-b) U_b(y-b+a)
-            plaquette_terms<false, false, true, true, 0, 3, 2, 1, true>(U, dQ, V, pl, b, ya, a, yb, b, y, y, ya, yab, yb,
-                                                                       H);
-            plaquette_terms<true, true, false, false, 2, 1, 0, 3, false>(U, dQ, V, pl, b, ymb, a, ymb, b, yamb, ya, y, ymb,
-                                                                        yamb, H);
+            const Plaquette<false, false, true, true> p{U, dQ, V, pl, b, ya, a, yb, b, y, y, ya, yab, yb};
+            const Plaquette<true, true, false, false> m{U, dQ, V, pl, b, ymb, a, ymb, b, yamb, ya, y, ymb, yamb};
+            p.begun_at_b(A, B, put(0));  // leaf 2
+            mat_mul_plain(A, B, AB);
+            pin9(AB);
+            p.begun_at_c(AB, C, put(1));  // leaf 3
+            mat_mul_plain(AB, C, X);
+            pin9(X);
+            p.begun_at_l(X, set(h0));
+            pin9(h0);
+            p.begun_at_a(X, set(h1));
+            pin9(h1);
+            m.begun_at_b(A, B, add(h0));
+            pin9(h0);
+            m.link_b(B);
+            mat_mul_plain(A, B, AB);
+            pin9(AB);
+            m.begun_at_c(AB, C, add(h1));
+            add9(h0, h1);
+            pin9(h0);
+            mat_mul_plain(AB, C, X);
+            pin9(X);
+            m.begun_at_l(X, fetch_add(0, h1));
+            add9(h0, h1);
+            pin9(h0);
+            m.begun_at_a(X, fetch_add(1, h1));
+            add9(h0, h1);
         } else {
             // the second: L U_b(y-b+a)^+ U_a(y-b)^+ U_b(y-b) and L^+ U_b(y) U_a(y+b) U_b(y+a)^+
-            plaquette_terms<false, true, true, false, 1, 0, 3, 2, true>(U, dQ, V, pl, b, yamb, a, ymb, b, ymb, y, ya, yamb,
-                                                                       ymb, H);
-            plaquette_terms<true, false, false, true, 3, 2, 1, 0, false>(U, dQ, V, pl, b, y, a, yb, b, ya, ya, y, yb, yab,
-                                                                        H);
+            const Plaquette<false, true, true, false> p{U, dQ, V, pl, b, yamb, a, ymb, b, ymb, y, ya, yamb, ymb};
+            const Plaquette<true, false, false, true> m{U, dQ, V, pl, b, y, a, yb, b, ya, ya, y, yb, yab};
+            p.begun_at_b(A, B, put(0));  // leaf 3
+            mat_mul_plain(A, B, AB);
+            pin9(AB);
+            p.begun_at_c(AB, C, set(h0));
+            pin9(h0);
+            mat_mul_plain(AB, C, X);
+            pin9(X);
+            p.begun_at_a(X, put(1));  // leaf 2
+            p.begun_at_l(X, set(h1));
+            pin9(h1);
+            m.begun_at_b(A, B, add(h1));
+            pin9(h1);
+            m.link_b(B);
+            mat_mul_plain(A, B, AB);
+            pin9(AB);
+            cx<double> h2[9];
+            m.begun_at_c(AB, C, fetch_add(1, h2));
+            pin9(h2);
+            mat_mul_plain(AB, C, X);
+            pin9(X);
+            m.begun_at_a(X, add(h0));
+            add9(h0, h1);
+            add9(h0, h2);
+            pin9(h0);
+            m.begun_at_l(X, fetch_add(0, h1));
+            add9(h0, h1);
         }
 #pragma unroll
-        for (int k = 0; k < 9; ++k) out[k] = cadd(out[k], cadd(cadd(cadd(H[0][k], H[1][k]), H[2][k]), H[3][k]));
+        for (int k = 0; k < 9; ++k) {
+            double2* o = dU + (size_t)(a * 9 + k) * V + y;
+            *o = make_double2(o->x + h0[k].re, o->y + h0[k].im);
+        }
     }
-#pragma unroll
-    for (int k = 0; k < 9; ++k) dU[(size_t)(a * 9 + k) * V + y] = make_double2(out[k].re, out[k].im);
 }
 
 int launch_clover_pullback(lmx_context* ctx, double2* dU, const double2* U, double2* dQ, const double2* dres,
@@ -398,8 +509,9 @@ int launch_clover_pullback(lmx_context* ctx, double2* dU, const double2* U, doub
     if (ctx->V == 0) return LMX_OK;
     hipLaunchKernelGGL(k_clover_cotangent, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, dQ, dres, psi,
                        (int)ctx->V, coefficient);
-    hipLaunchKernelGGL(k_clover_links_pullback, dim3((unsigned)((ctx->V + 63) / 64)), dim3(256), 0, ctx->stream, dU, U,
-                       (const double2*)dQ, ctx->g);
+    const SlabOrder so = slab_order(ctx->g, false);
+    hipLaunchKernelGGL(k_clover_links_pullback, dim3((unsigned)so.blocks), dim3(256), 0, ctx->stream, dU, U,
+                       (const double2*)dQ, ctx->g, so.slab);
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }
