@@ -116,9 +116,13 @@ __device__ __forceinline__ void put_clover_share(LdsCx<R> (&F)[27][kHopSites], i
 #pragma unroll
     for (int k = 0; k < CloverShare<W>::kNum; ++k) F[CloverShare<W>::kFirst + k][lane] = f[k];
 }
-template <typename R, int MODE>
+// Several fields alternate between two buffers, so that one barrier a field
+// is enough: the products of a field overwrite what was summed two fields ago
+// (one buffer and two barriers: four FP64 fields at 24^3 x 48 490 us against
+// 456, twelve FP32 ones at 32^4 1249 against 1165).
+template <typename R, int MODE, bool LOOP>
 struct HopLds {
-    HopBuf<R> b;
+    HopBuf<R> b[LOOP ? 2 : 1];
     LdsCx<R> psi[MODE == MODE_CLOVER ? 12 : 1][kHopSites];  // the site's own spinor, for the clover term
 };
 // two components of the site's own spinor
@@ -210,7 +214,7 @@ struct HopArgs {
 
 // Wavefront W's part of the workgroup (hop W; the sum of two components for W < 6).
 template <int W, int FPM, int MODE, int EPI, bool GP, bool LOOP, class In, class Lk, class Out, class Cl>
-__device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopLds<typename In::R, MODE>& sh,
+__device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopLds<typename In::R, MODE, LOOP>& sh,
                                          double (*pap)[kHopSites], const Geom& g, int s0, int lane, int end) {
     using R = typename In::R;
     constexpr int MU = W >> 1;
@@ -235,9 +239,10 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
     const int r1 = LOOP ? a.r1 : a.r0 + 1;
     for (int r = a.r0; r < r1; ++r) {
         cx<R> o[6], mine[2];
+        HopBuf<R>& buf = sh.b[LOOP ? (r - a.r0) & 1 : 0];
         hop_product<MU, PM, FWD, GP>(psi, u, w, g, o);
 #pragma unroll
-        for (int k = 0; k < 6; ++k) sh.b.hop[W][k][lane] = o[k];
+        for (int k = 0; k < 6; ++k) buf.hop[W][k][lane] = o[k];
         if constexpr (W < 6 && MODE != MODE_DONLY) {
             mine[0] = own[0];
             mine[1] = own[1];
@@ -255,10 +260,10 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
         if constexpr (MODE == MODE_CLOVER) ld_clover_share<W>(a.F, g.V, s, f);
         __syncthreads();
         cx<R> ra, rb;
-        if constexpr (W < 6) sum_hops<FPM, kHigh>(sh.b.hop, c, lane, ra, rb);
+        if constexpr (W < 6) sum_hops<FPM, kHigh>(buf.hop, c, lane, ra, rb);
         if constexpr (MODE == MODE_CLOVER) {
             __syncthreads();
-            put_clover_share<W>(sh.b.F, lane, f);
+            put_clover_share<W>(buf.F, lane, f);
             __syncthreads();
         }
         if constexpr (W < 6) {
@@ -270,7 +275,7 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
                 ra = cadd(mine[0], rmul(-a.kappa, ra));
                 rb = cadd(mine[1], rmul(-a.kappa, rb));
                 if constexpr (MODE == MODE_CLOVER)
-                    clover_pair<c, kHigh>(sh.b.F, sh.psi, lane, a.ccoef, ra, rb);
+                    clover_pair<c, kHigh>(buf.F, sh.psi, lane, a.ccoef, ra, rb);
             }
             if (live) {
                 a.out.st1(r, ka, s, ra);
@@ -283,7 +288,7 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
                 pap[kb][lane] = live ? cmul(cconj(pb), rb).re : 0.0;
             }
         }
-        if (LOOP || EPI == EPI_PAP) __syncthreads();
+        if (EPI == EPI_PAP) __syncthreads();
         if constexpr (EPI == EPI_PAP && W == 7) {
             double v = 0.0;
 #pragma unroll
@@ -296,7 +301,7 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
 
 // Wavefronts per SIMD to compile for: one field, all that LDS admits; several,
 // where the next field's operands stay in registers across the sum, half (FP64
-// at 4: spills, 24^3 x 48 x 4 597 us against 471).
+// at 4: spills, 24^3 x 48 x 4 597 us against 456).
 template <typename R>
 constexpr int hop_waves(bool loop) {
     return sizeof(R) == 8 ? (loop ? 2 : 4) : (loop ? 4 : 6);
@@ -310,7 +315,8 @@ __global__ void __launch_bounds__(512, hop_waves<typename In::R>(LOOP))
     using R = typename In::R;
     if (epi.st != nullptr && epi.st->done) return;
     if (epi.gate != nullptr && *epi.gate == 0) return;
-    __shared__ HopLds<R, MODE> sh;
+    static_assert(!LOOP || (MODE != MODE_CLOVER && EPI == EPI_NONE), "one barrier a field");
+    __shared__ HopLds<R, MODE, LOOP> sh;
     __shared__ double pap[EPI == EPI_PAP ? 12 : 1][kHopSites];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

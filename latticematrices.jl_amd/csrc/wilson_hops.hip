@@ -41,7 +41,7 @@ bool hops_f64(const lmx_context* ctx, int nrhs, bool clover) {
     // One field: 32^3 x 16 122 / 115, 32^4 253 / 230, but 16^3 x 32 26 / 31,
     // 24^3 x 48 146 / 198, 40^3 x 80 1185 / 1310, 48^3 x 96 2610 / 2920.
     // Several, two of them to its work item: 32^4 x 4 798 / 684, 40^3 x 80 x 2
-    // 2270 / 1940, but 16^3 x 32 x 4 80 / 93, 24^3 x 48 x 4 471 / 598.
+    // 2270 / 1940, but 16^3 x 32 x 4 80 / 93, 24^3 x 48 x 4 456 / 598.
     return st.tl < 8 || st.fill < 0.8 || (nrhs == 1 && st.wgs > 256);
 }
 
@@ -52,7 +52,7 @@ bool hops_f32(const lmx_context* ctx, int nrhs, bool clover) {
     // one field: 32^4 151 / 145, clover 200 / 189, but 24^3 x 48 63 / 79, clover
     // 113 / 129, 40^3 x 80 682 / 718, clover 908 / 920
     if (nrhs == 1) return st.tl < 8 || st.fill < 0.8 || st.wgs > 512;
-    // several share the links: 24^3 x 48 x 4 266 / 341, 32^4 x 12 1246 / 1546
+    // several share the links: 24^3 x 48 x 4 262 / 341, 32^4 x 12 1165 / 1546
     if (!clover) return true;
     // clover fields do not: 16^4 x 4 32 / 34, 24^3 x 48 x 4 371 / 417, 27x29x31x35
     // x 12 1460 / 1546, but 16^3 x 32 x 12 195 / 176, 20^3 x 40 x 4 171 / 165,

@@ -40,6 +40,30 @@ def test_wilson(gpu, L, phases, flags):
     assert np.array_equal(y.to_numpy(), ref)
 
 
+@pytest.mark.parametrize("nrhs", [2, 3, 13])  # even and odd numbers in turn; a second group of one
+@pytest.mark.parametrize("donly", [False, True])
+def test_fields_that_take_turns_in_a_workgroup(gpu, nrhs, donly):
+    # from 512 blocks of 64 sites on, up to twelve fields share a workgroup; one field alone is the kernel above
+    L = (9, 9, 13, 32)
+    print(f"fields in turn L={L} nrhs={nrhs} donly={donly}", flush=True)
+    lat = lmx.Lattice(L, ANTI)
+    Ug = lat.gauge_from_numpy(gen.links(L, "haar", 45))
+    A = lmx.WilsonDiracOperator4D_Donly(Ug) if donly else lmx.WilsonDiracOperator4D(Ug, 0.117)
+    psi = lat.spinor(nrhs)
+    lmx.randomize_gaussian_matrix_(psi, [lmx.RNGStreamKey(46 + r) for r in range(nrhs)])
+    one, y, z = lat.spinor(), lat.spinor(nrhs), lat.spinor()
+    p32 = psi.data.to(torch.float32)
+    y32, z32 = lmx.spinor_f32(lat, nrhs), lmx.spinor_f32(lat, 1)
+    lmx.mul_(y, A, psi)
+    lmx.mul_f32_(y32, A, p32)
+    for r in range(nrhs):
+        one.data.copy_(psi.data[r:r + 1])
+        lmx.mul_(z, A, one)
+        assert torch.equal(y.data[r], z.data[0])
+        lmx.mul_f32_(z32, A, p32[r:r + 1].contiguous())
+        assert torch.equal(y32[r], z32[0])
+
+
 @pytest.mark.parametrize("L", [(3, 5, 3, 3), (8, 8, 9, 4), (13, 13, 13, 3)])
 @pytest.mark.parametrize("dagger", [False, True])
 def test_clover_three_fields(gpu, L, dagger):
