@@ -163,6 +163,11 @@ inline bool rhsloop_ok(const lmx_context* ctx) {
 constexpr int kLdsStage = 1 << 29;
 // Whether a launch can take it: the RHS-loop conditions.
 inline bool lds_ok(const lmx_context* ctx) { return rhsloop_ok(ctx); }
+// t-slices per workgroup of that shape for n fields: four where they divide
+// the lattice and leave two workgroups per CU, else as few as fill the chip (0).
+inline int lds_slices(const lmx_context* ctx, int n) {
+    return ctx->g.L[3] % 4 == 0 && (long)ctx->V * n / 1024 >= 512 ? 4 : 0;
+}
 struct LoArgs {
     int link_prec, spinor_prec;
     const void* links;
@@ -205,8 +210,10 @@ struct LoArgs {
 };
 int launch_wilson_lo(lmx_context* ctx, const LoArgs& a);
 // The FP32 apply without an epilogue by the eight-wavefront kernel, and whether it is the faster one.
+bool lds_f32(const lmx_context* ctx, int nrhs, bool clover);
 bool hops_f32(const lmx_context* ctx, int nrhs, bool clover);
 int launch_hops_f32(lmx_context* ctx, const LoArgs& a);
+int launch_lds_f32(lmx_context* ctx, const LoArgs& a);
 
 int launch_clover_build_f64(lmx_context* ctx, const double2* U, double2* clover);
 int launch_clover_export(lmx_context* ctx, const double2* clover, double2* F_out);

@@ -599,7 +599,7 @@ static int default_rhs_block(lmx_wilson* op, int prec, int nrhs) {
         // work item, h16 clover 497 / 944; 32^4 x 12: h16 1499 / 1824, f32
         // 3048 / 3584), else as few as fill the chip (16^3 x 32 x 2 f32 78 / 116);
         // one z-range, so that no z-halo crosses XCDs
-        const bool four = c->g.L[3] % 4 == 0 && n / 1024 >= 512;
+        const bool four = lds_slices(c, per) == 4;
         // too little work to repay the staging in 16 bits: 16^3 x 32 x 1 33 / 35
         if (!four && prec == LMX_H16) return (1 << 20) | (per << 4) | 1;
         return kLdsStage | (1 << 20) | ((four ? 4 : 0) << 12) | (per << 4) | 1;

@@ -115,8 +115,10 @@ int launch_wilson_lo(lmx_context* ctx, const LoArgs& a) {
     if (ctx->V == 0 || a.nrhs == 0) return LMX_OK;
     const bool cl = a.clover != nullptr;
     const int V = (int)ctx->V;
-    if (a.link_prec == LMX_F32 && a.spinor_prec == LMX_F32 && a.epi == EPI_NONE && hops_f32(ctx, a.nrhs, cl))
-        return launch_hops_f32(ctx, a);
+    if (a.link_prec == LMX_F32 && a.spinor_prec == LMX_F32 && a.epi == EPI_NONE) {
+        if (lds_f32(ctx, a.nrhs, cl)) return launch_lds_f32(ctx, a);
+        if (hops_f32(ctx, a.nrhs, cl)) return launch_hops_f32(ctx, a);
+    }
     if (a.link_prec == LMX_F32 && a.spinor_prec == LMX_F32)
         return launch_lo_sp<SpF32In, SpF32Out>(ctx, a, LinkF32{(const float2*)a.links, V},
                                                F32Clover{(const float2*)a.clover}, cl);

@@ -1,4 +1,5 @@
-// wilson_hops.hip -- the eight-wavefront stencil's FP64 and FP32 launches.
+// wilson_hops.hip -- the eight-wavefront stencil's FP64 and FP32 launches, and
+// the LDS-staged stencil's on plain FP32 fields.
 #include "wilson_hops.h"
 
 namespace lmx {
@@ -45,19 +46,25 @@ bool hops_f64(const lmx_context* ctx, int nrhs, bool clover) {
     return st.tl < 8 || st.fill < 0.8 || (nrhs == 1 && st.wgs > 256);
 }
 
+// The LDS-staged kernel (streaming lattices) where it has work enough.
+bool lds_f32(const lmx_context* ctx, int nrhs, bool clover) {
+    if (!lds_ok(ctx)) return false;
+    const int64_t n = ctx->V * nrhs;
+    // clover, LDS-staged / eight wavefronts: 24^3 x 48 110 / 111, x 12 820 / 1031,
+    // 32^4 163 / 195, x 4 456 / 599, 16^3 x 32 x 4 58 / 61, but 32x16x24x36 68 / 60,
+    // 16^4 x 4 34 / 33
+    if (clover) return n >= 500000;
+    // 32^4 116 / 150, x 12 1063 / 1158, 24^3 x 48 x 2 136 / 151, x 4 252 / 256, but
+    // 24^3 x 48 69 / 63, 32x16x24x36 x 2 82 / 79; on a small lattice many fields
+    // share the links there: 16^3 x 32 x 12 113 / 108, 24^3 x 48 x 12 700 / 675
+    return n >= 1000000 && (nrhs <= 4 || ctx->V >= 1000000);
+}
+
+// Else the eight wavefronts, but for clover fields where they do not share the
+// links and the lattice does not stream: k_site at 20^3 x 40 x 4 159 against
+// 171, but 27x29x31x35 x 12 1546 against 1460.
 bool hops_f32(const lmx_context* ctx, int nrhs, bool clover) {
-    const Geom& g = ctx->g;
-    const bool streams = !g.general && g.phase_one[0] && g.phase_one[1] && g.phase_one[2];
-    const StreamUse st = streams ? stream_use(ctx, nrhs, 512) : StreamUse{0, 0, 0.0};
-    // one field: 32^4 151 / 145, clover 200 / 189, but 24^3 x 48 63 / 79, clover
-    // 113 / 129, 40^3 x 80 682 / 718, clover 908 / 920
-    if (nrhs == 1) return st.tl < 8 || st.fill < 0.8 || st.wgs > 512;
-    // several share the links: 24^3 x 48 x 4 262 / 341, 32^4 x 12 1165 / 1546
-    if (!clover) return true;
-    // clover fields do not: 16^4 x 4 32 / 34, 24^3 x 48 x 4 371 / 417, 27x29x31x35
-    // x 12 1460 / 1546, but 16^3 x 32 x 12 195 / 176, 20^3 x 40 x 4 171 / 165,
-    // 32^4 x 4 612 / 589
-    return ctx->V * nrhs <= 550000 || (ctx->V >= 500000 && st.fill < 0.99);
+    return nrhs == 1 || !clover || lds_ok(ctx) || ctx->V * nrhs <= 550000 || ctx->V >= 500000;
 }
 
 int launch_hops_f64(lmx_context* ctx, double2* out, const double2* in, const double2* U, const double2* clover,
@@ -74,6 +81,51 @@ int launch_hops_f64(lmx_context* ctx, double2* out, const double2* in, const dou
                                                                           flags, clover != nullptr, epi);
     return launch_hops<SpF64In, LinkF64, SpF64Out, F64Clover, EPI_NONE>(ctx, o, i, l, F, i, kappa, ccoef, nrhs, rhs_per_block(ctx, nrhs), flags,
                                                                        clover != nullptr, epi);
+}
+
+// D or D^dagger of FP32 fields, up to twelve in a launch.
+int launch_lds_f32(lmx_context* ctx, const LoArgs& a) {
+    const int V = (int)ctx->V;
+    const Geom& gg = ctx->g;
+    const bool rows = gg.L[0] <= 256 && 256 % gg.L[0] == 0 && gg.L[1] % (256 / gg.L[0]) == 0;
+    const bool dag = (a.flags & LMX_DAGGER) != 0, donly = (a.flags & LMX_DONLY) != 0, clover = a.clover != nullptr;
+    const LinkF32 U{(const float2*)a.links, V};
+    const F32Clover F{(const float2*)a.clover};
+    const double ccoef = (-a.kappa) * a.csw;
+    for (int r0 = 0; r0 < a.nrhs; r0 += 12) {
+        const int n = std::min(12, a.nrhs - r0);
+        const Shape sh = pick_shape(ctx, n, 512, lds_slices(ctx, n), 1);
+        const int nb = (int)(ctx->V / 256 / sh.TL) * n;
+        const SpF32Out o = SpF32Out::at(a.out, nullptr, V, r0);
+        const SpF32In i = SpF32In::at(a.in, nullptr, V, r0);
+        const EpiArgs epi{nullptr, 0, const_cast<CGState*>(a.st), a.gate};
+#define LMX_LDS_ONE(FPM, MODE, ROWS)                                                                                      \
+    hipLaunchKernelGGL((k_lds<SpF32In, LinkF32, SpF32Out, F32Clover, SpF32In, NoEx, FPM, MODE, EPI_NONE, ROWS>), dim3(nb), \
+                       dim3(256), 0, ctx->stream, o, i, U, F, i, NoEx{}, gg, a.kappa, ccoef, n, sh.TL, sh.ZS, epi)
+#define LMX_LDS_GO(FPM, MODE)               \
+    do {                                    \
+        if (rows)                           \
+            LMX_LDS_ONE(FPM, MODE, true);   \
+        else                                \
+            LMX_LDS_ONE(FPM, MODE, false);  \
+    } while (0)
+        if (donly && dag)
+            LMX_LDS_GO(1, MODE_DONLY);
+        else if (donly)
+            LMX_LDS_GO(-1, MODE_DONLY);
+        else if (dag && clover)
+            LMX_LDS_GO(1, MODE_CLOVER);
+        else if (dag)
+            LMX_LDS_GO(1, MODE_WILSON);
+        else if (clover)
+            LMX_LDS_GO(-1, MODE_CLOVER);
+        else
+            LMX_LDS_GO(-1, MODE_WILSON);
+#undef LMX_LDS_GO
+#undef LMX_LDS_ONE
+        LMX_HIP(hipGetLastError());
+    }
+    return LMX_OK;
 }
 
 int launch_hops_f32(lmx_context* ctx, const LoArgs& a) {

@@ -1378,11 +1378,23 @@ int launch_lo_nr(lmx_context* ctx, const LoArgs& a, Lk U, Cl F, bool clover) {
             LMX_TRY((dispatch<In, Lk, Out, Cl, In, TpEx<In, Out>, NR, EPI_TP, false, false>(
                 ctx, o, i, U, F, i, ex, a.kappa, ccoef, ngroups, n, a.flags, clover, epi, 512, tl, zs)));
         } else if (a.epi == EPI_NONE) {
-            // the single-precision user apply (FP32 spinors and links) also
-            // serves the hopping-only operator
-            constexpr bool kDonly = std::is_same<In, SpF32In>::value && std::is_same<Lk, LinkF32>::value && NR == 1;
-            LMX_TRY((dispatch<In, Lk, Out, Cl, In, NoEx, NR, EPI_NONE, false, kDonly>(
-                ctx, o, i, U, F, i, none, a.kappa, ccoef, ngroups, n, a.flags, clover, epi, 512, tl, zs)));
+            // the single-precision user apply (FP32 spinors and links) where
+            // the lattice does not stream: several clover fields (hops_f32)
+            if constexpr (std::is_same<In, SpF32In>::value && std::is_same<Lk, LinkF32>::value && NR == 1) {
+                LMX_CHECK(clover && (a.flags & LMX_DONLY) == 0, LMX_ERR_UNSUPPORTED, "no per-site FP32 Wilson stencil");
+                if ((a.flags & LMX_DAGGER) != 0)
+                    hipLaunchKernelGGL((k_site<In, Lk, Out, Cl, In, NoEx, 1, MODE_CLOVER, 1, EPI_NONE, true>),
+                                       dim3(nblocks(ctx->V) * n), dim3(256), 0, ctx->stream, o, i, U, F, i, none, ctx->g,
+                                       a.kappa, ccoef, n, n, epi);
+                else
+                    hipLaunchKernelGGL((k_site<In, Lk, Out, Cl, In, NoEx, -1, MODE_CLOVER, 1, EPI_NONE, true>),
+                                       dim3(nblocks(ctx->V) * n), dim3(256), 0, ctx->stream, o, i, U, F, i, none, ctx->g,
+                                       a.kappa, ccoef, n, n, epi);
+                LMX_HIP(hipGetLastError());
+            } else {
+                set_error("plain low-precision stencils are built for FP32 fields and links");
+                return LMX_ERR_UNSUPPORTED;
+            }
         } else {
             set_error("fused epilogue %d is not built for low-precision spinors", a.epi);
             return LMX_ERR_UNSUPPORTED;

@@ -64,6 +64,31 @@ def test_fields_that_take_turns_in_a_workgroup(gpu, nrhs, donly):
         assert torch.equal(y32[r], z32[0])
 
 
+@pytest.mark.parametrize("L,csw,donly,nrhs", [
+    ((16, 16, 16, 16), 1.0, False, 13),   # whole rows of a z-plane; a second launch of one field
+    ((24, 24, 24, 13), 1.0, False, 3),    # blocks that cut rows; one slice a workgroup
+    ((24, 24, 24, 20), 0.0, False, 4),    # four slices a workgroup
+    ((32, 16, 16, 32), 0.0, False, 4),
+    ((32, 16, 16, 32), 0.0, True, 4),
+])
+@pytest.mark.parametrize("dagger", [False, True])
+def test_fp32_fields_staged_in_lds(gpu, L, csw, donly, nrhs, dagger):
+    # enough FP32 fields on a streaming lattice take the LDS-staged stencil; one alone is the kernel above
+    print(f"FP32 LDS L={L} csw={csw} donly={donly} nrhs={nrhs} dagger={dagger}", flush=True)
+    lat = lmx.Lattice(L, ANTI)
+    Ug = lat.gauge_from_numpy(gen.links(L, "weak", 47, eps=0.15))
+    D = lmx.WilsonDiracOperator4D_Donly(Ug) if donly else lmx.WilsonDiracOperator4D(Ug, 0.117, csw)
+    A = lmx.adjoint(D) if dagger else D
+    psi = lat.spinor(nrhs)
+    lmx.randomize_gaussian_matrix_(psi, [lmx.RNGStreamKey(48 + r) for r in range(nrhs)])
+    p32 = psi.data.to(torch.float32)
+    y, z = lmx.spinor_f32(lat, nrhs), lmx.spinor_f32(lat, 1)
+    lmx.mul_f32_(y, A, p32)
+    for r in range(nrhs):
+        lmx.mul_f32_(z, A, p32[r:r + 1].contiguous())
+        assert torch.equal(y[r], z[0])
+
+
 @pytest.mark.parametrize("L", [(3, 5, 3, 3), (8, 8, 9, 4), (13, 13, 13, 3)])
 @pytest.mark.parametrize("dagger", [False, True])
 def test_clover_three_fields(gpu, L, dagger):
