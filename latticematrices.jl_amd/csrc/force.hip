@@ -16,26 +16,24 @@ namespace lmx {
 
 template <int MU>
 __device__ __forceinline__ void pullback_mu(double2* __restrict__ dU, const double2* __restrict__ dres,
-                                            const double2* __restrict__ psi, const Geom& g, int s, const int x[4],
-                                            const cx<double> d0[12], const cx<double> p0[12], double coefficient) {
+                                            const double2* __restrict__ psi, const Geom& g, int s, double coefficient) {
+    int x[4];
+    site_coords(s, g, x);
     bool w;
     const int sp = nbr_fwd(s, x, MU, g, w);
-    cx<double> d1[12], p1[12];
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-        double2 a = dres[(long)k * g.V + sp], b = psi[(long)k * g.V + sp];
-        d1[k] = mk<double>(a.x, a.y);
-        p1[k] = mk<double>(b.x, b.y);
-    }
-    if (w && !g.phase_one[MU]) {
-        phase_spinor(d1, g.ph_re[MU], g.ph_im[MU]);
-        phase_spinor(p1, g.ph_re[MU], g.ph_im[MU]);
-    }
+    const bool ph = w && !g.phase_one[MU];
     cx<double> plus_psi[6], minus_dres[6], dplus[6], mpsi[6];
-    half_project<-1, MU>(p1, plus_psi);
-    half_project<1, MU>(d1, minus_dres);
-    half_project<-1, MU>(d0, dplus);
-    half_project<1, MU>(p0, mpsi);
+    cx<double> z[12];
+    ld_comps(psi, g.V, sp, z);
+    if (ph) phase_spinor(z, g.ph_re[MU], g.ph_im[MU]);
+    half_project<-1, MU>(z, plus_psi);
+    ld_comps(dres, g.V, sp, z);
+    if (ph) phase_spinor(z, g.ph_re[MU], g.ph_im[MU]);
+    half_project<1, MU>(z, minus_dres);
+    ld_comps(dres, g.V, s, z);
+    half_project<-1, MU>(z, dplus);
+    ld_comps(psi, g.V, s, z);
+    half_project<1, MU>(z, mpsi);
 #pragma unroll
     for (int row = 0; row < 3; ++row) {
 #pragma unroll
@@ -44,7 +42,7 @@ __device__ __forceinline__ void pullback_mu(double2* __restrict__ dU, const doub
             v = cadd(v, cmul(dplus[2 * row + 1], cconj(plus_psi[2 * col + 1])));
             v = cadd(v, cmul(mpsi[2 * row], cconj(minus_dres[2 * col])));
             v = cadd(v, cmul(mpsi[2 * row + 1], cconj(minus_dres[2 * col + 1])));
-            const long i = (long)(MU * 9 + row * 3 + col) * g.V + s;
+            const size_t i = (size_t)(MU * 9 + row * 3 + col) * g.V + s;
             double2 o = dU[i];
             cx<double> nv = cadd(mk<double>(o.x, o.y), rmul(coefficient, v));
             dU[i] = make_double2(nv.re, nv.im);
@@ -52,23 +50,31 @@ __device__ __forceinline__ void pullback_mu(double2* __restrict__ dU, const doub
     }
 }
 
-__global__ void __launch_bounds__(256) k_pullback(double2* __restrict__ dU, const double2* __restrict__ dres,
-                                                  const double2* __restrict__ psi, Geom g, double coefficient) {
-    const int s = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
-    if (s >= g.V) return;
-    int x[4];
-    site_coords(s, g, x);
-    cx<double> d0[12], p0[12];
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-        double2 a = dres[(long)k * g.V + s], b = psi[(long)k * g.V + s];
-        d0[k] = mk<double>(a.x, a.y);
-        p0[k] = mk<double>(b.x, b.y);
+// A wavefront of a workgroup takes one direction of the workgroup's 64 sites,
+// blocks in the stencil's slab order: 126 registers and four wavefronts per
+// SIMD, where one work item for all four directions held two own spinors
+// besides two neighbours' (240, two).  Bound by its 384 B read and 1152 B read
+// and written per site: 16^3 x 32 49 us (4.1 TB/s) against 55.
+__global__ void __launch_bounds__(256, 3) k_pullback(double2* __restrict__ dU, const double2* __restrict__ dres,
+                                                     const double2* __restrict__ psi, Geom g, double coefficient,
+                                                     int slab) {
+    int s0, end;
+    slab_block(xcd_block(blockIdx.x, gridDim.x), slab, g, s0, end);
+    const int s = s0 + (threadIdx.x & 63);
+    if (s >= end) return;
+    switch (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {
+    case 0:
+        pullback_mu<0>(dU, dres, psi, g, s, coefficient);
+        break;
+    case 1:
+        pullback_mu<1>(dU, dres, psi, g, s, coefficient);
+        break;
+    case 2:
+        pullback_mu<2>(dU, dres, psi, g, s, coefficient);
+        break;
+    default:
+        pullback_mu<3>(dU, dres, psi, g, s, coefficient);
     }
-    pullback_mu<0>(dU, dres, psi, g, s, x, d0, p0, coefficient);
-    pullback_mu<1>(dU, dres, psi, g, s, x, d0, p0, coefficient);
-    pullback_mu<2>(dU, dres, psi, g, s, x, d0, p0, coefficient);
-    pullback_mu<3>(dU, dres, psi, g, s, x, d0, p0, coefficient);
 }
 
 // F = TA(U G^dagger): M[i][j] = muladdmulti over k of U[i][k] conj(G[j][k]),
@@ -113,8 +119,9 @@ __global__ void __launch_bounds__(256) k_ta_project(double2* __restrict__ F, con
 
 int launch_pullback_f64(lmx_context* ctx, double2* dU, const double2* dres, const double2* psi, double coefficient) {
     if (ctx->V == 0) return LMX_OK;
-    hipLaunchKernelGGL(k_pullback, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, dU, dres, psi, ctx->g,
-                       coefficient);
+    const SlabOrder so = slab_order(ctx->g, false);
+    hipLaunchKernelGGL(k_pullback, dim3((unsigned)so.blocks), dim3(256), 0, ctx->stream, dU, dres, psi, ctx->g,
+                       coefficient, so.slab);
     LMX_HIP(hipGetLastError());
     return LMX_OK;
 }
@@ -393,7 +400,7 @@ __device__ __forceinline__ int step_site(const Geom& g, int s, const int x[4], i
 // 4.8 cycles an instruction that two wavefronts per SIMD reach.  A wavefront
 // alone issues an FP64 instruction every six cycles, so the terms come in an
 // order that keeps few matrices at once, two wait in LDS and one link is read
-// twice: 248 registers and two wavefronts per SIMD, 284 us against 324 with
+// twice: 256 registers and two wavefronts per SIMD, 284 us against 324 with
 // everything in 460 registers at one.  (More links read again and less parked
 // loses it: 320 us at 1.4 times the loads.)  Blocks in the stencil's slab order.
 __global__ void __launch_bounds__(256, 2) k_clover_links_pullback(double2* dU,
