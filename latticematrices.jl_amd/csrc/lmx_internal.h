@@ -164,9 +164,16 @@ constexpr int kLdsStage = 1 << 29;
 // Whether a launch can take it: the RHS-loop conditions.
 inline bool lds_ok(const lmx_context* ctx) { return rhsloop_ok(ctx); }
 // t-slices per workgroup of that shape for n fields: four where they divide
-// the lattice and leave two workgroups per CU, else as few as fill the chip (0).
+// the lattice and leave two workgroups per CU, six where they leave enough to
+// fill the CUs several times over (D + D^dagger, us, six / four slices:
+// 24^3 x 48 x 12 f16 1728 / 1807, f32 1962 / 2018, h16 1021 / 1028, x 4 f32
+// 729 / 747, 32^3 x 48 x 4 f16 1362 / 1435, h16 811 / 849, but with 1536
+// workgroups 16^3 x 48 x 12 h16 306 / 295), else as few as fill the chip (0).
 inline int lds_slices(const lmx_context* ctx, int n) {
-    return ctx->g.L[3] % 4 == 0 && (long)ctx->V * n / 1024 >= 512 ? 4 : 0;
+    const int Lt = ctx->g.L[3];
+    const int64_t blocks = ctx->V / 256 * n;
+    if (Lt % 6 == 0 && blocks / 6 >= 1700) return 6;
+    return Lt % 4 == 0 && blocks / 4 >= 512 ? 4 : 0;
 }
 struct LoArgs {
     int link_prec, spinor_prec;

@@ -594,15 +594,15 @@ static int default_rhs_block(lmx_wilson* op, int prec, int nrhs) {
     const long n = (long)c->V * per;
     const bool clover = op->csw != 0.0;
     if (lds_ok(c)) {
-        // LDS-staged, four t-slices per workgroup where that leaves two
-        // workgroups per CU (24^3 x 48 x 4: f16 615 against 793 streaming two per
+        // LDS-staged, four or six t-slices per workgroup where there is work
+        // enough (lds_slices; 24^3 x 48 x 4: f16 629 against 793 streaming two per
         // work item, h16 clover 497 / 944; 32^4 x 12: h16 1499 / 1824, f32
         // 3048 / 3584), else as few as fill the chip (16^3 x 32 x 2 f32 78 / 116);
         // one z-range, so that no z-halo crosses XCDs
-        const bool four = lds_slices(c, per) == 4;
+        const int tl = lds_slices(c, per);
         // too little work to repay the staging in 16 bits: 16^3 x 32 x 1 33 / 35
-        if (!four && prec == LMX_H16) return (1 << 20) | (per << 4) | 1;
-        return kLdsStage | (1 << 20) | ((four ? 4 : 0) << 12) | (per << 4) | 1;
+        if (tl == 0 && prec == LMX_H16) return (1 << 20) | (per << 4) | 1;
+        return kLdsStage | (1 << 20) | (tl << 12) | (per << 4) | 1;
     }
     // no streaming there: two per work item share the links where there is
     // work enough (27x29x31x35 x 4 f32 1210 against 1335 one by one, but

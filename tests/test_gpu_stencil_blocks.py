@@ -68,6 +68,7 @@ def test_fields_that_take_turns_in_a_workgroup(gpu, nrhs, donly):
     ((16, 16, 16, 16), 1.0, False, 13),   # whole rows of a z-plane; a second launch of one field
     ((24, 24, 24, 13), 1.0, False, 3),    # blocks that cut rows; one slice a workgroup
     ((24, 24, 24, 20), 0.0, False, 4),    # four slices a workgroup
+    ((24, 24, 24, 18), 1.0, False, 12),   # six slices a workgroup
     ((32, 16, 16, 32), 0.0, False, 4),
     ((32, 16, 16, 32), 0.0, True, 4),
 ])
