@@ -272,11 +272,16 @@ __global__ void __launch_bounds__(256) k_cg_update_xp(typename Vec2<R>::T* __res
 // kernel reads the one and its block 0 writes the other, so no block reads
 // what another writes.
 // ---------------------------------------------------------------------------
-// The sum of n64 partials of 64 sites each, in all of the block's 256 threads.
-__device__ __forceinline__ double sum_wave_partials(const double* w, int n64, double* lds4) {
+// The sum of n64 partials of 64 sites each, in all of the block's 256 threads:
+// a thread's own share (loaded before the state is looked at, so that the two
+// waits are one), and the block's.
+__device__ __forceinline__ double own_wave_partials(const double* w, int n64) {
     const int nb = (n64 + 3) / 4;
     double acc = 0.0;
     for (int b = threadIdx.x; b < nb; b += kRedBlock) acc = acc + wave_quad(w, b, n64);
+    return acc;
+}
+__device__ __forceinline__ double sum_wave_partials(double acc, double* lds4) {
     acc = wave_halve(acc);
     if ((threadIdx.x & 63) == 0) lds4[threadIdx.x >> 6] = acc;
     __syncthreads();
@@ -300,8 +305,10 @@ __global__ void __launch_bounds__(256) k_cg_small_r(double2* __restrict__ r, con
             av[k] = Ap[(size_t)(3 * grp + k) * V + s];
         }
     }
+    const double own = own_wave_partials(pap, n64);
+    asm volatile("" ::: "memory");
     const bool was_done = in->done != 0;
-    const double pAp = was_done ? 0.0 : sum_wave_partials(pap, n64, lds4);
+    const double pAp = was_done ? 0.0 : sum_wave_partials(own, lds4);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *out = *in;
         if (!was_done) finalize_scalar(FIN_PAP, out, pAp, 0.0, nullptr);
@@ -351,8 +358,10 @@ __global__ void __launch_bounds__(256) k_cg_small_xp(double2* __restrict__ x, co
             rv[k] = r[i];
         }
     }
+    const double own = own_wave_partials(rr, n64);
+    asm volatile("" ::: "memory");
     const bool was_done = in->done != 0;
-    const double rr_new = was_done ? 0.0 : sum_wave_partials(rr, n64, lds4);
+    const double rr_new = was_done ? 0.0 : sum_wave_partials(own, lds4);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         *out = *in;
         if (!was_done) finalize_scalar(FIN_RRNEW, out, rr_new, 0.0, nullptr);

@@ -966,10 +966,13 @@ __device__ __forceinline__ double block_tree(double v, double* lds4) {
 // Second stage (its own one-block launch, after the producing kernel has
 // finished, so every partial is visible without a per-block fence): 256
 // lanes sum the block partials with stride 256 in order, then the block tree.
-__device__ __forceinline__ double finish_partials(const double* partials, int nb, double* lds4) {
+__device__ __forceinline__ double strided_sum(const double* partials, int nb) {
     double acc = 0.0;
     for (int b = threadIdx.x; b < nb; b += kRedBlock) acc = acc + partials[b];
-    return block_tree(acc, lds4);
+    return acc;
+}
+__device__ __forceinline__ double finish_partials(const double* partials, int nb, double* lds4) {
+    return block_tree(strided_sum(partials, nb), lds4);
 }
 
 // The partial of 256-site block b from the sums w of 64 consecutive sites (n64

@@ -139,44 +139,34 @@ enum { MX_INIT = 0, MX_PAP = 1, MX_RR = 2, MX_TRUE = 3 };
 // An RHS stops with LMX_CG_MAXITER when its iteration count reaches maxiter
 // (cg!, src/LinearAlgebras/cg.jl:105,135-136), in the iteration's own
 // finalize, so a graph replay that runs past maxiter leaves it untouched.
+//
+// The iterations after an update request do nothing: MX_PAP keeps what go was
+// as the iteration began, since MX_RR itself may clear it.  The last RHS of an
+// update (MX_TRUE) lets the next group run.
+// A launch is little but latency: the gates, the state and the partials are
+// loaded together, before any of them is looked at (one 16-bit field at
+// 8^3 x 16 5745 -> 5600 us a solve).
 template <int KIND>
-__device__ __forceinline__ void mx_finish(const double* __restrict__ partials, int nb, MixRhs* rhs, MixBatch* batch,
-                                          double rtol, double atol, int flag) {
-    const int i = blockIdx.x;
-    MixRhs* st = rhs + i;
-    const bool final_fold = KIND == MX_TRUE && flag && st->done && st->fold;
-    if (st->done && !final_fold) return;
-    if (threadIdx.x == 0) {
-        if (KIND == MX_RR) {
-            if (flag < kXBatch - 1) {
-                st->alpha_q[flag] = st->alpha;
-                st->pmask |= 1 << flag;
-            } else {
-                st->pmask = 0;  // the group's last iteration applied them
-            }
-        }
-        if (KIND == MX_TRUE) st->pmask = 0;  // k_mx_accum folded the deferred terms
-    }
-    __shared__ double lds4[4];
-    const double A = finish_partials(partials + (size_t)(2 * i) * nb, nb, lds4);
-    const double B = (KIND == MX_INIT) ? finish_partials(partials + (size_t)(2 * i + 1) * nb, nb, lds4) : 0.0;
-    if (threadIdx.x != 0) return;
+__device__ __forceinline__ void mx_finish(MixRhs* st, const MixRhs& z, MixBatch* batch, const MixBatch& q, double A,
+                                          double B, double rtol, double atol, int flag) {
+    const bool final_fold = KIND == MX_TRUE && flag && z.done && z.fold;
     if (KIND == MX_INIT) {  // A = |r|^2, B = |b|^2
-        st->bnorm = sqrt(B);
-        st->tol = fmax(atol, rtol * st->bnorm);
+        const double bnorm = sqrt(B), tol = fmax(atol, rtol * bnorm), rtrue = sqrt(A);
+        st->bnorm = bnorm;
+        st->tol = tol;
         st->rr = A;
         st->rr_prev = A;
-        st->rtrue = sqrt(A);
-        st->rref = st->rtrue;
+        st->rtrue = rtrue;
+        st->rref = rtrue;
         st->since = 0;
         st->iterations = 0;
         st->updates = 0;
         st->beta = 0.0;
         if (!isfinite(A) || !isfinite(B))
             retire(st, batch, LMX_CG_BREAKDOWN, 0, 0);
-        else if (st->rtrue <= st->tol)
+        else if (rtrue <= tol)
             retire(st, batch, LMX_CG_CONVERGED, 1, 0);
-        else if (batch->maxiter <= 0)
+        else if (q.maxiter <= 0)
             retire(st, batch, LMX_CG_MAXITER, 0, 0);
     } else if (KIND == MX_PAP) {  // A = p.Ap = |D p|^2
         st->pAp = A;
@@ -185,67 +175,81 @@ __device__ __forceinline__ void mx_finish(const double* __restrict__ partials, i
         else if (A <= 0.0)
             retire(st, batch, LMX_CG_NONPOSITIVE_CURVATURE, 0, 1);
         else
-            st->alpha = st->rr / A;
+            st->alpha = z.rr / A;
     } else if (KIND == MX_RR) {  // A = |r_inner|^2
-        st->iterations += 1;
-        st->since += 1;
+        if (flag < kXBatch - 1) {
+            st->alpha_q[flag] = z.alpha;
+            st->pmask = z.pmask | 1 << flag;
+        } else {
+            st->pmask = 0;  // the group's last iteration applied them
+        }
+        const int iterations = z.iterations + 1, since = z.since + 1;
+        st->iterations = iterations;
+        st->since = since;
         if (!isfinite(A)) {
             retire(st, batch, LMX_CG_BREAKDOWN, 0, 1);
             return;
         }
-        const double rn = sqrt(A);
-        st->rref = fmax(st->rref, rn);
-        st->rr_prev = st->rr;
-        st->beta = A / st->rr;
+        const double rn = sqrt(A), rref = fmax(z.rref, rn);
+        st->rref = rref;
+        st->rr_prev = z.rr;
+        st->beta = A / z.rr;
         st->rr = A;
-        if (st->iterations >= batch->maxiter) {
+        if (iterations >= q.maxiter) {
             // the final pass folds x_inner in; a true residual within the
             // tolerance there still counts as converged
             retire(st, batch, LMX_CG_MAXITER, 0, 1);
             return;
         }
-        if (rn < batch->delta * st->rref || st->since >= batch->rmax || rn <= st->tol) {
+        if (rn < q.delta * rref || since >= q.rmax || rn <= z.tol) {
             atomicOr(&batch->do_update, 1);
             batch->go = 0;
         }
-    } else if (final_fold) {  // MX_TRUE on a retired RHS: A = |b - A x|^2 after its fold
-        st->rtrue = sqrt(A);
-        st->updates += 1;
-        st->fold = 0;
-        if (st->reason == LMX_CG_MAXITER && isfinite(A) && st->rtrue <= st->tol) {
-            st->reason = LMX_CG_CONVERGED;
-            st->converged = 1;
-        }
     } else {  // MX_TRUE: A = |b - A x|^2 in FP64
-        st->rtrue = sqrt(A);
-        st->updates += 1;
-        if (!isfinite(A)) {
+        const double rtrue = sqrt(A);
+        st->pmask = 0;  // k_mx_accum folded the deferred terms
+        st->rtrue = rtrue;
+        st->updates = z.updates + 1;
+        if (final_fold) {  // on a retired RHS, after its fold
+            st->fold = 0;
+            if (z.reason == LMX_CG_MAXITER && isfinite(A) && rtrue <= z.tol) {
+                st->reason = LMX_CG_CONVERGED;
+                st->converged = 1;
+            }
+        } else if (!isfinite(A)) {
             retire(st, batch, LMX_CG_BREAKDOWN, 0, 0);
-        } else if (st->rtrue <= st->tol) {
+        } else if (rtrue <= z.tol) {
             retire(st, batch, LMX_CG_CONVERGED, 1, 0);
         } else {
-            st->beta = A / st->rr_prev;
+            st->beta = A / z.rr_prev;
             st->rr = A;
-            st->rref = st->rtrue;
+            st->rref = rtrue;
             st->since = 0;
         }
     }
 }
 
-// The iterations after an update request do nothing: MX_PAP keeps what go was
-// as the iteration began, since MX_RR itself may clear it.  The last RHS of an
-// update (MX_TRUE) lets the next group run.
 template <int KIND>
 __global__ void __launch_bounds__(256) k_mx_fin(const double* __restrict__ partials, int nb, MixRhs* rhs,
                                                 MixBatch* batch, double rtol, double atol, int flag) {
+    __shared__ double lds4[4];
+    const int i = blockIdx.x;
+    const MixRhs z = rhs[i];
+    const MixBatch q = *batch;
+    const double a = strided_sum(partials + (size_t)(2 * i) * nb, nb);
+    const double b = KIND == MX_INIT ? strided_sum(partials + (size_t)(2 * i + 1) * nb, nb) : 0.0;
+    asm volatile("" ::: "memory");  // no load sinks below the gates
     if (KIND == MX_PAP) {
-        const int go = batch->go;
-        if (blockIdx.x == 0 && threadIdx.x == 0) batch->live = go;
-        if (!go) return;
+        if (i == 0 && threadIdx.x == 0) batch->live = q.go;
+        if (!q.go) return;
     }
-    if (KIND == MX_RR && !batch->live) return;
-    if (KIND == MX_TRUE && !flag && !batch->do_update) return;
-    mx_finish<KIND>(partials, nb, rhs, batch, rtol, atol, flag);
+    if (KIND == MX_RR && !q.live) return;
+    if (KIND == MX_TRUE && !flag && !q.do_update) return;
+    if (!z.done || (KIND == MX_TRUE && flag && z.fold)) {
+        const double A = block_tree(a, lds4);
+        const double B = KIND == MX_INIT ? block_tree(b, lds4) : 0.0;
+        if (threadIdx.x == 0) mx_finish<KIND>(rhs + i, z, batch, q, A, B, rtol, atol, flag);
+    }
     if (KIND == MX_TRUE && !flag && threadIdx.x == 0) {
         __threadfence();
         if (atomicAdd(&batch->ticket, 1) == (int)gridDim.x - 1) {
