@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(256) k_convert(const double2* __restrict__ in,
 
 int launch_clover_build_f64(lmx_context* ctx, const double2* U, double2* clover) {
     if (ctx->V == 0) return LMX_OK;
-    const SlabOrder so = slab_order(ctx->g, false);
+    const SlabOrder so = slab_order(ctx->g, false, 12 * sizeof(double2));
     hipLaunchKernelGGL(k_clover_build, dim3((unsigned)so.blocks), dim3(384), 0, ctx->stream, U, clover, ctx->g, so.slab);
     LMX_HIP(hipGetLastError());
     return LMX_OK;

@@ -119,7 +119,7 @@ __global__ void __launch_bounds__(256) k_ta_project(double2* __restrict__ F, con
 
 int launch_pullback_f64(lmx_context* ctx, double2* dU, const double2* dres, const double2* psi, double coefficient) {
     if (ctx->V == 0) return LMX_OK;
-    const SlabOrder so = slab_order(ctx->g, false);
+    const SlabOrder so = slab_order(ctx->g, false, 12 * sizeof(double2));
     hipLaunchKernelGGL(k_pullback, dim3((unsigned)so.blocks), dim3(256), 0, ctx->stream, dU, dres, psi, ctx->g,
                        coefficient, so.slab);
     LMX_HIP(hipGetLastError());
@@ -516,7 +516,7 @@ int launch_clover_pullback(lmx_context* ctx, double2* dU, const double2* U, doub
     if (ctx->V == 0) return LMX_OK;
     hipLaunchKernelGGL(k_clover_cotangent, dim3(nblocks(ctx->V)), dim3(256), 0, ctx->stream, dQ, dres, psi,
                        (int)ctx->V, coefficient);
-    const SlabOrder so = slab_order(ctx->g, false);
+    const SlabOrder so = slab_order(ctx->g, false, 12 * sizeof(double2));
     hipLaunchKernelGGL(k_clover_links_pullback, dim3((unsigned)so.blocks), dim3(256), 0, ctx->stream, dU, U,
                        (const double2*)dQ, ctx->g, so.slab);
     LMX_HIP(hipGetLastError());

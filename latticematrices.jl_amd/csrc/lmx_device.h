@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 namespace lmx {
@@ -123,11 +124,21 @@ struct SlabOrder {
     int slab;
     long blocks;
 };
-// whole: blocks must not be cut by the end of a slice (else at most 1/32 of
-// the lanes idle there); slices of fewer blocks than XCDs make no slabs
-inline SlabOrder slab_order(const Geom& g, bool whole) {
+// Slices of fewer than 64 blocks take lattice order, where an XCD's share is
+// whole slices: several of those fit its L2, and in slabs of a block or two
+// nearly all of a site's neighbours lie on other XCDs (FP64 D, us, lattice /
+// slabs: 8^3 x 128 12.4 / 19.2, 8^3 x 256 21.9 / 40.4, 8x16x16x128 41 / 56,
+// 12^3 x 64 20 / 23; at 64 blocks 16^4 15.9 / 14.7, 16^3 x 64 51.1 / 47.5).
+// A slab's spinors of one slice take at most 3 MB of the XCD's 4 MB, or its
+// neighbours in t have left L2 when they are due: site_bytes for a site's
+// spinor, 256 blocks in FP64 (72^3 x 8 831 / 1002 with the eighth of 729, 64^3
+// x 24 1729 / 1823; 128 blocks lose: 48^3 x 16, 216 of them, 420 / 454).
+// whole: blocks must not be cut by the end of a slice (else at most 1/64 of
+// the lanes idle there).
+inline SlabOrder slab_order(const Geom& g, bool whole, int site_bytes) {
     const int V3 = g.stride[3], n3 = (V3 + kSlabSites - 1) / kSlabSites;
-    if (n3 >= 8 && (V3 % kSlabSites == 0 || (!whole && n3 >= 32))) return {(n3 + 7) / 8, (long)n3 * g.L[3]};
+    const int most = 3 * (1 << 20) / (kSlabSites * site_bytes);
+    if (n3 >= 64 && (V3 % kSlabSites == 0 || !whole)) return {std::min((n3 + 7) / 8, most), (long)n3 * g.L[3]};
     return {0, ((long)g.V + kSlabSites - 1) / kSlabSites};
 }
 // First site of block lb and the end of the sites it may take.

@@ -18,7 +18,7 @@
 // wavefronts per SIMD in FP64.  Here it waits for one, at 88 VGPRs and five
 // wavefronts per SIMD, at the price of 1.5 KB of LDS traffic per site and of
 // the neighbours in t read again.  To keep those in L2 the blocks are ordered
-// slab by slab: an eighth of the 3-D volume, which is one XCD's share, for
+// slab by slab (slab_order): an eighth of the 3-D volume, one XCD's share, for
 // t = 0, 1, ... (lattice order instead: 174 against 148 us at 24^3 x 48, 3400
 // against 2650 us at 48^3 x 96; tiles in y and z, nontemporal loads of links
 // and a walk over t within the workgroup were no faster).  Bound by the L2
@@ -349,7 +349,8 @@ int launch_hops(lmx_context* ctx, Out out, In in, Lk U, Cl F, In aux, double kap
                 int flags, bool clover, const EpiArgs& epi) {
     const bool dag = (flags & LMX_DAGGER) != 0, donly = (flags & LMX_DONLY) != 0;
     const Geom& g = ctx->g;
-    const SlabOrder so = slab_order(g, EPI == EPI_PAP);  // the sums of EPI_PAP need whole blocks
+    // the sums of EPI_PAP need whole blocks
+    const SlabOrder so = slab_order(g, EPI == EPI_PAP, 24 * sizeof(typename In::R));
     // clover fields one by one: a loop over them would hold the planes' entries too
     const int per = clover || EPI != EPI_NONE ? 1 : std::min(std::max(per_hint, 1), nrhs);
     const int ngroups = (nrhs + per - 1) / per;
@@ -613,7 +614,7 @@ int launch_hops_pad(lmx_context* ctx, Lk l, Cl F, bool clover, double kappa, dou
     pg.Vp = st;
     LMX_CHECK(st < (1L << 31), LMX_ERR_ARG, "padded volume too large");
     const double ccoef = (-kappa) * csw;
-    const SlabOrder so = slab_order(g, false);
+    const SlabOrder so = slab_order(g, false, 12 * sizeof(E));
     const long nb = so.blocks * nrhs;
     LMX_CHECK(nb < (1L << 31), LMX_ERR_ARG, "too many right-hand sides (%d)", nrhs);
     const bool dag = (flags & LMX_DAGGER) != 0, donly = (flags & LMX_DONLY) != 0;

@@ -25,7 +25,7 @@ static bool shape_forced(const lmx_context* ctx) { return ctx->tune_tl > 0 || ct
 // alone fill the chip (24^3 x 48, 12 FP64 fields: 1280 us against 1500 one by
 // one), one where they do not (8^3 x 16: 17 against 24).
 static int rhs_per_block(const lmx_context* ctx, int nrhs) {
-    return slab_order(ctx->g, false).blocks >= 512 ? std::min(nrhs, 12) : 1;
+    return slab_order(ctx->g, false, 12 * sizeof(double2)).blocks >= 512 ? std::min(nrhs, 12) : 1;
 }
 
 // Measured, us, this kernel / the other.
