@@ -115,6 +115,8 @@ int launch_wilson_f64(lmx_context* ctx, const double2* U, const double2* clover,
 // the faster one on this lattice.  Epilogue kind 1 leaves one p.Ap sum per 64
 // consecutive sites in e.partials (for launch_finalize's `waves`).
 bool hops_f64(const lmx_context* ctx, int nrhs, bool clover);
+// The caller has named a streaming shape (LMX_STREAM_TL, LMX_STREAM_ZS).
+inline bool shape_forced(const lmx_context* ctx) { return ctx->tune_tl > 0 || ctx->tune_zs > 0; }
 int launch_hops_f64(lmx_context* ctx, double2* out, const double2* in, const double2* U, const double2* clover,
                     const double2* p, double kappa, double csw, int nrhs, int flags, const Epilogue& e);
 // FP64 D^dagger of the mixed solver's reliable update with the true residual

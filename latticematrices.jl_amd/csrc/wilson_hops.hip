@@ -18,9 +18,6 @@ static StreamUse stream_use(const lmx_context* ctx, int ngroups, int round) {
     const long wgs = ctx->V / 256 / sh.TL * ngroups;
     return {sh.TL, wgs, (double)wgs / (double)((wgs + round - 1) / round * round)};
 }
-// The caller has named a streaming shape (LMX_STREAM_TL, LMX_STREAM_ZS).
-static bool shape_forced(const lmx_context* ctx) { return ctx->tune_tl > 0 || ctx->tune_zs > 0; }
-
 // Right-hand sides per workgroup: all that share the links where the blocks
 // alone fill the chip (24^3 x 48, 12 FP64 fields: 1280 us against 1500 one by
 // one), one where they do not (8^3 x 16: 17 against 24).
@@ -28,22 +25,46 @@ static int rhs_per_block(const lmx_context* ctx, int nrhs) {
     return slab_order(ctx->g, false, 12 * sizeof(double2)).blocks >= 512 ? std::min(nrhs, 12) : 1;
 }
 
+// Slices this large (64^3, 64x64x48) leave no slab in an XCD's L2 from one
+// slice to the next without cutting it small; k_stream keeps its neighbours in
+// t in registers.
+constexpr long kLargeSlice = 150000;
+
 // Measured, us, this kernel / the other.
 bool hops_f64(const lmx_context* ctx, int nrhs, bool clover) {
     const StreamUse st = stream_use(ctx, clover ? nrhs : (nrhs + 1) / 2, 256);
     // against k_site: 18x20x22x30 42 / 80, four fields 173 / 252; clover 65 / 93, 227 / 242
     if (st.tl == 0 || ctx->g.general) return true;
     if (shape_forced(ctx)) return false;
+    const long V3 = ctx->g.stride[3];
+    const bool large = V3 >= kLargeSlice;
     // k_stream wins where its workgroups fill the 256 CUs an exact number of
-    // times and walk far.  Clover, one field per work item: 32^4 335 / 324, x 4
-    // 1055 / 981, 16^4 x 4 53 / 50, but 16^3 x 32 35 / 39, 24^3 x 48 192 / 270,
-    // 40^3 x 80 1560 / 1697, 48^3 x 96 3501 / 3866.
-    if (clover) return st.fill < 0.99 || st.tl < (nrhs >= 4 ? 4 : 8);
-    // One field: 32^3 x 16 122 / 115, 32^4 253 / 230, but 16^3 x 32 26 / 31,
-    // 24^3 x 48 146 / 198, 40^3 x 80 1185 / 1310, 48^3 x 96 2610 / 2920.
-    // Several, two of them to its work item: 32^4 x 4 798 / 684, 40^3 x 80 x 2
-    // 2270 / 1940, but 16^3 x 32 x 4 80 / 93, 24^3 x 48 x 4 456 / 598.
-    return st.tl < 8 || st.fill < 0.8 || (nrhs == 1 && st.wgs > 256);
+    // times and walk far, the sooner the larger the slices.  Clover, one field
+    // per work item: 32^4 335 / 324, x 4 1055 / 981, 16^4 x 4 53 / 50, 32^3 x 4 x 2
+    // 61 / 56, 64^3 x 4 377 / 361, x 2 640 / 586, but 16^3 x 32 35 / 39, 24^3 x 48
+    // 192 / 270, 40^3 x 80 1560 / 1697, 48^3 x 96 3501 / 3866.
+    if (clover) return st.fill < 0.99 || st.tl < (nrhs >= 4 || large || (nrhs >= 2 && V3 >= 32768) ? 4 : 8);
+    // One field: 32^3 x 16 122 / 115, 32^4 253 / 230 and 16^3 x 128 (one round of
+    // workgroups, 256), but two rounds or more 32^3 x 64 491 / 503, 64x32^3 510 /
+    // 523, 32^3 x 96 737 / 744, 96x32^3 808 / 840, on the largest slices 64^3 x 8
+    // 585 / 564, x 12 856 / 844, 64x64x32x8 287 / 275 (128x64x32x8 600 / 642: rows
+    // longer than a quarter of its blocks); 16^3 x 32 26 / 31, 24^3 x 48 146 / 198,
+    // 40^3 x 80 1185 / 1310, 48^3 x 96 2610 / 2920.
+    if (nrhs == 1) {
+        const bool stream_large = V3 >= (st.tl == ctx->g.L[3] ? 131072 : kLargeSlice) && ctx->g.L[0] <= 64 &&
+                                  st.tl >= 4 && st.fill >= 0.99;
+        return !stream_large && (st.tl < 8 || st.fill < 0.8 || st.wgs > 256);
+    }
+    // Two, in turn here, in one work item there: 32^4 381 / 374, 32^3 x 48 725 / 666,
+    // 48x32^3 754 / 696, 24^3 x 32 187 / 179, 40^3 x 8 242 / 214, 64^3 x 4 556 / 435,
+    // but 16^3 x 96 170 / 178, 32x32x16x16 at one round of workgroups, 24^3 x 48
+    // (0.63 full) 250 / 297.
+    if (nrhs == 2 && st.fill >= 0.75 && st.tl >= (st.wgs > 256 ? 4 : 8) && V3 >= 13000) return false;
+    // More: 32^4 x 4 798 / 684, 32^3 x 12 x 4 294 / 276, 64^3 x 4 x 6 1378 / 1297, but
+    // 32^3 x 12 x 6 and x 12 are 8 and 9% faster here, 16^3 x 32 x 4 80 / 93, 24^3 x
+    // 48 x 4 456 / 598.
+    if (st.tl == 4 && st.wgs > 256 && st.fill >= 0.9 && V3 >= 32768 && (nrhs <= 4 || large)) return false;
+    return st.tl < 8 || st.fill < 0.8;
 }
 
 // The LDS-staged kernel (streaming lattices) where it has work enough.
