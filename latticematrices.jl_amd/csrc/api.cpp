@@ -155,7 +155,8 @@ static int noalloc_scratch_address(int device, void** out) {
 // Lattices up to this volume take the small-lattice iteration (four launches
 // instead of six): 8^3 x 16 22 us an iteration against 34, 16^4 56 against 67,
 // but 16^3 x 32 112 against 104, where every block summing all partials costs
-// more than the two launches it saves.
+// more than the two launches it saves.  It runs on the eight-wavefront stencil
+// alone, so a forced streaming shape takes the general iteration.
 constexpr int64_t kSmallCgVolume = 1 << 16;
 static int small_cg_n64(const lmx_context* c) { return (int)((c->V + 63) / 64); }
 // Its second state record lies after the two rows of 64-site sums.
@@ -181,7 +182,7 @@ static int cg_ddagd_run(lmx_wilson* op, lmx_context* c, void* x, const void* b, 
     const int chunk = chunk_of(params);
     const long max_polls = (long)params->maxiter / chunk + 3;
     long polls = 0;
-    if (c->nc == 3 && c->V <= kSmallCgVolume) {
+    if (c->nc == 3 && c->V <= kSmallCgVolume && !shape_forced(c)) {
         // small lattices (blas.hip): the state alternates between two records
         CGState* st2 = small_cg_state2(c);
         double *pap_w = c->partials, *rr_w = c->partials + small_cg_n64(c);

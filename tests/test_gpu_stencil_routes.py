@@ -34,3 +34,19 @@ def test_route(gpu, L, csw, nrhs, stream):
     names = launched(lambda: lmx.mul_(y, D, x))
     assert count(names, "k_stream") == (1 if stream else 0)
     assert count(names, "k_hops") == (0 if stream else 1)
+
+
+@pytest.mark.parametrize("csw", [0.0, 1.0])
+def test_forced_shape_in_the_solver(gpu, monkeypatch, csw):
+    # D^dagger with the fused p.Ap follows a forced streaming shape on small lattices too
+    print(f"forced shape CG csw={csw}", flush=True)
+    monkeypatch.setenv("LMX_STREAM_TL", "4")
+    monkeypatch.setenv("LMX_STREAM_ZS", "2")
+    lat = lmx.Lattice((16, 8, 4, 8), ANTI)
+    D = lmx.WilsonDiracOperator4D(lmx.GaugeField(lat), 0.12, csw)
+    b = lat.spinor()
+    b.data.fill_(1.0)
+    x, r, p, Ap, tmp = (lat.spinor() for _ in range(5))
+    names = launched(lambda: lmx.cg_(x, lmx.DdagDOp(D, tmp), b, r, p, Ap, rtol=0.0, maxiter=8, check_every=8))
+    assert count(names, "k_hops") == 0 and count(names, "k_cg_small") == 0
+    assert count(names, "k_stream") >= 16
