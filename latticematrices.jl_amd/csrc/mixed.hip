@@ -423,8 +423,8 @@ static SO out_of(const InnerVec& v, int V) {
     return SO::at(v.p, v.n, V, 0);
 }
 
-static int apply_ddagd64(MixRun& R, double2* out, const double2* in, double2* tmp, const int* gate) {
-    Epilogue e{0, nullptr, nullptr, nullptr, nullptr, gate};
+static int apply_ddagd64(MixRun& R, double2* out, const double2* in, double2* tmp) {
+    const Epilogue e{0, nullptr, nullptr, nullptr, nullptr};
     lmx_wilson* op = R.op;
     LMX_TRY(launch_wilson_f64(R.ctx, op->links, op->clover64, op->kappa, op->csw, tmp, in, R.nrhs, 0, e));
     return launch_wilson_f64(R.ctx, op->links, op->clover64, op->kappa, op->csw, out, tmp, R.nrhs, LMX_DAGGER, e);
@@ -653,7 +653,7 @@ int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void
     R.update_each = rmax < 2 * kXBatch;  // updates so dense that most groups would be cut short
     hipLaunchKernelGGL(k_mx_reset, dim3(1), dim3(64), 0, c->stream, R.w.rhs, R.w.batch, nrhs, params->reliable_delta,
                        rmax, params->maxiter);
-    LMX_TRY(apply_ddagd64(R, R.w.r64, x, R.w.t64, nullptr));
+    LMX_TRY(apply_ddagd64(R, R.w.r64, x, R.w.t64));
     if (R.spinor_prec == LMX_H16)
         enqueue_init<SpH16Out>(R, grid);
     else
