@@ -18,7 +18,8 @@
 //   sequence of launches that can be captured once in a hipGraph and replayed.
 //   The iteration that requests an update is the last of its group to run (the
 //   rest find their gate off), so an update still follows the iteration that
-//   asked for it.
+//   asked for it.  Where updates come every iteration or two (kEachDelta)
+//   the gated update follows each iteration instead; the arithmetic is the same.
 // The reference solver this replaces is cg! (src/LinearAlgebras/cg.jl:73-137)
 // on DdagDOp (src/Operators/DiracOperators.jl:104-121).
 #include <algorithm>
@@ -47,6 +48,8 @@ struct MixBatch {
     int go;         // iterations run: an RHS is active and no update is pending
     int live;       // go as the current iteration began
     int ticket;     // RHS whose update has ended
+    int ran;        // iterations that ran
+    int asked;      // updates that ran
     double delta;
     int rmax;
     int maxiter;    // an RHS stops once its inner iteration count reaches it
@@ -240,7 +243,10 @@ __global__ void __launch_bounds__(256) k_mx_fin(const double* __restrict__ parti
     const double b = KIND == MX_INIT ? strided_sum(partials + (size_t)(2 * i + 1) * nb, nb) : 0.0;
     asm volatile("" ::: "memory");  // no load sinks below the gates
     if (KIND == MX_PAP) {
-        if (i == 0 && threadIdx.x == 0) batch->live = q.go;
+        if (i == 0 && threadIdx.x == 0) {
+            batch->live = q.go;
+            if (q.go) batch->ran = q.ran + 1;
+        }
         if (!q.go) return;
     }
     if (KIND == MX_RR && !q.live) return;
@@ -254,6 +260,7 @@ __global__ void __launch_bounds__(256) k_mx_fin(const double* __restrict__ parti
         __threadfence();
         if (atomicAdd(&batch->ticket, 1) == (int)gridDim.x - 1) {
             batch->ticket = 0;
+            batch->asked = q.asked + 1;
             batch->do_update = 0;
             batch->go = atomicAdd(&batch->n_active, 0) > 0;
         }
@@ -308,6 +315,8 @@ __global__ void k_mx_reset(MixRhs* rhs, MixBatch* batch, int nrhs, double delta,
         batch->go = 1;
         batch->live = 0;
         batch->ticket = 0;
+        batch->ran = 0;
+        batch->asked = 0;
         batch->delta = delta;
         batch->rmax = rmax;
         batch->maxiter = maxiter;
@@ -378,7 +387,8 @@ __device__ __forceinline__ void copy_site(const SpH16In& from, const InnerVec& t
 }
 
 // An update that cuts a group short also puts the newest p where the next
-// group's first iteration reads it, in the ring's last slot.
+// group's first iteration reads it, in the ring's last slot (last; null where
+// no group follows or the phases go on).
 // (grid-stride over the sites: a small grid, so that the launch costs little
 // on the groups where the update is gated off)
 template <class SI>
@@ -391,7 +401,7 @@ __global__ void __launch_bounds__(256) k_mx_accum(double2* __restrict__ x, float
     const int mask = rhs[i].pmask;  // slots not yet overwritten by a later p update
     for (int s = blockIdx.x * 256 + threadIdx.x; s < V; s += gridDim.x * 256) {
         accum_site(x, xlo, ring, V, rhs[i], mask, o, o4, i, s);
-        if (force) continue;
+        if (last.p == nullptr) continue;
 #pragma unroll
         for (int j = 0; j < kXBatch - 1; ++j)
             if (mask >> j == 1) copy_site(ring.p[j], last, V, i, s);
@@ -542,26 +552,38 @@ static RingSlots<SI> ring_of(MixRun& R) {
     for (int j = 0; j < kXBatch - 1; ++j) g.p[j] = in_of<SI>(R.w.p[j], (int)R.ctx->V);
     return g;
 }
-static void enqueue_accum(MixRun& R, dim3 grid, int force) {
+static void enqueue_accum(MixRun& R, dim3 grid, int force, bool new_group) {
     const int V = (int)R.ctx->V;
+    const InnerVec last = new_group ? R.w.p[kXBatch - 1] : InnerVec{nullptr, nullptr};
     grid.x = std::min(grid.x, kUpdateBlocks);
     if (R.spinor_prec == LMX_H16)
         hipLaunchKernelGGL((k_mx_accum<SpH16In>), grid, dim3(256), 0, R.ctx->stream, R.x, R.w.xlo, ring_of<SpH16In>(R),
-                           R.w.p[kXBatch - 1], V, R.w.rhs, R.w.batch, force);
+                           last, V, R.w.rhs, R.w.batch, force);
     else
         hipLaunchKernelGGL((k_mx_accum<SpF32In>), grid, dim3(256), 0, R.ctx->stream, R.x, R.w.xlo, ring_of<SpF32In>(R),
-                           R.w.p[kXBatch - 1], V, R.w.rhs, R.w.batch, force);
+                           last, V, R.w.rhs, R.w.batch, force);
+}
+
+static int enqueue_update(MixRun& R) {
+    lmx_context* c = R.ctx;
+    const int nb = nblocks(c->V);
+    enqueue_accum(R, dim3(nb, R.nrhs), 0, !R.update_each);
+    LMX_TRY(enqueue_true_ddagd(R, R.x, &R.w.batch->do_update, 0));
+    hipLaunchKernelGGL(k_mx_fin<MX_TRUE>, dim3(R.nrhs), dim3(256), 0, c->stream, R.w.partials, nb, R.w.rhs, R.w.batch,
+                       0.0, 0.0, 0);
+    LMX_HIP(hipGetLastError());
+    return LMX_OK;
 }
 
 // One iteration with phase e in its group, and after the group's last one the
-// gated update.  A launch that finds its gate off still costs 1.5 us, and only
-// one iteration in 18 (8^3 x 16) to 35 (24^3 x 48) asks for an update: with the
-// update's four launches after every iteration one right-hand side in 16 bits
-// took 33.9 us an iteration at 8^3 x 16 against 28.8, four with FP16 links
-// 93.2 at 16^4 against 89.3.
+// gated update.  A launch that finds its gate off still costs 1.5 us, and at
+// the default delta only one iteration in 18 (8^3 x 16) to 35 (24^3 x 48) asks
+// for an update: with the update's four launches after every iteration one
+// right-hand side in 16 bits took 33.9 us an iteration at 8^3 x 16 against
+// 28.8, four with FP16 links 93.2 at 16^4 against 89.3.
 static int enqueue_iteration(MixRun& R, int e) {
     lmx_context* c = R.ctx;
-    dim3 grid(nblocks(c->V), R.nrhs), blk(256);
+    const dim3 blk(256);
     const int nb = nblocks(c->V);
     MixRhs* rhs = R.w.rhs;
     MixBatch* bt = R.w.batch;
@@ -569,12 +591,39 @@ static int enqueue_iteration(MixRun& R, int e) {
     hipLaunchKernelGGL(k_mx_fin<MX_PAP>, dim3(R.nrhs), blk, 0, c->stream, R.w.partials, nb, rhs, bt, 0.0, 0.0, 0);
     LMX_TRY(apply_ddag_xr(R, e));
     hipLaunchKernelGGL(k_mx_fin<MX_RR>, dim3(R.nrhs), blk, 0, c->stream, R.w.partials, nb, rhs, bt, 0.0, 0.0, e);
-    if (R.update_each || e == kXBatch - 1) {
-        enqueue_accum(R, grid, 0);
-        LMX_TRY(enqueue_true_ddagd(R, R.x, &bt->do_update, 0));
-        hipLaunchKernelGGL(k_mx_fin<MX_TRUE>, dim3(R.nrhs), blk, 0, c->stream, R.w.partials, nb, rhs, bt, 0.0, 0.0, 0);
-    }
     LMX_HIP(hipGetLastError());
+    return R.update_each || e == kXBatch - 1 ? enqueue_update(R) : LMX_OK;
+}
+
+// Updates as dense as every second iteration follow each iteration instead: a
+// group that they cut short idles through its remaining iterations, which then
+// costs more than the gated launches that the groups save.  One 16-bit
+// right-hand side at 8^3 x 16, an update every 1, 1.4, 3.5, 6 iterations: in
+// groups 2530, 14500, 10180, 8620 us a solve, after each 1530, 9300, 10170,
+// 9740; 16^4 the same.  The default delta stays in groups: 2.6 iterations
+// apart at the least (kappa = 0.05), 1160 against 1220.  Above it the first
+// iterations tell, up to a delta where no solve gains from groups.
+constexpr double kGroupDelta = 0.1, kEachDelta = 0.6;
+constexpr int kDecideAfter = 2 * kXBatch, kDenseInterval = 3;
+
+// `n` iterations captured on a stream of their own, to be replayed.
+static int capture_iterations(MixRun& R, int n, hipGraph_t* graph, hipGraphExec_t* exec) {
+    lmx_context* c = R.ctx;
+    hipStream_t cap;
+    LMX_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
+    hipStream_t saved = c->stream;
+    c->stream = cap;
+    hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeRelaxed);
+    int rc = LMX_OK;
+    if (e == hipSuccess) {
+        for (int k = 0; k < n && rc == LMX_OK; ++k) rc = enqueue_iteration(R, k % kXBatch);
+        e = hipStreamEndCapture(cap, graph);
+    }
+    c->stream = saved;
+    (void)hipStreamDestroy(cap);
+    LMX_TRY(rc);
+    LMX_HIP(e);
+    LMX_HIP(hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0));
     return LMX_OK;
 }
 
@@ -650,7 +699,10 @@ int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void
     R.rhs_block = params->rhs_block > 0 ? params->rhs_block : default_rhs_block(op, params->precision, nrhs);
     dim3 grid(nblocks(c->V), nrhs), blk(256);
     const int rmax = params->reliable_maxiter > 0 ? params->reliable_maxiter : 100;
-    R.update_each = rmax < 2 * kXBatch;  // updates so dense that most groups would be cut short
+    const double delta = params->reliable_delta;
+    R.update_each = rmax < 2 * kXBatch || delta > kGroupDelta;
+    // whether the first iterations tell if groups pay
+    const bool decide = rmax >= 2 * kXBatch && delta > kGroupDelta && delta < kEachDelta;
     hipLaunchKernelGGL(k_mx_reset, dim3(1), dim3(64), 0, c->stream, R.w.rhs, R.w.batch, nrhs, params->reliable_delta,
                        rmax, params->maxiter);
     LMX_TRY(apply_ddagd64(R, R.w.r64, x, R.w.t64));
@@ -668,47 +720,38 @@ int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void
     if (params->use_graph) chunk = (chunk + kXBatch - 1) / kXBatch * kXBatch;
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
-    if (params->use_graph) {
-        hipStream_t cap;
-        LMX_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
-        hipStream_t saved = c->stream;
-        c->stream = cap;
-        hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeRelaxed);
-        int rc = LMX_OK;
-        if (e == hipSuccess) {
-            for (int k = 0; k < chunk && rc == LMX_OK; ++k) rc = enqueue_iteration(R, k % kXBatch);
-            e = hipStreamEndCapture(cap, &graph);
-        }
-        c->stream = saved;
-        (void)hipStreamDestroy(cap);
-        if ((rc != LMX_OK || e != hipSuccess) && graph) (void)hipGraphDestroy(graph);
-        LMX_TRY(rc);
-        LMX_HIP(e);
-        LMX_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    }
     std::vector<MixRhs> hs(nrhs);
     MixBatch hb;
     // every group runs at least one of its iterations, so the device has
     // retired all RHS by maxiter at the latest after maxiter groups
     const int64_t most = (int64_t)kXBatch * params->maxiter;
+    // How the updates are launched decides where the groups of deferred x
+    // updates begin, so it changes after a fixed number of iterations, not at
+    // whatever poll sees the need: the bits do not depend on check_every.
     int64_t launched = 0;
     int rc = LMX_OK;
     while (true) {
-        LMX_HIP(hipMemcpyAsync(&hb, R.w.batch, sizeof(MixBatch), hipMemcpyDeviceToHost, c->stream));
-        LMX_HIP(hipStreamSynchronize(c->stream));
+        hipError_t e = hipMemcpyAsync(&hb, R.w.batch, sizeof(MixBatch), hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        if (e != hipSuccess) {
+            rc = LMX_ERR_HIP;
+            set_error("mixed solver poll failed: %s", hipGetErrorString(e));
+            break;
+        }
         if (hb.n_active <= 0 || launched >= most) break;
-        if (exec) {
-            if (hipGraphLaunch(exec, c->stream) != hipSuccess) {
+        if (decide && launched == kDecideAfter) R.update_each = hb.ran < kDenseInterval * hb.asked;
+        const int n = decide && launched < kDecideAfter ? std::min(chunk, kDecideAfter - (int)launched) : chunk;
+        if (params->use_graph && !(decide && launched < kDecideAfter)) {
+            if (!exec) rc = capture_iterations(R, chunk, &graph, &exec);
+            if (rc == LMX_OK && hipGraphLaunch(exec, c->stream) != hipSuccess) {
                 rc = LMX_ERR_HIP;
                 set_error("hipGraphLaunch failed");
-                break;
             }
-            launched += chunk;
         } else {
-            for (int k = 0; k < chunk && rc == LMX_OK; ++k) rc = enqueue_iteration(R, (int)((launched + k) % kXBatch));
-            if (rc != LMX_OK) break;
-            launched += chunk;
+            for (int k = 0; k < n && rc == LMX_OK; ++k) rc = enqueue_iteration(R, (int)((launched + k) % kXBatch));
         }
+        if (rc != LMX_OK) break;
+        launched += n;
     }
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -716,7 +759,7 @@ int cg_batched_impl(lmx_wilson* op, double2* x, const double2* b, int nrhs, void
     // RHS stopped by maxiter (or retired by a breakdown): fold the inner
     // solution in and report the true residual; the ring slots marked in
     // pmask hold the still deferred alpha p
-    enqueue_accum(R, grid, 1);
+    enqueue_accum(R, grid, 1, false);
     LMX_TRY(enqueue_true_ddagd(R, x, nullptr, 1));
     hipLaunchKernelGGL(k_mx_fin<MX_TRUE>, dim3(nrhs), blk, 0, c->stream, R.w.partials, nblocks(c->V), R.w.rhs,
                        R.w.batch, 0.0, 0.0, 1);
