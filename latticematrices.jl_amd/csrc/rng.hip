@@ -458,6 +458,13 @@ __global__ void __launch_bounds__(256) k_rng_fill_padded(void* __restrict__ out,
 // 32^4 812 us over three, 1068 over twelve) and no faster on small lattices
 // (8^3 x 16 6 us either way).
 constexpr int kFillBatch = 16;
+
+// Uniform fields of this many sites take a launch each: the fill is then bound
+// by its writes, which a grid over several fields spreads worse (twelve at 32^4
+// 517 us one by one, 600 together; 48^3 x 32 the same either way, 24^3 x 48 277
+// and 254, 16^3 x 32 71 and 51).
+constexpr int64_t kUniformAlone = 1000000;
+
 struct FieldSeeds {
     FieldSeed f[kFillBatch];
 };
@@ -621,8 +628,9 @@ int launch_spinor_randomize(lmx_context* ctx, void* dst, int nrhs, int dist, con
     LMX_TRY(make_fill_geom(ctx, 0, goff, gdims, g));
     if (ctx->V == 0) return LMX_OK;
     const int gauss = dist == LMX_FILL_GAUSSIAN;
-    for (int r = 0; r < nrhs; r += kFillBatch) {
-        const int n = std::min(nrhs - r, kFillBatch);
+    const int batch = gauss || ctx->V < kUniformAlone ? kFillBatch : 1;
+    for (int r = 0; r < nrhs; r += batch) {
+        const int n = std::min(nrhs - r, batch);
         FieldSeeds f = {};
         for (int k = 0; k < n; ++k) f.f[k] = field_seed(keys[r + k]);
         double2* out = (double2*)dst + (size_t)r * 12 * ctx->V;
