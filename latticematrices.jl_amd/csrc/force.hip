@@ -210,7 +210,9 @@ __device__ __forceinline__ void cotangent_plane(double2* __restrict__ dQ, const 
 #pragma unroll
     for (int k = 0; k < 9; ++k) f[k] = rmul(coefficient, f[k]);
     double2* q = dQ + (size_t)PL * 5 * V;
-    const double d0 = 0.125 * (f[0].im + f[0].im), d1 = 0.125 * (f[4].im + f[4].im), d2 = 0.125 * (f[8].im + f[8].im);
+    // (re - re is zero, or the NaN of an infinite real part, which the imaginary part carries on)
+    const auto diag = [](cx<double> z) { return 0.125 * (z.im + z.im) + (z.re - z.re); };
+    const double d0 = diag(f[0]), d1 = diag(f[4]), d2 = diag(f[8]);
     const cx<double> u0 = rmul(0.125, csub(f[1], cconj(f[3]))), u1 = rmul(0.125, csub(f[2], cconj(f[6]))),
                      u2 = rmul(0.125, csub(f[5], cconj(f[7])));
     q[s] = make_double2(d0, d1);
