@@ -198,8 +198,13 @@ __device__ __forceinline__ void cotangent_add(const cx<double> d[12], const cx<d
             f[3 * c + ic] = cadd(f[3 * c + ic], cmul(d[O * 3 + c], cconj(i_pow<e.pow>(p[e.col * 3 + ic]))));
 }
 template <int PL, int MU, int NU>
-__device__ __forceinline__ void cotangent_plane(double2* __restrict__ dQ, const cx<double> d[12], const cx<double> p[12],
+__device__ __forceinline__ void cotangent_plane(double2* __restrict__ dQ, cx<double> (&d)[12], const cx<double> p[12],
                                                 int s, int V, double coefficient) {
+    // the planes three by three: the products of all interleaved spill
+    if (PL == 3) {
+#pragma unroll
+        for (int k = 0; k < 12; ++k) asm volatile("" : "+v"(d[k].re), "+v"(d[k].im)::"memory");
+    }
     cx<double> f[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) f[k] = mk<double>(0.0, 0.0);
