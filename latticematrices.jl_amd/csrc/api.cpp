@@ -153,9 +153,10 @@ static int noalloc_scratch_address(int device, void** out) {
 }
 
 // Lattices up to this volume take the small-lattice iteration (four launches
-// instead of six): 8^3 x 16 22 us an iteration against 34, 16^4 56 against 67,
-// but 16^3 x 32 112 against 104, where every block summing all partials costs
-// more than the two launches it saves.  It runs on the eight-wavefront stencil
+// instead of six): 8^3 x 16 20.6 us an iteration against 31.4, 16^4 52 against
+// 65, with the clover term 22.0 / 32.4 and 62 / 75; at 16^3 x 32 102 against 102
+// (clover 120 / 120), where every block summing all partials costs as much as
+// the two launches it saves.  It runs on the eight-wavefront stencil
 // alone, so a forced streaming shape takes the general iteration.
 constexpr int64_t kSmallCgVolume = 1 << 16;
 static int small_cg_n64(const lmx_context* c) { return (int)((c->V + 63) / 64); }

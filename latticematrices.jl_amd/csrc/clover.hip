@@ -59,13 +59,15 @@ __device__ __forceinline__ void leaf(const double2* __restrict__ U, int V, cx<do
 
 // A wavefront of a workgroup takes one plane of the workgroup's 64 sites: the
 // six share their links in L1, a leaf's last link is the next leaf's first,
-// and blocks follow slab_block's order.  Bound by the 78 link loads (11.2 KB)
-// per site that pass through L1 (19 TB/s over the chip at 24^3 x 48; its 72
-// products are 131 us there with every lane busy); 400 us there and 76 us at
-// 16^3 x 32, against 868 and 155 us for one work item per site that kept all
-// planes' results in scratch, in lattice order over all XCDs.  Without pin9
+// and blocks follow slab_block's order.  Bound by latency: the 78 link loads of
+// a site (11.2 KB through L1) come in eight rounds, each behind the product
+// before it, and wavefronts wait 39% of their cycles (the 72 products are 131
+// us at 24^3 x 48 with every lane busy; 56 loads, shared links through LDS,
+// were slower).  400-430 us there and 76 us at 16^3 x 32, against 868 and 155
+// us for one work item per site that kept all planes' results in scratch, in
+// lattice order over all XCDs.  Without pin9
 // the loads are hoisted and spilled (690 us), at 4 wavefronts per SIMD it
-// spills (1180), at 2 it waits (430).
+// spills (1180), at 2 it waits (430); at 3 one of the 168 registers spills.
 __global__ void __launch_bounds__(384, 3) k_clover_build(const double2* __restrict__ U, double2* __restrict__ F, Geom g,
                                                          int slab) {
     int s0, end;

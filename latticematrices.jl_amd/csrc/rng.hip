@@ -452,8 +452,8 @@ __global__ void __launch_bounds__(256) k_rng_fill_padded(void* __restrict__ out,
 // spin, site-major planes): the Gaussian or uniform (3,4) ComplexF64 fill of
 // right-hand side blockIdx.y.  Bound by its instructions, about 170 per entry
 // with Philox, 16 of them at a quarter of the rate: twelve Gaussian fields at
-// 32^4 in 755 us, 3.2 TB/s written, against 1118 us with the device library's
-// logarithm, square root, sine and cosine and one launch per field.  The
+// 32^4 in 755-800 us, 3.0-3.2 TB/s written, against 1118-1143 us with the device
+// library's logarithm, square root, sine and cosine and one launch per field.  The
 // entries of a site split over several work items are slower (12 fields at
 // 32^4 812 us over three, 1068 over twelve) and no faster on small lattices
 // (8^3 x 16 6 us either way).

@@ -15,15 +15,18 @@
 //
 // Why: with the hops one after the other in one work item (k_site, k_stream)
 // a site waits for nine loads in turn, at 230-256 VGPRs and one or two
-// wavefronts per SIMD in FP64.  Here it waits for one, at 88 VGPRs and five
-// wavefronts per SIMD, at the price of 1.5 KB of LDS traffic per site and of
-// the neighbours in t read again.  To keep those in L2 the blocks are ordered
-// slab by slab (slab_order): an eighth of the 3-D volume, one XCD's share, for
-// t = 0, 1, ... (lattice order instead: 174 against 148 us at 24^3 x 48, 3400
-// against 2650 us at 48^3 x 96; tiles in y and z, nontemporal loads of links
-// and a walk over t within the workgroup were no faster).  Bound by the L2
-// misses that remain (24^3 x 48: 0.79 GB moved at 5.3 TB/s, 1.23x the fields
-// themselves).
+// wavefronts per SIMD in FP64.  Here it waits for one, at four wavefronts per
+// SIMD (a workgroup is two on each; 88 VGPRs in FP64, 120 with complex phases,
+// 128 with the clover term, where D^dagger with p.Ap spills 12 of them and the
+// complex-phase variants 8 and 13), at the price of 1.5 KB of LDS traffic per
+// site and of the neighbours in t read again.  To keep those in L2 the blocks
+// are ordered slab by slab (slab_order): an eighth of the 3-D volume, one XCD's
+// share, for t = 0, 1, ... (lattice order instead: 174 against 148 us at 24^3 x
+// 48, 3400 against 2650 us at 48^3 x 96; tiles in y and z, nontemporal loads of
+// links and a walk over t within the workgroup were no faster).  Bound by the
+// L2 misses that remain: 24^3 x 48 0.78 GB moved at 5.2 TB/s, 1.22x the fields
+// themselves, with the clover term 1.09 GB at 5.3 TB/s (1.18x), 48^3 x 96 with
+// it 23.8 GB at 6.7 TB/s (1.61x); the vector pipes issue a fifth of the time.
 //
 #pragma once
 
@@ -299,9 +302,10 @@ __device__ __forceinline__ void hop_wave(const HopArgs<In, Lk, Out, Cl>& a, HopL
     }
 }
 
-// Wavefronts per SIMD to compile for: one field, all that LDS admits; several,
-// where the next field's operands stay in registers across the sum, half (FP64
-// at 4: spills, 24^3 x 48 x 4 597 us against 456).
+// Wavefronts per SIMD to compile for: one field, four in FP64 (its registers;
+// LDS would admit six without the clover term) and six in FP32; several, where
+// the next field's operands stay in registers across the sum, two and four
+// (FP64 at four: spills, 24^3 x 48 x 4 597 us against 456).
 template <typename R>
 constexpr int hop_waves(bool loop) {
     return sizeof(R) == 8 ? (loop ? 2 : 4) : (loop ? 4 : 6);
